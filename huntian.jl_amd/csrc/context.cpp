@@ -1,5 +1,6 @@
 // context.cpp -- host side of libhuntian_hip.so: contexts, error messages, buffer cache,
 // shell-table and collapse-table uploads, and the host-only ABI functions.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <mutex>
@@ -65,7 +66,9 @@ void release_work(SAWork& w) {
     }
     DevBuf* bufs[] = {&w.recs, &w.keys_a, &w.keys_b, &w.vals_a, &w.vals_b, &w.cub_tmp, &w.slots,
                       &w.gtiles, &w.tiles, &w.tilemeta, &w.stops, &w.feats, &w.prof, &w.queue,
-                      &w.flag, &w.skip, &w.paint, &w.tables.cells, &w.tables.start, &w.tables.count,
+                      &w.flag, &w.skip, &w.paint, &w.cross, &w.bcnt, &w.boff, &w.bbase,
+                      &w.slots2, &w.slots3, &w.brick, &w.far, &w.tables.cell8, &w.tables.win,
+                      &w.tables.rinv, &w.tables.brick_tab, &w.tables.near_order, &w.tables.cells, &w.tables.start, &w.tables.count,
                       &w.tables.r2, &w.tables.rad, &w.tables.kw, &w.tables.kw_idx,
                       &w.ctab.table, &w.akk};
     for (DevBuf* b : bufs) release(*b);
@@ -127,6 +130,40 @@ hnt_status finish_call(hnt_ctx* ctx, const char* what) {
         }
     }
     return HNT_OK;
+}
+
+// SPH kernel table of RadialShell._build_atab4 (RadialShell.jl:125-142), FP64.
+static std::vector<double> sph_kernel_table() {
+    std::vector<double> akk(1101);
+    const double ca = 3.0 / (2.0 * kPi);
+    const double cb = 1.0 / (4.0 * kPi);
+    const double two_thirds = 2.0 / 3.0;
+    for (int i = 1; i <= 1100; ++i) {
+        double u = (double)(i - 1) * 0.01;
+        double ru = std::sqrt(u);
+        double v;
+        if (ru < 1.0) {
+            v = ca * (two_thirds - u + 0.5 * u * ru);
+        } else if (ru <= 2.0) {
+            double t = 2.0 - ru;
+            v = cb * (t * t * t);
+        } else {
+            v = 0.0;
+        }
+        akk[i - 1] = v;
+    }
+    akk[1100] = 0.0;
+    return akk;
+}
+
+// An integer of at most 11 bits as Float16 bits (exact).
+static uint16_t small_half(int v) {
+    if (v == 0) return 0;
+    const uint16_t sign = v < 0 ? 0x8000 : 0;
+    uint32_t a = (uint32_t)(v < 0 ? -v : v);
+    int e = 0;
+    while ((a >> (e + 1)) != 0) ++e;
+    return (uint16_t)(sign | ((uint32_t)(e + 15) << 10) | ((a << (10 - e)) & 0x3ff));
 }
 
 // Shell tables: validated on the host (the library does not trust the caller's grouping),
@@ -211,7 +248,80 @@ hnt_status upload_tables_to(hnt_ctx* ctx, TablesDev& T, const hnt_shell_tables* 
             kw.push_back(hRinteg(u0, u12) / (dd * dd));
         }
     }
-    if (kw.empty()) kw.push_back(0.0);
+    // the centre (mp = 1, RadialShell.jl:255-270): 0.5 W(u) / rad by the SPH kernel table, for
+    // the shells whose table index floor(100 rad^2) lies in it; infinite at the centre itself
+    {
+        std::vector<double> akk = sph_kernel_table();
+        int32_t hi = 0;
+        kidx[3] = 1;
+        kidx[5] = (int32_t)kw.size();
+        for (int32_t m1 = 1; m1 <= ns; ++m1) {
+            const double rm1 = rad[m1], con = 100.0 * rm1 * rm1, fl = std::floor(con);
+            if (!(fl >= 0.0 && fl < 1100.0)) break;
+            const int icon = (int)fl;
+            const double diff = con - (double)icon;
+            const double aww = akk[icon] + diff * (akk[icon + 1] - akk[icon]);
+            kw.push_back(0.5 * aww / rm1);
+            hi = m1;
+        }
+        kidx[4] = hi;
+    }
+    // windows of the walk's shells (shell-block path).  A walk that meets a shell exactly 2
+    // cells out drops it if a shell beyond lies in the window of the step before: blocks_ok
+    // says that such a shell is always there, and the offsets fit a byte
+    std::vector<int32_t> win((size_t)3 * (ns + 2), 1);
+    bool blocks_ok = t->rmax <= 127 && ns <= 8000;
+    {
+        const int32_t m = ns - 1;
+        for (int32_t s = 1; s <= m; ++s) {
+            int32_t lt = s, le = s, g = s;
+            while (lt < m && rad[lt + 1] < rad[s] + 2.0) ++lt;
+            le = lt;
+            while (le < m && rad[le + 1] <= rad[s] + 2.0) ++le;
+            const double rlow = rad[s] - 2.0 > 0.0 ? rad[s] - 2.0 : 0.0;
+            while (g > 1 && rad[g - 1] > rlow) --g;
+            if (!(rad[g] > rlow)) ++g;  // the centre's own rad, 0, is not above 0
+            win[3 * s] = lt;
+            win[3 * s + 1] = le;
+            win[3 * s + 2] = g;
+            if (le != lt && (le != lt + 1 || (le < m && s < m && !(rad[le + 1] < rad[s + 1] + 2.0))))
+                blocks_ok = false;
+        }
+    }
+    std::vector<double> rinv((size_t)ns + 2, 0.0);
+    for (int32_t s = 2; s <= ns; ++s) rinv[s] = 1.0 / rad[s];
+    // shells with r <= 8 cells (below the last shell, which no peak gathers), and their order by
+    // falling number of cells
+    int32_t near_shells = 0;
+    while (near_shells < ns - 1 && t->shell_r2[near_shells] <= 64) ++near_shells;
+    const int32_t near_cells = t->shell_start[near_shells - 1] + t->shell_count[near_shells - 1];
+    std::vector<uint8_t> order((size_t)near_shells);
+    bool even = true;
+    for (int32_t s = 1; s <= near_shells; ++s) {
+        order[s - 1] = (uint8_t)s;
+        even = even && (s == 1 || t->shell_count[s - 1] % 2 == 0);
+    }
+    // a shell's cells by rising planes (the far gather takes them plane by plane)
+    for (int32_t s = 0; s < ns; ++s)
+        for (int32_t c = 1; c < t->shell_count[s]; ++c)
+            blocks_ok = blocks_ok && t->dk[t->shell_start[s] + c] >= t->dk[t->shell_start[s] + c - 1];
+    std::stable_sort(order.begin(), order.end(), [&](uint8_t a, uint8_t b) {
+        return t->shell_count[a - 1] > t->shell_count[b - 1];
+    });
+    std::vector<uint32_t> btab((size_t)std::max(near_cells, 1) * 4);
+    for (int32_t q = 0; q < near_cells; ++q) {
+        const int32_t x = t->di[q], y = t->dj[q], z = t->dk[q];
+        const int32_t o[2] = {x + 32 * y + 1024 * z, z + 32 * x + 1024 * y};
+        for (int v = 0; v < 2; ++v) {
+            uint32_t* w = btab.data() + 2 * ((size_t)v * near_cells + q);
+            w[0] = (uint32_t)(o[v] & 0xffff) | ((uint32_t)small_half(x) << 16);
+            w[1] = (uint32_t)small_half(y) | ((uint32_t)small_half(z) << 16);
+        }
+    }
+    std::vector<uint32_t> cell8((size_t)nc);
+    for (int64_t q = 0; q < nc; ++q)
+        cell8[q] = (uint32_t)(t->di[q] & 0xff) | ((uint32_t)(t->dj[q] & 0xff) << 8) |
+                   ((uint32_t)(t->dk[q] & 0xff) << 16);
     HNT_TRY(reserve_in(ctx, T.cells, cells4.size() * sizeof(int32_t), ar));
     HNT_TRY(reserve_in(ctx, T.start, (size_t)ns * sizeof(int32_t), ar));
     HNT_TRY(reserve_in(ctx, T.count, (size_t)ns * sizeof(int32_t), ar));
@@ -233,10 +343,30 @@ hnt_status upload_tables_to(hnt_ctx* ctx, TablesDev& T, const hnt_shell_tables* 
                            ctx->stream));
     HNT_HIP(hipMemcpyAsync(T.kw_idx.p, kidx.data(), kidx.size() * sizeof(int32_t),
                            hipMemcpyHostToDevice, ctx->stream));
+    if (!ar) {  // the fixed scratch runs no shell blocks
+        HNT_TRY(reserve(ctx, T.cell8, cell8.size() * sizeof(uint32_t)));
+        HNT_TRY(reserve(ctx, T.win, win.size() * sizeof(int32_t)));
+        HNT_TRY(reserve(ctx, T.rinv, rinv.size() * sizeof(double)));
+        HNT_TRY(reserve(ctx, T.brick_tab, btab.size() * sizeof(uint32_t)));
+        HNT_TRY(reserve(ctx, T.near_order, order.size()));
+        HNT_HIP(hipMemcpyAsync(T.near_order.p, order.data(), order.size(), hipMemcpyHostToDevice,
+                               ctx->stream));
+        HNT_HIP(hipMemcpyAsync(T.rinv.p, rinv.data(), rinv.size() * sizeof(double),
+                               hipMemcpyHostToDevice, ctx->stream));
+        HNT_HIP(hipMemcpyAsync(T.brick_tab.p, btab.data(), btab.size() * sizeof(uint32_t),
+                               hipMemcpyHostToDevice, ctx->stream));
+        HNT_HIP(hipMemcpyAsync(T.cell8.p, cell8.data(), cell8.size() * sizeof(uint32_t),
+                               hipMemcpyHostToDevice, ctx->stream));
+        HNT_HIP(hipMemcpyAsync(T.win.p, win.data(), win.size() * sizeof(int32_t),
+                               hipMemcpyHostToDevice, ctx->stream));
+    }
     HNT_HIP(hipStreamSynchronize(ctx->stream));
     T.rmax = t->rmax;
     T.nshells = ns;
     T.ncells = nc;
+    T.near_cells = near_cells;
+    T.near_shells = near_shells;
+    T.blocks_ok = !ar && blocks_ok && near_cells <= 2112 && near_shells <= 62 && even;
     T.host.swap(h);
     return HNT_OK;
 }
@@ -263,32 +393,14 @@ hnt_status upload_ctab_to(hnt_ctx* ctx, CTabDev& D, const hnt_ctab* c, Arena* ar
     return HNT_OK;
 }
 
-// SPH kernel table of RadialShell._build_atab4 (RadialShell.jl:125-142), FP64.
 hnt_status ensure_akk(hnt_ctx* ctx) { return ensure_akk_to(ctx, ctx->akk, nullptr); }
 
 hnt_status ensure_akk_to(hnt_ctx* ctx, DevBuf& akk_buf, Arena* ar) {
     if (!ar && akk_buf.p) return HNT_OK;
-    double akk[1101];
-    const double ca = 3.0 / (2.0 * kPi);
-    const double cb = 1.0 / (4.0 * kPi);
-    const double two_thirds = 2.0 / 3.0;
-    for (int i = 1; i <= 1100; ++i) {
-        double u = (double)(i - 1) * 0.01;
-        double ru = std::sqrt(u);
-        double v;
-        if (ru < 1.0) {
-            v = ca * (two_thirds - u + 0.5 * u * ru);
-        } else if (ru <= 2.0) {
-            double t = 2.0 - ru;
-            v = cb * (t * t * t);
-        } else {
-            v = 0.0;
-        }
-        akk[i - 1] = v;
-    }
-    akk[1100] = 0.0;
-    HNT_TRY(reserve_in(ctx, akk_buf, sizeof(akk), ar));
-    HNT_HIP(hipMemcpyAsync(akk_buf.p, akk, sizeof(akk), hipMemcpyHostToDevice, ctx->stream));
+    const std::vector<double> akk = sph_kernel_table();
+    const size_t bytes = akk.size() * sizeof(double);
+    HNT_TRY(reserve_in(ctx, akk_buf, bytes, ar));
+    HNT_HIP(hipMemcpyAsync(akk_buf.p, akk.data(), bytes, hipMemcpyHostToDevice, ctx->stream));
     HNT_HIP(hipStreamSynchronize(ctx->stream));
     return HNT_OK;
 }
@@ -376,7 +488,8 @@ hnt_status hnt_ctx_destroy(hnt_ctx* ctx) {
     DevBuf* bufs[] = {&ctx->fieldptrs, &ctx->fcrit, &ctx->akk, &ctx->small,
                       &ctx->tables.cells, &ctx->tables.start, &ctx->tables.count,
                       &ctx->tables.r2, &ctx->tables.rad, &ctx->tables.kw,
-                      &ctx->tables.kw_idx, &ctx->ctab.table, &ctx->mlp.wt, &ctx->mlp.x0,
+                      &ctx->tables.kw_idx, &ctx->tables.cell8, &ctx->tables.win,
+                      &ctx->tables.rinv, &ctx->tables.brick_tab, &ctx->tables.near_order, &ctx->ctab.table, &ctx->mlp.wt, &ctx->mlp.x0,
                       &ctx->mlp.z, &ctx->mlp.h, &ctx->mlp.y, &ctx->mlp.dy, &ctx->mlp.dyf,
                       &ctx->mlp.dz, &ctx->mlp.gw, &ctx->mlp.part, &ctx->mlp.gradv};
     for (DevBuf* b : bufs) release(*b);

@@ -31,16 +31,29 @@ struct TablesDev {
     DevBuf rad;                 // double [nshells + 2], rad[s] = sqrt(r2 of shell s), 1-based
     // kernel_strain weights hRinteg(u0, u12) / (u12 - u0^2)^2 of shell m1 around shell mp,
     // for the shells with u0^2 < 4 (u0 = rad[mp] - rad[m1]): m1 in [kw_lo[mp], kw_hi[mp]],
-    // weight at kw[kw_off[mp] + m1 - kw_lo[mp]]; mp = 2 .. nshells
+    // weight at kw[kw_off[mp] + m1 - kw_lo[mp]]; mp = 1 .. nshells
+    // (mp = 1: the centre's weights, shells with rad^2 < 11)
     DevBuf kw;                  // double
     DevBuf kw_idx;              // int32 [3 * (nshells + 2)]: lo, hi, off of each mp
+    DevBuf cell8;               // uint32 per cell: di, dj, dk as three signed bytes
+    DevBuf win;                 // int32 [3 * (nshells + 2)]: per shell s < nshells the last m1 with
+                                // rad < rad[s] + 2, the last with <=, the first > rad[s] - 2
+    DevBuf rinv;                // double [nshells + 2], 1 / rad
+    // cells within the brick gather's halo (8 cells): box offsets (x + 32 y + 1024 z as 16 bits)
+    // and offsets as Float16, for the fields, then for the transposed delta (z + 32 x + 1024 y)
+    DevBuf brick_tab;           // uint2 [2 * near_cells]
+    DevBuf near_order;          // uint8: the shells within the halo by falling number of cells
+    int32_t near_cells = 0;     // table cells of the shells within the halo
+    int32_t near_shells = 0;    // those shells, 1 .. near_shells
+    bool blocks_ok = false;     // the shell-block path can use these tables
 };
 
 // One tile of a call, in device memory.  A wavefront's peaks all belong to one tile, so a
 // wave reads its tile's descriptor with scalar loads.
 struct TileDev {
     const float4* recs;   // 32-byte cell records of this tile
-    const float* delta;   // the caller's delta (crossing pass)
+    const float* delta;   // the caller's fields (crossing pass, shell blocks)
+    const float *etax, *etay, *etaz, *eta2x, *eta2y, *eta2z;
     const float* lapd;
     int n, has_eta2, has_lapd;
     int64_t s1, s2;
@@ -92,7 +105,8 @@ struct Arena {
 // otherwise they are the context's.  With an arena every buffer is carved from it.
 struct SAWork {
     DevBuf recs, keys_a, keys_b, vals_a, vals_b, cub_tmp, slots, gtiles, tiles, tilemeta, stops,
-        feats, prof, queue, flag, skip, paint;
+        feats, prof, queue, flag, skip, paint, cross, bcnt, boff, bbase, slots2,
+        slots3, brick, far;
     std::vector<TileDev> tile_host;
     std::vector<int64_t> meta_host;
     bool own_tables = false;

@@ -29,6 +29,8 @@
 //    of the sorted peak list, so neighbouring peaks share an XCD's L2.  A wave that
 //    drains its queue moves on to the next queue; every wave exits once all eight are
 //    empty.
+// The crossing schedule of a direct call, the default, no longer runs this way but by blocks
+// of shells (shell_blocks.h), with the same results bit for bit.
 #include <hipcub/hipcub.hpp>
 
 #include <mutex>
@@ -1715,7 +1717,8 @@ __device__ int crossing_stop(const SAArgs& a, double Rf, int scross) {
 // arithmetic as the gather, so each peak's exact gather extent.  Workgroup b takes group
 // (b % 8) * G8 + b / 8, G8 an eighth of the groups: each XCD walks its own contiguous eighth.
 __global__ __launch_bounds__(64) void crossing_kernel(SAArgs a, int64_t G8,
-                                                      int32_t* __restrict__ stop_out) {
+                                                      int32_t* __restrict__ stop_out,
+                                                      int32_t* __restrict__ cross_out) {
     const int64_t g = (int64_t)(blockIdx.x & 7) * G8 + (blockIdx.x >> 3);
     if (g >= a.ngroups) return;
     const TileDev& T = a.tiles[a.gtile[g]];
@@ -1755,7 +1758,10 @@ __global__ __launch_bounds__(64) void crossing_kernel(SAArgs a, int64_t G8,
     }
     if (!valid) return;
     stop_out[T.base + p] = crossing_stop(a, Rf, scross);
+    if (cross_out) cross_out[T.base + p] = scross;
 }
+
+#include "shell_blocks.h"
 
 // Bracket-network features of every peak in schedule order (same grouping and XCD mapping
 // as the crossing pass), read from the cell records; feats[(base + p) * 18 + j].
@@ -1975,6 +1981,227 @@ void launch_main(hipStream_t st, const LaunchDesc& d) {
         hipLaunchKernelGGL(shell_analyse_kernel<SumF64>, grid, blk, 0, st, d.A);
 }
 
+// The analysis by shell blocks, from the first order on: crossing pass, block offsets, the
+// radial logic's order, then per chunk of the schedule the gather, Fbar and the radial logic,
+// and the halos' mask.
+template <class OrderBy>
+hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT, int ntiles,
+                          const hnt_batch* batches, hnt_results* results, int8_t* const* masks,
+                          const std::vector<int64_t>& meta, int64_t ntot, int64_t ngroups,
+                          OrderBy&& order_by) {
+    hipStream_t st = ctx->stream;
+    bool any_mask = false;
+    for (int t = 0; t < ntiles; ++t) any_mask = any_mask || (masks && masks[t] && batches[t].npeaks);
+    stage_begin(ctx, HNT_STAGE_SA_CROSS);
+    HNT_TRY(reserve(ctx, W.stops, (size_t)ntot * 4));
+    HNT_TRY(reserve(ctx, W.cross, (size_t)ntot * 4));
+    HNT_TRY(reserve(ctx, W.bcnt, (size_t)ntot * 4));
+    HNT_TRY(reserve(ctx, W.boff, (size_t)ntot * 8));
+    HNT_TRY(reserve(ctx, W.bbase, (size_t)ntot * 8));
+    HNT_TRY(reserve(ctx, W.slots2, (size_t)ngroups * 64 * 4));
+    if (any_mask) {
+        HNT_TRY(reserve(ctx, W.paint, (size_t)ntot * 4));
+        A.paint = (int32_t*)W.paint.p;
+    }
+    int32_t* stops = (int32_t*)W.stops.p;
+    int32_t* cross = (int32_t*)W.cross.p;
+    const bool few = ntot < (1 << 17);
+    if (few) {
+        hipLaunchKernelGGL(crossing_rows_kernel<16>, dim3((unsigned)(ngroups * 16)), dim3(64), 0, st,
+                           A, stops, cross);
+    } else {
+        const int64_t G8 = (ngroups + 7) / 8;
+        hipLaunchKernelGGL(crossing_kernel, dim3((unsigned)(8 * G8)), dim3(64), 0, st, A, G8,
+                           stops, cross);
+    }
+    std::vector<const int32_t*> prim((size_t)ntiles);
+    for (int t = 0; t < ntiles; ++t) {
+        prim[t] = stops + meta[t];
+        if (results[t].schedule_extent && batches[t].npeaks > 0)
+            HNT_HIP(hipMemcpyAsync(results[t].schedule_extent, stops + meta[t],
+                                   (size_t)batches[t].npeaks * 4, hipMemcpyDeviceToDevice, st));
+    }
+    const unsigned nb = (unsigned)((ntot + 255) / 256);
+    int32_t* cnt = (int32_t*)W.bcnt.p;
+    int64_t* off = (int64_t*)W.boff.p;
+    const int32_t* vals = (const int32_t*)W.vals_b.p;
+    const uint64_t* keys = (const uint64_t*)W.keys_b.p;
+    size_t tmp = 0;
+    HNT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, cnt, off, (int)ntot, st));
+    HNT_TRY(reserve(ctx, W.cub_tmp, tmp > 0 ? tmp : 16));
+    // bricks of 16^3 cells with their peaks, and the peaks they do not gather entirely, unless
+    // the tiles hold only a few peaks per brick (staging a brick costs about as much as the
+    // direct gather of five peaks)
+    int64_t vol = 0;
+    for (int t = 0; t < ntiles; ++t) {
+        const int64_t b = (W.tile_host[t].n + BR_CORE - 1) / BR_CORE;
+        vol += batches[t].npeaks > 0 ? b * b * b : 0;
+    }
+    const bool bricks = ntot >= 4 * vol;
+    const int64_t maxbr = std::min(vol, ntot);
+    int32_t* far_slot = (int32_t*)W.slots.p;
+    int32_t* far_cnt = nullptr;
+    BrickArgs K{};
+    if (bricks) {
+        HNT_TRY(reserve(ctx, W.brick, (size_t)(maxbr + 1) * 8 + (size_t)maxbr * 4 + 8 + (size_t)ntiles * 4));
+        HNT_TRY(reserve(ctx, W.far, (size_t)ntot * 8));
+        HNT_TRY(reserve(ctx, W.slots3, (size_t)ngroups * 64 * 4));
+        int64_t* bstart = (int64_t*)W.brick.p;
+        int32_t* btile = (int32_t*)(bstart + maxbr + 1);
+        int32_t* bcount = btile + maxbr;
+        int32_t* fcnt = bcount + 1;
+        far_slot = (int32_t*)W.slots3.p;
+        hipLaunchKernelGGL(brick_head_kernel, dim3(nb), dim3(256), 0, st, keys, ntot, 11 + 3 * 4, cnt);
+        size_t tb = W.cub_tmp.bytes;
+        HNT_HIP(hipcub::DeviceScan::ExclusiveSum(W.cub_tmp.p, tb, cnt, off, (int)ntot, st));
+        hipLaunchKernelGGL(brick_list_kernel, dim3(nb), dim3(256), 0, st, keys, cnt,
+                           (const int64_t*)off, ntot, bstart, btile, bcount);
+        far_cnt = fcnt;
+        hipLaunchKernelGGL(fill_i32, dim3((unsigned)((ntiles + 256) / 256)), dim3(256), 0, st, fcnt,
+                           (int64_t)ntiles + 1, 0);
+        hipLaunchKernelGGL(fill_i32, dim3((unsigned)((ngroups * 64 + 255) / 256)), dim3(256), 0, st,
+                           far_slot, ngroups * 64, -1);
+        hipLaunchKernelGGL(far_list_kernel, dim3(nb), dim3(256), 0, st, A.tiles, keys, vals, stops,
+                           A.rad, ntot, TT.near_shells, (const int64_t*)W.tilemeta.p + ntiles, fcnt,
+                           far_slot, (int64_t*)W.far.p);
+        K = BrickArgs{bstart, btile, bcount, vals, (const uint2*)TT.brick_tab.p,
+                      (const uint8_t*)TT.near_order.p, TT.near_cells, TT.near_shells};
+    }
+    // profile offsets in the first order
+    hipLaunchKernelGGL(block_count_kernel, dim3(nb), dim3(256), 0, st, vals, stops, ntot, cnt);
+    tmp = W.cub_tmp.bytes;
+    HNT_HIP(hipcub::DeviceScan::ExclusiveSum(W.cub_tmp.p, tmp, cnt, off, (int)ntot, st));
+    hipLaunchKernelGGL(block_base_kernel, dim3(nb), dim3(256), 0, st, vals, off, ntot,
+                       (int64_t*)W.bbase.p);
+    // profile space: every peak at its deepest if that is little (no word from the device
+    // needed), else what the scan found; at most kBlockBudget at a time
+    const int nbmax = (A.NS >> 2) + 1;
+    constexpr int64_t kBlockBytes = BLK_DOUBLES * 8;
+    constexpr int64_t kBlockBudget = ((int64_t)32 << 30) / kBlockBytes;
+    std::vector<int64_t> pos{0, ntot}, first{0, ntot * nbmax};  // chunk boundaries
+    const int L2 = std::min(std::max(ctx->brick_log2, 4), 7);
+    if (ntot * nbmax * kBlockBytes > ((int64_t)1 << 30)) {
+        int64_t last_off = 0;
+        int32_t last_cnt = 0;
+        HNT_HIP(hipMemcpyAsync(&last_off, off + (ntot - 1), 8, hipMemcpyDeviceToHost, st));
+        HNT_HIP(hipMemcpyAsync(&last_cnt, cnt + (ntot - 1), 4, hipMemcpyDeviceToHost, st));
+        HNT_HIP(hipStreamSynchronize(st));
+        const int64_t total = last_off + last_cnt;
+        first[1] = total;
+        if (total > kBlockBudget) {
+            const int nc = (int)((total + kBlockBudget - 1) / kBlockBudget);
+            HNT_TRY(reserve(ctx, W.flag, (size_t)nc * 16));
+            hipLaunchKernelGGL(chunk_bounds_kernel, dim3((unsigned)((nc + 63) / 64)), dim3(64), 0,
+                               st, (const uint64_t*)W.keys_b.p, (const int64_t*)off, ntot,
+                               11 + 3 * L2, kBlockBudget, nc, (int64_t*)W.flag.p);
+            std::vector<int64_t> h(2 * (size_t)nc);
+            HNT_HIP(hipMemcpyAsync(h.data(), W.flag.p, h.size() * 8, hipMemcpyDeviceToHost, st));
+            HNT_HIP(hipStreamSynchronize(st));
+            pos.assign(1, 0);
+            first.assign(1, 0);
+            for (int c = 1; c < nc; ++c)
+                if (h[2 * c] > pos.back() && h[2 * c] < ntot) {
+                    pos.push_back(h[2 * c]);
+                    first.push_back(h[2 * c + 1]);
+                }
+            pos.push_back(ntot);
+            first.push_back(total);
+        }
+    }
+    int64_t cap = 0;
+    for (size_t c = 0; c + 1 < pos.size(); ++c) cap = std::max(cap, first[c + 1] - first[c]);
+    HNT_TRY(reserve(ctx, W.prof, (size_t)cap * kBlockBytes));
+    // the radial logic's order: like extents together (few peaks: the first order)
+    int32_t* slot2 = (int32_t*)W.slots.p;
+    if (!few) {
+        slot2 = (int32_t*)W.slots2.p;
+        // the second sort takes over the first order's arrays: the bricks keep a copy of its ids
+        HNT_HIP(hipMemcpyAsync(cnt, vals, (size_t)ntot * 4, hipMemcpyDeviceToDevice, st));
+        K.vals = cnt;
+        HNT_TRY(order_by(prim.data(), L2, slot2));
+    }
+    stage_end(ctx, HNT_STAGE_SA_CROSS);
+
+    stage_begin(ctx, HNT_STAGE_SA_KERNEL);
+    BlockArgs B;
+    B.stop = stops;
+    B.cross = cross;
+    B.base = (const int64_t*)W.bbase.p;
+    B.cell8 = (const uint32_t*)TT.cell8.p;
+    B.rinv = (const double*)TT.rinv.p;
+    B.win = (const int32_t*)TT.win.p;
+    double* q = (double*)W.prof.p;
+    for (int f = 0; f < BLK_FIELDS; ++f) B.line[f] = q + (int64_t)f * cap * 4 * BLK;
+    B.fb = q + (int64_t)BLK_FIELDS * cap * 4 * BLK;
+    // sorted position -> slot: a tile's slots start at a multiple of 64
+    auto slot_of = [&](int64_t at) {
+        int t = 0;
+        while (t + 1 < ntiles && meta[t + 1] <= at) ++t;
+        return meta[ntiles + t] + (at - meta[t]);
+    };
+    // 16-byte loads of the boxes' rows: sides and field pointers that keep every row aligned
+    bool vec4 = true;
+    for (const TileDev& T : W.tile_host) {
+        if (T.npeaks == 0) continue;
+        vec4 = vec4 && (T.n & 3) == 0;
+        for (const float* f : {T.delta, T.etax, T.etay, T.etaz})
+            vec4 = vec4 && ((uintptr_t)f & 15) == 0;
+    }
+    if (bricks) {
+        // more than the default 64 KB of LDS per workgroup
+        HNT_HIP(hipFuncSetAttribute((const void*)gather_bricks_kernel<true>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(BrickLds)));
+        HNT_HIP(hipFuncSetAttribute((const void*)gather_bricks_kernel<false>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(BrickLds)));
+    }
+    const size_t lds = (size_t)nbmax * 8 + (size_t)(nbmax + 1) * 4;
+    for (size_t c = 0; c + 1 < pos.size(); ++c) {
+        B.e0 = first[c];
+        B.ne = first[c + 1] - first[c];
+        const int64_t s0 = slot_of(pos[c]) & ~(int64_t)63;
+        const int64_t s1 = c + 2 == pos.size() ? ngroups * 64 : slot_of(pos[c + 1]);
+        const int64_t g0 = s0 >> 6, ng = (s1 - s0 + 63) >> 6;
+        // (the far peaks' slots are in no chunk's order: every launch looks through all of them)
+        const int64_t h0 = bricks ? 0 : g0, hn = bricks ? ngroups : ng;
+        const int shares = (int)std::min<int64_t>(8, std::max<int64_t>(1, 2048 / hn));
+        SAArgs A1 = A;
+        if (bricks) {
+            const dim3 grid((unsigned)((maxbr + 511) / 512 * 512));
+            if (vec4)
+                hipLaunchKernelGGL(gather_bricks_kernel<true>, grid, dim3(BR_T), sizeof(BrickLds), st,
+                                   A1, B, K);
+            else
+                hipLaunchKernelGGL(gather_bricks_kernel<false>, grid, dim3(BR_T), sizeof(BrickLds), st,
+                                   A1, B, K);
+            for (int f = 0; f < BLK_FIELDS; ++f)
+                hipLaunchKernelGGL(gather_far_kernel, dim3((unsigned)(std::max(8, ctx->num_cus / 8 * 8) * FAR_WG)),
+                                   dim3(FAR_T), 0, st, A1, B, (const int64_t*)W.far.p,
+                                   (const int32_t*)far_cnt, TT.near_shells, f);
+            A1.slot = far_slot;
+        }
+        hipLaunchKernelGGL(gather_blocks_kernel, dim3((unsigned)(8 * ((hn * shares + 7) / 8))),
+                           dim3(256), lds, st, A1, B, h0, hn, shares);
+        hipLaunchKernelGGL(block_fbar_kernel, dim3((unsigned)ng), dim3(64), 0, st, A, B, g0);
+        SAArgs A2 = A;
+        A2.slot = slot2;
+        if (few)
+            hipLaunchKernelGGL(radial_rows_kernel<16>, dim3((unsigned)(8 * ((ng * 16 + 7) / 8))),
+                               dim3(64), 0, st, A2, B, s0, ng * 64);
+        else
+            hipLaunchKernelGGL(radial_rows_kernel<4>, dim3((unsigned)(8 * ((ng * 4 + 7) / 8))),
+                               dim3(64), 0, st, A2, B, s0, ng * 64);
+        hipLaunchKernelGGL(block_sbar_kernel, dim3((unsigned)ng, 3), dim3(64), 0, st, A, B, g0);
+    }
+    stage_end(ctx, HNT_STAGE_SA_KERNEL);
+    stage_begin(ctx, HNT_STAGE_SA_MASK);
+    LaunchDesc D;
+    D.A = A;
+    D.A.slot = slot2;
+    launch_paint(st, D);
+    stage_end(ctx, HNT_STAGE_SA_MASK);
+    return HNT_OK;
+}
+
 // All tiles of a call in one persistent launch: peaks of every tile share the eight queues;
 // a wavefront's 64 lanes belong to one tile.  W holds the call's device buffers; desc (if
 // not NULL) receives what a replay launches.
@@ -2047,8 +2274,18 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
         HNT_REQUIRE(!(bad & 2ull), "hnt_shell_analyse: per-peak ZZon must be > -1");
     }
 
+    // The crossing schedule of a direct call runs by shell blocks (shell_blocks.h); plans
+    // (whose replays re-read changed fields, so that no extent is known beforehand), the fixed
+    // scratch, the other schedules, limits and sums keep a lane (or gang) per peak.
+    const bool early0 = params->early_exit && !limited;
+    int maxn = 1;
+    for (int t = 0; t < ntiles; ++t) maxn = std::max(maxn, fields[t].n1);
+    const bool blocks = early0 && !desc && !W.arena && params->order == HNT_ORDER_CROSSING &&
+                        params->precision == HNT_PREC_FP64 && ctx->gang == 1 && TT.blocks_ok &&
+                        (int64_t)(tables->rmax + 1) * maxn * maxn < (1LL << 31);
+
     // ---- repack every tile's fields into 32-byte cell records ----
-    HNT_TRY(reserve_in(ctx, W.recs, (size_t)ncell * 32, W.arena));
+    if (!blocks) HNT_TRY(reserve_in(ctx, W.recs, (size_t)ncell * 32, W.arena));
     std::vector<TileDev>& TD = W.tile_host;
     TD.assign((size_t)ntiles, TileDev{});
     std::vector<RepackJob> jobs;
@@ -2057,13 +2294,19 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
         for (int t = 0; t < ntiles; ++t) {
             const hnt_fields& f = fields[t];
             const int n = f.n1;
-            float4* recs = (float4*)W.recs.p + 2 * off;
-            if (batches[t].npeaks > 0)
+            float4* recs = blocks ? nullptr : (float4*)W.recs.p + 2 * off;
+            if (batches[t].npeaks > 0 && !blocks)
                 jobs.push_back(RepackJob{f.delta, f.etax, f.etay, f.etaz, f.eta2x, f.eta2y,
                                          f.eta2z, n, recs});
             TileDev& T = TD[t];
             T.recs = recs;
             T.delta = f.delta;
+            T.etax = f.etax;
+            T.etay = f.etay;
+            T.etaz = f.etaz;
+            T.eta2x = f.eta2x;
+            T.eta2y = f.eta2y;
+            T.eta2z = f.eta2z;
             T.lapd = f.lapd;
             T.n = n;
             T.has_eta2 = f.eta2x != nullptr;
@@ -2116,12 +2359,10 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
     // several tiles
     int cb = 0, tb = 0;
     {
-        int maxn = 1;
-        for (int t = 0; t < ntiles; ++t) maxn = std::max(maxn, fields[t].n1);
         while ((1 << cb) < maxn) ++cb;
         while ((1LL << tb) < (int64_t)ntiles) ++tb;
     }
-    auto order_by = [&](const int32_t* const* prim, int L) -> hnt_status {
+    auto order_by = [&](const int32_t* const* prim, int L, int32_t* slot) -> hnt_status {
         const int key_bits = ntiles > 1 ? std::min(64, 50 + tb)
                                         : std::min(50, std::max(3 * cb, 3 * L) + 11);
         for (int t = 0; t < ntiles; ++t) {
@@ -2150,7 +2391,7 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
     // the reference GPU path (ext/CUDAExt.jl:2235-2236): the schedule pass has nothing to order
     const bool early = params->early_exit && !limited;
     const bool two_orders = early && params->order != HNT_ORDER_PLAIN;
-    HNT_TRY(order_by(prim.data(), two_orders ? 4 : ctx->brick_log2));
+    HNT_TRY(order_by(prim.data(), two_orders ? 4 : ctx->brick_log2, slot));
     hipLaunchKernelGGL(group_tile_kernel, dim3((unsigned)((ngroups + 255) / 256)), dim3(256), 0,
                        st, tile_pad, ntiles, ngroups, (int32_t*)W.gtiles.p);
 
@@ -2181,6 +2422,12 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
     A.variant = params->variant;
     A.early = early ? 1 : 0;
     A.rmax2rs = params->rmax2rs;
+
+    if (blocks) {
+        stage_end(ctx, HNT_STAGE_SA_PREP);
+        return analyse_blocks(ctx, W, A, TT, ntiles, batches, results, masks, meta, ntot, ngroups,
+                              order_by);
+    }
 
     const bool kahan = params->precision == HNT_PREC_FP32_KAHAN;
     // the ganged kernels analyse every peak to the last shell: a shell limit takes the
@@ -2259,7 +2506,7 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
         if (params->order == HNT_ORDER_CROSSING) {
             const int64_t G8 = (ngroups + 7) / 8;
             hipLaunchKernelGGL(crossing_kernel, dim3((unsigned)(8 * G8)), dim3(64), 0, st, A, G8,
-                               stops);
+                               stops, nullptr);
         } else if (params->order == HNT_ORDER_GIVEN) {
             // the caller's extents order the peaks; no pass of the library's own
             HNT_HIP(hipMemcpyAsync(stops, params->extent, (size_t)ntot * 4,
@@ -2285,7 +2532,7 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
                                            (size_t)batches[t].npeaks * 4,
                                            hipMemcpyDeviceToDevice, st));
         }
-        HNT_TRY(order_by(prim.data(), ctx->brick_log2));
+        HNT_TRY(order_by(prim.data(), ctx->brick_log2, slot));
         stage_end(ctx, HNT_STAGE_SA_CROSS);
     }
 

@@ -1,0 +1,1265 @@
+// shell_blocks.h -- the shell analysis by shell blocks, included by shell_analyse.hip inside
+// its namespace after the device helpers it shares with the lane-per-peak kernels.
+//
+// The crossing pass gives every peak its gather extent before any gather, and a shell's sums
+// start from zero and depend on no other shell.  So the gather's unit of work here is not a
+// peak but four consecutive shells of a peak (a block): peaks of 170 and of 14 000 cells give
+// work items of similar length, a wavefront's 64 lanes take blocks of the same shells, and
+// the items of a single deep peak run side by side (one lane per peak ran as long as its
+// wavefront's deepest peak: 5.7 of the 7.4 ms of a 128^3 tile).  Within a shell the cells are
+// summed in the reference's order by one lane, with the reference's Float32 products, so the
+// profile is the lane-per-peak kernels' bit for bit.  The fields are read as the caller gave
+// them: no cell records are written.
+//
+// Measured against the lane-per-peak kernel with its records (same bits): shell analysis of the
+// 1024^3 tile 327 -> 264 ms, of the 512^3 tile 51.6 -> 32.5 ms, of a 128^3 tile 7.9 -> 1.5 ms, of a
+// 40^3 tile 1.37 -> 0.43 ms, of 24 tiles of 96^3 to 256^3 37 -> 26 ms.
+//
+// A block's sums are five 128-byte lines, one per field (delta, its transpose, psi_1 xyz),
+// four doubles per shell: {F, G0, G1, G2}, {H0, H1, H2, -}, {S, R0, R1, R2} x 3; G, H and R
+// divided by the shell's radius.  Shell s of a peak is entry 4 base + s (entry 0 unused).
+
+constexpr int BLK = 4;          // shells per block
+constexpr int BLK_FIELDS = 5;   // lines per block
+// doubles of a block: five lines of 4 shells x 4 doubles, and Fbar of its 4 shells
+constexpr int BLK_DOUBLES = BLK_FIELDS * 4 * BLK + BLK;
+
+struct BlockArgs {
+    const int32_t* stop;   // per global peak id: last shell of the gather
+    int32_t* cross;        // per global peak id: crossing shell, 0 = none; then, from the radial
+                           // logic on, the first shell beyond RTHL's, 0 = no collapse
+    const int64_t* base;   // per global peak id: first block of its profile
+    int64_t e0, ne;        // blocks [e0, e0 + ne) are the ones of this launch
+    double* line[BLK_FIELDS];
+    double* fb;            // [4 ne] Fbar of each shell
+    const uint32_t* cell8; // offsets of every table cell: three signed bytes
+    const double* rinv;    // 1 / rad of each shell
+    const int32_t* win;    // per shell s: last m1 with rad < rad[s] + 2, last with <=, first
+                           // with rad > rad[s] - 2 (not below 0)
+};
+
+__device__ __forceinline__ int blocks_of(int stop) { return (stop >> 2) + 1; }
+
+__global__ void block_count_kernel(const int32_t* __restrict__ vals,
+                                   const int32_t* __restrict__ stop, int64_t ntot,
+                                   int32_t* __restrict__ cnt) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < ntot) cnt[q] = blocks_of(stop[vals ? vals[q] : q]);
+}
+
+__global__ void block_base_kernel(const int32_t* __restrict__ vals,
+                                  const int64_t* __restrict__ off, int64_t ntot,
+                                  int64_t* __restrict__ base) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < ntot) base[vals ? vals[q] : q] = off[q];
+}
+
+// index of the r-th set bit of m (r < popcount)
+__device__ __forceinline__ int nth_bit(uint64_t m, int r) {
+    int pos = 0;
+#pragma unroll
+    for (int w = 32; w >= 1; w >>= 1) {
+        const uint64_t low = m & ((1ull << w) - 1ull);
+        const int c = __popcll(low);
+        const bool up = r >= c;
+        r -= up ? c : 0;
+        pos += up ? w : 0;
+        m = up ? m >> w : low;
+    }
+    return pos;
+}
+
+__device__ __forceinline__ int byte_of(uint32_t w, int q) {
+    return (int)(int8_t)((w >> (8 * q)) & 0xffu);
+}
+
+// a / r, correctly rounded, with y = 1 / r correctly rounded: two Newton steps on the quotient
+// (the second, from a quotient already within an ulp, rounds it correctly: Markstein, IBM J.
+// Res. Dev. 34, 1990), 5 operations instead of the division's 12.  An infinite or NaN a keeps
+// its product.  Checked against the division in tests/test_shell_blocks_cpu.py.
+__device__ __forceinline__ double div_rad(double a, double r, double y) {
+    const double q0 = a * y;
+    const double q1 = fma(fma(-q0, r, a), y, q0);
+    const double q2 = fma(fma(-q1, r, a), y, q1);
+    return fabs(q0) <= 1.7976931348623157e308 ? q2 : q0;
+}
+
+// The peak's ball of radius R (cells) leaves the grid.
+__device__ __forceinline__ bool ball_outside(const TileDev& T, int ci, int cj, int ck, int R) {
+    return !(ci - R >= 1 && ci + R <= T.n && cj - R >= 1 && cj + R <= T.n && ck - R >= 1 &&
+             ck + R <= T.n);
+}
+
+// ------------------------------------------------------------------ gather from bricks
+// The blocks within BR_H cells (97 % of the 1024^3 tile's peaks entirely, 90 % of its cells):
+// a workgroup takes the peaks of one 16^3 brick of the first order and stages the brick with
+// an 8-cell halo, 32^3 floats of one field at a time, in LDS (128 KB of the CU's 160), each
+// wavefront load bringing whole rows; the items of the brick then sum their shells from LDS.
+// An item is a lane's; its offsets come from a table in LDS, so that a wavefront may mix
+// blocks (a brick has some 120 peaks, few of them deep).  One field needs 4 FP64 sums, so the
+// five fields take turns in the one box: with all eight values of a cell side by side the box
+// would hold a brick of 17 cells halo included.
+constexpr int BR_CORE = 16, BR_H = 8, BR_W = 32, BR_T = 1024;
+constexpr int BR_PK = 256;      // peaks at a time, at most
+constexpr int BR_SH = 64;       // shells within BR_H, at most
+constexpr int BR_CELLS = 2112;  // cells within BR_H (2109), padded
+constexpr int BR_ITEMS = 4864;  // items at a time (a brick of the 1024^3 tile has some 2900)
+
+struct BrickArgs {
+    const int64_t* start;   // [count + 1] sorted position of each brick's first peak
+    const int32_t* tile;    // [count]
+    const int32_t* count;
+    const int32_t* vals;    // global peak id by sorted position
+    const uint2* tab;       // [2][ncell]: box offset (16 bits) and offsets as Float16; then the
+                            // transposed field's
+    const uint8_t* order;   // [nsh] shells within BR_H by falling number of cells
+    int ncell, nsh;         // cells and shells within BR_H
+};
+
+// v times the Float16 in the low or high half of w, as a Float32 product: an FMA with mz = -0,
+// which leaves every product as it is (-0 and NaN included), in the form that takes the half as it
+// is (a conversion and a multiply otherwise: 3 of the 18 operations of a cell)
+template <bool HIGH>
+__device__ __forceinline__ float mul_half(float v, uint32_t w, float mz) {
+    float r;
+    if (HIGH)
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(v), "v"(w), "s"(mz));
+    else
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(v), "v"(w), "s"(mz));
+    return r;
+}
+
+// The box value at byte address `cen` + 4 (the signed 16-bit offset in the low half of w)
+__device__ __forceinline__ float box_at(uint32_t cen, uint32_t w) {
+    uint32_t at;
+    asm("v_mad_i32_i16 %0, %1, 4, %2" : "=v"(at) : "v"(w), "v"(cen));
+    return *(const __attribute__((address_space(3))) float*)at;
+}
+
+struct BrickLds {
+    float box[BR_W * BR_W * BR_W];
+    uint2 tab[BR_CELLS];
+    uint64_t mask[BR_SH * (BR_PK / 64)];
+    double rad[BR_SH], rinv[BR_SH];
+    int base[BR_PK];
+    int ctr[BLK_FIELDS], np, tot;
+    uint16_t cen[BR_PK], cenT[BR_PK];
+    uint16_t pre[BR_SH * (BR_PK / 64)];
+    uint16_t sstart[BR_SH + 1];
+    uint16_t item[BR_ITEMS];  // shell << 8 | peak, shells of most cells first
+    uint8_t stop[BR_PK];
+};
+static_assert(sizeof(BrickLds) <= 160 * 1024, "one brick per CU");
+
+template <bool VEC4>
+__device__ __forceinline__ void stage_box(float* box, const float* __restrict__ f, int n, int f0,
+                                          int r0, int q0, int64_t s1, int64_t s2) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // cells outside the grid are read as its nearest cell: no item that needs them is here
+    if (VEC4) {
+        const int fx = min(max(f0 + 4 * (lane & 7), 0), n - 4);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int g = k * (BR_T / 64) + wave, row = g * 8 + (lane >> 3);
+            const int r = min(max(r0 + (row & 31), 0), n - 1), q = min(max(q0 + (row >> 5), 0), n - 1);
+            __builtin_amdgcn_global_load_lds(
+                f + fx + r * s1 + q * s2,
+                (__attribute__((address_space(3))) void*)(box + g * 256), 16, 0, 0);
+        }
+    } else {
+        const int fx = min(max(f0 + (lane & 31), 0), n - 1);
+#pragma unroll 8
+        for (int k = 0; k < 32; ++k) {
+            const int g = k * (BR_T / 64) + wave, row = g * 2 + (lane >> 5);
+            const int r = min(max(r0 + (row & 31), 0), n - 1), q = min(max(q0 + (row >> 5), 0), n - 1);
+            __builtin_amdgcn_global_load_lds(
+                f + fx + r * s1 + q * s2,
+                (__attribute__((address_space(3))) void*)(box + g * 64), 4, 0, 0);
+        }
+    }
+}
+
+__device__ __forceinline__ void store4(double* __restrict__ p, double a, double b, double c,
+                                       double d) {
+    reinterpret_cast<double2*>(p)[0] = make_double2(a, b);
+    reinterpret_cast<double2*>(p)[1] = make_double2(c, d);
+}
+
+// The items of one field: sums of v, v dx, v dy, v dz (PLAIN: the first too) of every item's
+// shell.  A wavefront takes 64 items at a time.
+template <bool PLAIN>
+__device__ __forceinline__ void brick_items(BrickLds& L, int tot, int* ctr,
+                                            const uint16_t* __restrict__ cen,
+                                            double* __restrict__ line) {
+    const int lane = threadIdx.x & 63;
+    for (;;) {
+        int t0 = 0;
+        if (lane == 0) t0 = atomicAdd(ctr, 64);
+        t0 = __builtin_amdgcn_readfirstlane(t0);
+        if (t0 >= tot) break;
+        const int t = t0 + lane;
+        if (t >= tot) continue;
+        const int it = L.item[t], q = it & 255, s = it >> 8;
+        // LDS byte address of the peak's cell in the box
+        const uint32_t c0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)L.box + 4u * cen[q];
+        double* out = line + ((int64_t)L.base[q] * BLK + s) * 4;
+        double A = 0.0, A0 = 0.0, A1 = 0.0, A2 = 0.0;
+        if (s == 1) {
+            if (PLAIN) A = (double)box_at(c0, 0);
+        } else {
+            int c = L.sstart[s];
+            const int e = L.sstart[s + 1];
+            auto add = [&](float v, uint2 w) {
+                if (PLAIN) A += (double)v;
+                A0 += (double)mul_half<true>(v, w.x, -0.0f);
+                A1 += (double)mul_half<false>(v, w.y, -0.0f);
+                A2 += (double)mul_half<true>(v, w.y, -0.0f);
+            };
+            for (; c + 4 <= e; c += 4) {
+                uint2 w[4];
+                float v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) w[k] = L.tab[c + k];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = box_at(c0, w[k].x);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) add(v[k], w[k]);
+            }
+            if (c < e) {  // a shell's cells come in pairs
+                const uint2 w0 = L.tab[c], w1 = L.tab[c + 1];
+                const float v0 = box_at(c0, w0.x), v1 = box_at(c0, w1.x);
+                add(v0, w0);
+                add(v1, w1);
+            }
+            const double r = L.rad[s], y = L.rinv[s];
+            A0 = div_rad(A0, r, y);
+            A1 = div_rad(A1, r, y);
+            A2 = div_rad(A2, r, y);
+        }
+        if (PLAIN) store4(out, A, A0, A1, A2);
+        else store4(out, A0, A1, A2, 0.0);
+    }
+}
+
+template <bool VEC4>
+__global__ __launch_bounds__(BR_T) void gather_bricks_kernel(SAArgs a, BlockArgs B, BrickArgs K) {
+    extern __shared__ char lds_raw[];
+    BrickLds& L = *reinterpret_cast<BrickLds*>(lds_raw);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // runs of 64 bricks (a 64^3 brick) per XCD in turn
+    const int j = (int)(blockIdx.x >> 3);
+    const int k = (((j >> 6) << 3) + (int)(blockIdx.x & 7)) * 64 + (j & 63);
+    if (k >= *K.count) return;
+    const int64_t q0 = K.start[k], q1 = K.start[k + 1];
+    const TileDev& T = a.tiles[K.tile[k]];
+    {
+        // a brick lies in one chunk
+        const int64_t e = B.base[K.vals[q0]] - B.e0;
+        if (e < 0 || e >= B.ne) return;
+    }
+    const int p0 = (int)(K.vals[q0] - T.base);
+    const int ox = ((T.pi[p0] - 1) & ~(BR_CORE - 1)) - BR_H, oy = ((T.pj[p0] - 1) & ~(BR_CORE - 1)) - BR_H,
+              oz = ((T.pk[p0] - 1) & ~(BR_CORE - 1)) - BR_H;
+    const int nsh = K.nsh;  // shells 1 .. nsh
+    constexpr int NW = BR_PK / 64;
+    for (int s = tid; s <= nsh + 1; s += BR_T) {
+        // table start of shell s, s = nsh + 1 the end of the last one
+        L.sstart[s] = (uint16_t)(s < 1 ? 0 : s <= nsh ? a.shell_start[s - 1] : K.ncell);
+        if (s >= 1 && s <= nsh) {
+            L.rad[s] = a.rad[s];
+            L.rinv[s] = B.rinv[s];
+        }
+    }
+    int np = 0;
+    for (int64_t qs = q0; qs < q1; qs += np) {
+        const int npm = (int)min((int64_t)BR_PK, q1 - qs);
+        int stop = 0;  // shells of this thread's peak, 0: none here
+        if (tid < npm) {
+            const int64_t id = K.vals[qs + tid];
+            const int p = (int)(id - T.base);
+            const int ci = T.pi[p], cj = T.pj[p], ck = T.pk[p];
+            const int st = B.stop[id];
+            if (!ball_outside(T, ci, cj, ck, min(BR_H, (int)a.rad[st]))) stop = min(st, nsh);
+            const int x = ci - 1 - ox, y = cj - 1 - oy, z = ck - 1 - oz;
+            L.base[tid] = (int)(B.base[id] - B.e0);
+            L.cen[tid] = (uint16_t)(x + BR_W * y + BR_W * BR_W * z);
+            L.cenT[tid] = (uint16_t)(z + BR_W * x + BR_W * BR_W * y);
+            L.stop[tid] = (uint8_t)stop;
+        }
+        __syncthreads();
+        // as many peaks as the item list holds
+        if (wave == 0) {
+            int n = 0, sum = 0;
+            for (int w = 0; w < NW; ++w) {
+                const int i = w * 64 + lane;
+                int run = i < npm ? (int)L.stop[i] : 0;
+                for (int d = 1; d < 64; d <<= 1) {
+                    const int o = __shfl_up(run, d);
+                    if (lane >= d) run += o;
+                }
+                n += (int)__popcll(__ballot(i < npm && sum + run <= BR_ITEMS));
+                sum += __shfl(run, 63);
+            }
+            if (lane == 0) L.np = n;
+            if (lane < BLK_FIELDS) L.ctr[lane] = 0;
+        }
+        __syncthreads();
+        np = L.np;
+        if (wave < NW)
+            for (int i = 0; i < nsh; ++i) {
+                const uint64_t m = __ballot(tid < np && stop >= (int)K.order[i]);
+                if (lane == 0) L.mask[i * NW + wave] = m;
+            }
+        __syncthreads();
+        if (wave == 0) {
+            int mine[NW], all = 0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                mine[w] = lane < nsh ? __popcll(L.mask[lane * NW + w]) : 0;
+                all += mine[w];
+            }
+            int sum = all;
+            for (int d = 1; d < 64; d <<= 1) {
+                const int o = __shfl_up(sum, d);
+                if (lane >= d) sum += o;
+            }
+            int at = sum - all;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                if (lane < nsh) L.pre[lane * NW + w] = (uint16_t)at;
+                at += mine[w];
+            }
+            if (lane == 63) L.tot = sum;
+        }
+        __syncthreads();
+        for (int e = wave; e < nsh * NW; e += BR_T / 64) {
+            const uint64_t m = L.mask[e];
+            if ((m >> lane) & 1ull) {
+                const int r = __popcll(m & ((1ull << lane) - 1ull));
+                L.item[L.pre[e] + r] = (uint16_t)(((int)K.order[e / NW] << 8) | ((e & (NW - 1)) * 64 + lane));
+            }
+        }
+        const int tot = L.tot;
+        // the transposed delta first, then delta, psi_1 xyz through the other table
+        const float* const src[BLK_FIELDS] = {T.delta, T.delta, T.etax, T.etay, T.etaz};
+        for (int f = 0; f < BLK_FIELDS && tot > 0; ++f) {
+            if (f < 2)
+                for (int c = tid; c < K.ncell; c += BR_T) L.tab[c] = K.tab[(f == 0 ? K.ncell : 0) + c];
+            if (f == 0) stage_box<VEC4>(L.box, src[f], T.n, oz, ox, oy, T.s1, T.s2);
+            else stage_box<VEC4>(L.box, src[f], T.n, ox, oy, oz, T.s1, T.s2);
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            if (f == 0) brick_items<false>(L, tot, &L.ctr[0], L.cenT, B.line[1]);
+            else brick_items<true>(L, tot, &L.ctr[f], L.cen, B.line[f == 1 ? 0 : f]);
+            __syncthreads();
+        }
+        __syncthreads();
+    }
+}
+
+// Bricks of the first order: flags, then (after a scan of the flags) start and tile of each.
+__global__ void brick_head_kernel(const uint64_t* __restrict__ keys, int64_t ntot, int shift,
+                                  int32_t* __restrict__ flag) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < ntot) flag[q] = q == 0 || (keys[q] >> shift) != (keys[q - 1] >> shift);
+}
+
+__global__ void brick_list_kernel(const uint64_t* __restrict__ keys,
+                                  const int32_t* __restrict__ flag,
+                                  const int64_t* __restrict__ rank, int64_t ntot,
+                                  int64_t* __restrict__ start, int32_t* __restrict__ tile,
+                                  int32_t* __restrict__ count) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= ntot) return;
+    if (flag[q]) {
+        start[rank[q]] = q;
+        tile[rank[q]] = (int32_t)(keys[q] >> 50);
+    }
+    if (q == ntot - 1) {
+        start[rank[q] + flag[q]] = ntot;
+        *count = (int32_t)(rank[q] + flag[q]);
+    }
+}
+
+// Peaks the bricks do not gather entirely: those whose ball leaves the grid are appended to
+// their tile's slots of `slot` (all -1 before; cnt[1 + t] of them), for gather_blocks_kernel;
+// those that reach beyond BR_H to `far` (cnt[0] of them), tile << 32 | peak.
+__global__ void far_list_kernel(const TileDev* __restrict__ tiles, const uint64_t* __restrict__ keys,
+                                const int32_t* __restrict__ vals, const int32_t* __restrict__ stop,
+                                const double* __restrict__ rad, int64_t ntot, int nsh,
+                                const int64_t* __restrict__ tile_pad, int32_t* __restrict__ cnt,
+                                int32_t* __restrict__ slot, int64_t* __restrict__ far) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    bool deep = false;
+    int t = 0, p = 0;
+    if (q < ntot) {
+        t = (int)(keys[q] >> 50);
+        const TileDev& T = tiles[t];
+        const int64_t id = vals[q];
+        p = (int)(id - T.base);
+        const int s = stop[id];
+        if (ball_outside(T, T.pi[p], T.pj[p], T.pk[p], (int)rad[s]))
+            slot[tile_pad[t] + atomicAdd(&cnt[1 + t], 1)] = p;
+        else deep = s > nsh;
+    }
+    const int lane = threadIdx.x & 63;
+    const uint64_t m = __ballot(deep);
+    if (m == 0) return;
+    int at = 0;
+    if (lane == 0) at = atomicAdd(&cnt[0], (int)__popcll(m));
+    at = __builtin_amdgcn_readfirstlane(at) + (int)__popcll(m & ((1ull << lane) - 1ull));
+    if (deep) far[at] = ((int64_t)t << 32) | (int64_t)p;
+}
+
+// The shells beyond BR_H of the deep peaks, one field per launch: a wavefront per peak, a lane
+// per shell, read from the field as it is.  A peak's ball is read many times over (every lane
+// its own cells), its neighbours' balls overlap it (the list is in brick order), and a launch
+// of one field keeps what an XCD's resident peaks read within its L2; with the fields in turn,
+// or each peak's box brought into LDS first, four of five lines came from beyond it.
+constexpr int FAR_T = 256, FAR_WG = 4;  // workgroups per CU
+
+__global__ __launch_bounds__(FAR_T) void gather_far_kernel(SAArgs a, BlockArgs B,
+                                                           const int64_t* __restrict__ far,
+                                                           const int32_t* __restrict__ count,
+                                                           int nsh, int f) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    constexpr int NWV = FAR_T / 64;
+    const int nfar = *count, G = (int)(gridDim.x >> 3) * NWV;
+    const bool tr = f == 1;  // the transposed delta
+    // runs of 64 peaks per XCD in turn
+    for (int l = (int)(blockIdx.x >> 3) * NWV + wave;; l += G) {
+        const int i = (((l >> 6) << 3) + (int)(blockIdx.x & 7)) * 64 + (l & 63);
+        if ((l >> 6) * 512 >= nfar) break;
+        if (i >= nfar) continue;
+        const int64_t e = far[i];
+        const TileDev& T = a.tiles[__builtin_amdgcn_readfirstlane((int)(e >> 32))];
+        const int p = __builtin_amdgcn_readfirstlane((int)(e & 0xffffffff));
+        const int64_t eb = B.base[T.base + p] - B.e0;
+        if (eb < 0 || eb >= B.ne) continue;
+        const int stop = B.stop[T.base + p];
+        const int s1 = T.n, s2 = T.n * T.n;
+        const int ci = T.pi[p] - 1, cj = T.pj[p] - 1, ck = T.pk[p] - 1;
+        const float* __restrict__ src = f <= 1 ? T.delta : f == 2 ? T.etax : f == 3 ? T.etay : T.etaz;
+        // strides of i, j and k in the field read
+        const int ax = tr ? s1 : 1, ay = tr ? s2 : s1, az = tr ? 1 : s2;
+        src += (int64_t)ci * ax + (int64_t)cj * ay + (int64_t)ck * az;
+        for (int s = nsh + 1 + lane; s <= stop; s += 64) {
+            int c = a.shell_start[s - 1];
+            const int en = c + a.shell_count[s - 1];
+            double A = 0.0, A0 = 0.0, A1 = 0.0, A2 = 0.0;
+            auto at = [&](uint32_t w) {
+                return src[byte_of(w, 0) * ax + byte_of(w, 1) * ay + byte_of(w, 2) * az];
+            };
+            auto add = [&](float v, uint32_t w) {
+                A += (double)v;
+                A0 += (double)(v * (float)byte_of(w, 0));
+                A1 += (double)(v * (float)byte_of(w, 1));
+                A2 += (double)(v * (float)byte_of(w, 2));
+            };
+            for (; c + 8 <= en; c += 8) {
+                uint32_t w[8];
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) w[u] = B.cell8[c + u];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = at(w[u]);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) add(v[u], w[u]);
+            }
+            if (c < en) {  // up to seven more, loaded together
+                uint32_t w[7];
+                float v[7];
+#pragma unroll
+                for (int u = 0; u < 7; ++u) w[u] = B.cell8[min(c + u, en - 1)];
+#pragma unroll
+                for (int u = 0; u < 7; ++u) v[u] = at(w[u]);
+#pragma unroll
+                for (int u = 0; u < 7; ++u)
+                    if (c + u < en) add(v[u], w[u]);
+            }
+            const double r = a.rad[s], y = B.rinv[s];
+            A0 = div_rad(A0, r, y);
+            A1 = div_rad(A1, r, y);
+            A2 = div_rad(A2, r, y);
+            double* o = B.line[f] + (eb * BLK + s) * 4;
+            if (tr) store4(o, A0, A1, A2, 0.0);
+            else store4(o, A, A0, A1, A2);
+        }
+    }
+}
+
+// ------------------------------------------------------------------ gather from the fields
+struct BlockSums {
+    double F, G0, G1, G2, H0, H1, H2;
+    double S0, S1, S2, R00, R01, R02, R10, R11, R12, R20, R21, R22;
+    __device__ __forceinline__ void zero() {
+        F = G0 = G1 = G2 = H0 = H1 = H2 = 0.0;
+        S0 = S1 = S2 = R00 = R01 = R02 = R10 = R11 = R12 = R20 = R21 = R22 = 0.0;
+    }
+    // the reference's Float32 products, added in FP64
+    __device__ __forceinline__ void add(float d, float t, float x, float y, float z, float fx,
+                                        float fy, float fz) {
+        F += (double)d;
+        G0 += (double)(d * fx);
+        G1 += (double)(d * fy);
+        G2 += (double)(d * fz);
+        H0 += (double)(t * fx);
+        H1 += (double)(t * fy);
+        H2 += (double)(t * fz);
+        S0 += (double)x;
+        R00 += (double)(x * fx);
+        R01 += (double)(x * fy);
+        R02 += (double)(x * fz);
+        S1 += (double)y;
+        R10 += (double)(y * fx);
+        R11 += (double)(y * fy);
+        R12 += (double)(y * fz);
+        S2 += (double)z;
+        R20 += (double)(z * fx);
+        R21 += (double)(z * fy);
+        R22 += (double)(z * fz);
+    }
+};
+
+
+struct BlockFields {
+    const float *d, *x, *y, *z;
+};
+
+// The shell's sums of one lane: cells [st, st + nc) of the table around the peak whose cell is
+// c0 (cT in the transposed field).  CHECK: some lane's ball leaves the grid; its cells outside
+// are skipped.
+template <bool CHECK>
+__device__ __forceinline__ void block_shell(const BlockFields& f, const uint32_t* __restrict__ cell8,
+                                            int st, int nc, int n, int ci, int cj, int ck,
+                                            int64_t c0, int64_t cT, BlockSums& A) {
+    const int s1 = n, s2 = n * n;
+    constexpr int U = CHECK ? 1 : 4;
+    int c = 0;
+    if (!CHECK) {
+        for (; c + U <= nc; c += U) {
+            uint32_t w[U];
+            float d[U], t[U], x[U], y[U], z[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) w[u] = cell8[st + c + u];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int ox = byte_of(w[u], 0), oy = byte_of(w[u], 1), oz = byte_of(w[u], 2);
+                const int64_t o = c0 + (ox + oy * s1 + oz * s2);
+                d[u] = f.d[o];
+                t[u] = f.d[cT + (oz + ox * s1 + oy * s2)];
+                x[u] = f.x[o];
+                y[u] = f.y[o];
+                z[u] = f.z[o];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                A.add(d[u], t[u], x[u], y[u], z[u], (float)byte_of(w[u], 0),
+                      (float)byte_of(w[u], 1), (float)byte_of(w[u], 2));
+        }
+    }
+    for (; c < nc; ++c) {
+        const uint32_t w = cell8[st + c];
+        const int ox = byte_of(w, 0), oy = byte_of(w, 1), oz = byte_of(w, 2);
+        if (CHECK) {
+            const int i1 = ci + ox, i2 = cj + oy, i3 = ck + oz;
+            if (i1 < 1 || i1 > n || i2 < 1 || i2 > n || i3 < 1 || i3 > n) continue;
+        }
+        const int64_t o = c0 + (ox + oy * s1 + oz * s2);
+        A.add(f.d[o], f.d[cT + (oz + ox * s1 + oy * s2)], f.x[o], f.y[o], f.z[o], (float)ox,
+              (float)oy, (float)oz);
+    }
+}
+
+// Gather of the blocks of 64 schedule slots (a workgroup per group and share of its items):
+// the first wavefront lists, for each block index b, which of the group's peaks reach it; item
+// t is the (t - first item of b)-th of them.
+__global__ __launch_bounds__(256) void gather_blocks_kernel(SAArgs a, BlockArgs B, int64_t g0,
+                                                            int64_t ng, int shares) {
+    extern __shared__ uint64_t lds[];
+    const int nbmax = (a.NS >> 2) + 1;
+    uint64_t* mask = lds;                    // [nbmax] peaks with more than b blocks
+    int* pre = (int*)(mask + nbmax);         // [nbmax + 1] items before block b
+    __shared__ int64_t s_base[64];
+    __shared__ int s_pos[3][64], s_stop[64], s_out[64], s_nb;
+    // contiguous runs of groups per XCD (workgroups are dealt to the XCDs in turn)
+    const int64_t nwg = (int64_t)gridDim.x, per = nwg >> 3;
+    const int64_t w = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    const int64_t g = g0 + w / shares;
+    const int share = (int)(w % shares);
+    if (g >= g0 + ng) return;
+    const TileDev& T = a.tiles[a.gtile[g]];
+    const int tid = threadIdx.x;
+    if (tid < 64) {
+        const int p = a.slot[g * 64 + tid];
+        int nb = 0;
+        if (p >= 0) {
+            const int64_t b0 = B.base[T.base + p] - B.e0;
+            if (b0 >= 0 && b0 < B.ne) {
+                const int stop = B.stop[T.base + p], R = (int)a.rad[stop];
+                const int ci = T.pi[p], cj = T.pj[p], ck = T.pk[p];
+                nb = blocks_of(stop);
+                s_base[tid] = b0;
+                s_stop[tid] = stop;
+                s_pos[0][tid] = ci;
+                s_pos[1][tid] = cj;
+                s_pos[2][tid] = ck;
+                s_out[tid] = ball_outside(T, ci, cj, ck, R);
+            }
+        }
+        int sum = 0, b = 0;
+        for (; b < nbmax; ++b) {
+            const uint64_t m = __ballot(nb > b);
+            if (m == 0) break;
+            if (tid == 0) {
+                mask[b] = m;
+                pre[b] = sum;
+            }
+            sum += __popcll(m);
+        }
+        if (tid == 0) {
+            pre[b] = sum;
+            s_nb = b;
+        }
+    }
+    __syncthreads();
+    const int nb = s_nb, tot = pre[nb];
+    const BlockFields f{T.delta, T.etax, T.etay, T.etaz};
+    for (int t0 = share * 256 + (tid & ~63); t0 < tot; t0 += 256 * shares) {
+        const int t = t0 + (tid & 63);
+        const bool on = t < tot;
+        int lo = 0, hi = nb - 1;  // last b with pre[b] <= t
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (pre[mid] <= t) lo = mid;
+            else hi = mid - 1;
+        }
+        const int b = lo;
+        const int q = on ? nth_bit(mask[b], t - pre[b]) : 0;
+        const int stop = on ? s_stop[q] : 0;
+        const int ci = s_pos[0][q], cj = s_pos[1][q], ck = s_pos[2][q];
+        const int n = T.n;
+        const int64_t c0 = (int64_t)(ci - 1) + (cj - 1) * T.s1 + (ck - 1) * T.s2;
+        const int64_t cT = (int64_t)(ck - 1) + (ci - 1) * T.s1 + (cj - 1) * T.s2;
+        const bool check = __ballot(on && s_out[q]) != 0ull;
+        const int64_t e = on ? s_base[q] + b : 0;
+        for (int u = 0; u < BLK; ++u) {
+            const int s = BLK * b + u;
+            if (s < 1 || s > stop) continue;
+            BlockSums A;
+            A.zero();
+            if (s == 1) {
+                // the peak's cell: its values and no first-order terms
+                A.F = (double)f.d[c0];
+                A.S0 = 0.0 + (double)f.x[c0];
+                A.S1 = 0.0 + (double)f.y[c0];
+                A.S2 = 0.0 + (double)f.z[c0];
+            } else {
+                const int st = a.shell_start[s - 1], nc = a.shell_count[s - 1];
+                if (check) block_shell<true>(f, B.cell8, st, nc, n, ci, cj, ck, c0, cT, A);
+                else block_shell<false>(f, B.cell8, st, nc, n, ci, cj, ck, c0, cT, A);
+                const double r = a.rad[s], y = B.rinv[s];
+                for (double* v : {&A.G0, &A.G1, &A.G2, &A.H0, &A.H1, &A.H2, &A.R00, &A.R01, &A.R02,
+                                  &A.R10, &A.R11, &A.R12, &A.R20, &A.R21, &A.R22})
+                    *v = div_rad(*v, r, y);
+            }
+            const int64_t o = (e * BLK + u) * 4;
+            store4(B.line[0] + o, A.F, A.G0, A.G1, A.G2);
+            store4(B.line[1] + o, A.H0, A.H1, A.H2, 0.0);
+            store4(B.line[2] + o, A.S0, A.R00, A.R01, A.R02);
+            store4(B.line[3] + o, A.S1, A.R10, A.R11, A.R12);
+            store4(B.line[4] + o, A.S2, A.R20, A.R21, A.R22);
+        }
+    }
+}
+
+// Cells of shell s inside the grid around a peak (all of them unless the ball leaves it).
+__device__ __forceinline__ int shell_cells_in(const SAArgs& a, const TileDev& T, int s, int ci,
+                                              int cj, int ck, bool out) {
+    const int nc = a.shell_count[s - 1];
+    if (!out) return nc;
+    const int st = a.shell_start[s - 1];
+    int in = 0;
+    for (int c = 0; c < nc; ++c) {
+        const int4 o = a.cells[st + c];
+        const int i1 = ci + o.x, i2 = cj + o.y, i3 = ck + o.z;
+        in += i1 >= 1 && i1 <= T.n && i2 >= 1 && i2 <= T.n && i3 >= 1 && i3 <= T.n;
+    }
+    return in;
+}
+
+// Fbar of every gathered shell (RadialShell.jl:410-416), a lane per peak of slots
+// [s0, s0 + ns): a serial recurrence over the shells' delta sums.
+__global__ __launch_bounds__(64) void block_fbar_kernel(SAArgs a, BlockArgs B, int64_t g0) {
+    const int64_t g = g0 + blockIdx.x;
+    const TileDev& T = a.tiles[a.gtile[g]];
+    const int p = a.slot[g * 64 + threadIdx.x];
+    if (p < 0) return;
+    const int64_t eb = B.base[T.base + p] - B.e0;
+    if (eb < 0 || eb >= B.ne) return;
+    const int stop = B.stop[T.base + p];
+    const int ci = T.pi[p], cj = T.pj[p], ck = T.pk[p];
+    const bool out = ball_outside(T, ci, cj, ck, (int)a.rad[stop]);
+    const double* L = B.line[0] + eb * BLK * 4;
+    double* fb = B.fb + eb * BLK;
+    // the four sums of a block's line together, the next line's on their way meanwhile (shell by
+    // shell, with 32 wavefronts per CU, every sum fetched its line anew)
+    double Fprev = L[4], dFbarp = Fprev, Fn[BLK];
+#pragma unroll
+    for (int u = 0; u < BLK; ++u) Fn[u] = L[u * 4];
+    for (int s0 = 0; s0 <= stop; s0 += BLK) {
+        double F[BLK], Fb[BLK];
+#pragma unroll
+        for (int u = 0; u < BLK; ++u) F[u] = Fn[u];
+        if (s0 + BLK <= stop) {
+#pragma unroll
+            for (int u = 0; u < BLK; ++u) Fn[u] = L[(s0 + BLK + u) * 4];
+        }
+#pragma unroll
+        for (int u = 0; u < BLK; ++u) {
+            const int s = s0 + u;
+            if (s >= 2 && s <= stop) {
+                const int nin = shell_cells_in(a, T, s, ci, cj, ck, out);
+                const double dFbar = nin > 0 ? F[u] / (double)nin : 0.0;
+                const double rad3p = cube(a.rad[s - 1]), rad3 = cube(a.rad[s]);
+                Fprev = (rad3p * Fprev + 0.5 * (dFbarp + dFbar) * (rad3 - rad3p)) / rad3;
+                dFbarp = dFbar;
+            }
+            Fb[u] = Fprev;
+        }
+        store4(fb + s0, Fb[0], Fb[1], Fb[2], Fb[3]);
+    }
+}
+
+// Sbar and Sbar2 of the collapsed peaks: the sums of psi_1 (from the profile) and psi_2 over
+// shells 1 .. mc - 1, added shell by shell, over their cells.  The psi_2 sums are needed here
+// only and up to there, so they are gathered here, a lane per peak and component (workgroup y),
+// rather than with every shell of every peak.
+__global__ __launch_bounds__(64) void block_sbar_kernel(SAArgs a, BlockArgs B, int64_t g0) {
+    const int64_t g = g0 + blockIdx.x;
+    const int l = blockIdx.y;
+    const TileDev& T = a.tiles[a.gtile[g]];
+    const int p = a.slot[g * 64 + threadIdx.x];
+    if (p < 0) return;
+    const int64_t eb = B.base[T.base + p] - B.e0;
+    if (eb < 0 || eb >= B.ne) return;
+    const int mc = B.cross[T.base + p];
+    if (mc <= 0) return;
+    const int ci = T.pi[p], cj = T.pj[p], ck = T.pk[p];
+    const bool out = ball_outside(T, ci, cj, ck, (int)a.rad[mc - 1]);
+    const int64_t c0 = (int64_t)(ci - 1) + (cj - 1) * T.s1 + (ck - 1) * T.s2;
+    const double* __restrict__ L = B.line[2 + l] + eb * BLK * 4;
+    const float* __restrict__ e2 = l == 0 ? T.eta2x : (l == 1 ? T.eta2y : T.eta2z);
+    const int s1 = (int)T.s1, s2 = (int)T.s2;
+    double cS = L[4], cT = T.has_eta2 ? 0.0 + (double)e2[c0] : 0.0, cN = 1.0;
+    auto off = [&](uint32_t w) {
+        return c0 + (byte_of(w, 0) + byte_of(w, 1) * s1 + byte_of(w, 2) * s2);
+    };
+    for (int s = 2; s <= mc - 1; ++s) {
+        const int st = a.shell_start[s - 1], nc = a.shell_count[s - 1];
+        double A = 0.0;
+        int nin = nc;
+        if (!out) {
+            if (T.has_eta2) {
+                int c = 0;
+                for (; c + 8 <= nc; c += 8) {
+                    float v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = e2[off(B.cell8[st + c + u])];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) A += (double)v[u];
+                }
+                if (c < nc) {  // up to seven more, loaded together
+                    float v[7];
+#pragma unroll
+                    for (int u = 0; u < 7; ++u) v[u] = e2[off(B.cell8[st + min(c + u, nc - 1)])];
+#pragma unroll
+                    for (int u = 0; u < 7; ++u)
+                        if (c + u < nc) A += (double)v[u];
+                }
+            }
+        } else {
+            nin = 0;
+            for (int c = 0; c < nc; ++c) {
+                const uint32_t w = B.cell8[st + c];
+                const int i1 = ci + byte_of(w, 0), i2 = cj + byte_of(w, 1), i3 = ck + byte_of(w, 2);
+                if (i1 < 1 || i1 > T.n || i2 < 1 || i2 > T.n || i3 < 1 || i3 > T.n) continue;
+                nin += 1;
+                if (T.has_eta2) A += (double)e2[off(w)];
+            }
+        }
+        if (nin > 0) {
+            cN += (double)nin;
+            cS += L[s * 4];
+            cT += A;
+        }
+    }
+    if (cN > 0.0) {
+        cS /= cN;
+        cT /= cN;
+    }
+    const int64_t o = (int64_t)p * 3 + l;
+    T.res.Sbar[o] = cS;
+    T.res.Sbar2[o] = cT;
+}
+
+// ------------------------------------------------------------------ radial logic by rows
+// W lanes per peak (a row): the walk's kernel_strain, eigenvalues and table lookup at shell mp
+// depend on mp only, not on the shells before it, so the row evaluates W shells at once and
+// takes the first that collapses; every lane of the row reads the same profile entry, once for
+// W steps.  The formation redshift's ten radii, the final strain's eigenvalues and the
+// filter-scale gradients are one more batch or three.
+
+// kernel_strain of a row: lane l's shell mp with window [mlow, mupp], for lanes with `on`;
+// eb = first block of the row's peak.  The sums run over the shells in ascending order, as
+// kstrain's.
+template <int W>
+__device__ __forceinline__ KS kstrain_row(const SAArgs& a, const BlockArgs& B, int64_t eb, int mp,
+                                          int mlow, int mupp, bool on) {
+    KS r = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const int mpc = on ? mp : 1;
+    const int lo0 = a.kidx[3 * mpc], hi0 = a.kidx[3 * mpc + 1];
+    const double* __restrict__ wt0 = a.kw + (a.kidx[3 * mpc + 2] - lo0);
+    const int lo = on ? (mlow > lo0 ? mlow : lo0) : 0x7fff;
+    const int hi = on ? (mupp < hi0 ? mupp : hi0) : -1;
+    int rlo = lo, rhi = hi;
+#pragma unroll
+    for (int d = 1; d < W; d <<= 1) {
+        rlo = min(rlo, __shfl_xor(rlo, d, W));
+        rhi = max(rhi, __shfl_xor(rhi, d, W));
+    }
+    const int64_t o0 = eb * BLK * 4;
+    for (int m1 = rlo; m1 <= rhi; ++m1) {
+        const int64_t o = o0 + (int64_t)m1 * 4;
+        const double2 ga = *reinterpret_cast<const double2*>(B.line[0] + o);
+        const double2 gb = *reinterpret_cast<const double2*>(B.line[0] + o + 2);
+        const double2 ha = *reinterpret_cast<const double2*>(B.line[1] + o);
+        const double h2 = B.line[1][o + 2];
+        const double2 xa = *reinterpret_cast<const double2*>(B.line[2] + o);
+        const double2 xb = *reinterpret_cast<const double2*>(B.line[2] + o + 2);
+        const double2 ya = *reinterpret_cast<const double2*>(B.line[3] + o);
+        const double2 yb = *reinterpret_cast<const double2*>(B.line[3] + o + 2);
+        const double2 za = *reinterpret_cast<const double2*>(B.line[4] + o);
+        const double2 zb = *reinterpret_cast<const double2*>(B.line[4] + o + 2);
+        if (m1 >= lo && m1 <= hi) {
+            const double wt = wt0[m1], hw = 0.5 * wt;
+            r.g0 += wt * ga.y;
+            r.g1 += wt * gb.x;
+            r.g2 += wt * gb.y;
+            r.f0 += wt * ha.x;
+            r.f1 += wt * ha.y;
+            r.f2 += wt * h2;
+            r.E11 -= hw * (xa.y + xa.y);
+            r.E12 -= hw * (xb.x + ya.y);
+            r.E13 -= hw * (xb.y + za.y);
+            r.E22 -= hw * (yb.x + yb.x);
+            r.E23 -= hw * (yb.y + zb.x);
+            r.E33 -= hw * (zb.y + zb.y);
+        }
+    }
+    const double sc = mpc > 1 ? a.wRnor / a.rad[mpc] : a.aRnor;
+    r.E11 *= sc; r.E12 *= sc; r.E13 *= sc; r.E22 *= sc; r.E23 *= sc; r.E33 *= sc;
+    r.g0 *= sc; r.g1 *= sc; r.g2 *= sc; r.f0 *= sc; r.f1 *= sc; r.f2 *= sc;
+    return r;
+}
+
+__device__ __forceinline__ KS shfl_ks(const KS& k, int src) {
+    KS r;
+    r.E11 = __shfl(k.E11, src); r.E12 = __shfl(k.E12, src); r.E13 = __shfl(k.E13, src);
+    r.E22 = __shfl(k.E22, src); r.E23 = __shfl(k.E23, src); r.E33 = __shfl(k.E33, src);
+    r.g0 = __shfl(k.g0, src); r.g1 = __shfl(k.g1, src); r.g2 = __shfl(k.g2, src);
+    r.f0 = __shfl(k.f0, src); r.f1 = __shfl(k.f1, src); r.f2 = __shfl(k.f2, src);
+    return r;
+}
+
+__device__ __forceinline__ void pick_ks(KS& d, const KS& s, bool c) {
+    d.E11 = c ? s.E11 : d.E11; d.E12 = c ? s.E12 : d.E12; d.E13 = c ? s.E13 : d.E13;
+    d.E22 = c ? s.E22 : d.E22; d.E23 = c ? s.E23 : d.E23; d.E33 = c ? s.E33 : d.E33;
+    d.g0 = c ? s.g0 : d.g0; d.g1 = c ? s.g1 : d.g1; d.g2 = c ? s.g2 : d.g2;
+    d.f0 = c ? s.f0 : d.f0; d.f1 = c ? s.f1 : d.f1; d.f2 = c ? s.f2 : d.f2;
+}
+
+// Running lapd sum over the cells of shells 1 .. sR: variants B and C from the centre on,
+// skipping cells outside the grid; variant A without the centre, up to the first cell outside.
+__device__ double block_d2f(const SAArgs& a, const TileDev& T, int ci, int cj, int ck, int sR) {
+    const int64_t c0 = (int64_t)(ci - 1) + (cj - 1) * T.s1 + (ck - 1) * T.s2;
+    const bool varA = a.variant == HNT_VARIANT_A;
+    double lap = 0.0;
+    int64_t n = 0;
+    const int first = varA ? a.shell_start[1] : 0;
+    const int last = sR >= 1 ? a.shell_start[sR - 1] + a.shell_count[sR - 1] : 0;
+    for (int c = first; c < last; ++c) {
+        const int4 o = a.cells[c];
+        const int i1 = ci + o.x, i2 = cj + o.y, i3 = ck + o.z;
+        if (i1 < 1 || i1 > T.n || i2 < 1 || i2 > T.n || i3 < 1 || i3 > T.n) {
+            if (varA) break;
+            continue;
+        }
+        lap += (double)T.lapd[c0 + o.x + o.y * T.s1 + o.z * T.s2];
+        n += 1;
+    }
+    return n > 0 ? lap / (double)n : 0.0;
+}
+
+template <int W>
+__global__ __launch_bounds__(64) void radial_rows_kernel(SAArgs a, BlockArgs B, int64_t slot0,
+                                                         int64_t nslot) {
+    constexpr int NR = 64 / W;
+    const int lane = threadIdx.x, l = lane & (W - 1), row0 = lane & ~(W - 1);
+    const int64_t per = (int64_t)gridDim.x >> 3;
+    const int64_t w = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (w * NR >= nslot) return;
+    const int64_t sl = slot0 + w * NR + lane / W;
+    const TileDev& T = a.tiles[a.gtile[(slot0 + w * NR) >> 6]];
+    const int p = a.slot[sl];
+    int64_t eb = 0;
+    bool valid = p >= 0;
+    if (valid) {
+        eb = B.base[T.base + p] - B.e0;
+        valid = eb >= 0 && eb < B.ne;
+        if (!valid) eb = 0;
+    }
+    if (__ballot(valid) == 0ull) return;
+    const double* __restrict__ rad = a.rad;
+    const int m = a.NS - 1;
+    int ci = 1, cj = 1, ck = 1, ir2min = 0, scross = 0, stop = 1;
+    double ZZon = 0.0, fcrit = 0.0, Rf = 0.0;
+    if (valid) {
+        ci = T.pi[p];
+        cj = T.pj[p];
+        ck = T.pk[p];
+        ir2min = T.ir2min[p];
+        Rf = T.Rf[p];
+        ZZon = T.ZZon ? T.ZZon[p] : T.ZZon_s;
+        fcrit = T.fcrit ? T.fcrit[p] : T.fcrit_s;
+        scross = B.cross[T.base + p];
+        stop = B.stop[T.base + p];
+    }
+    const double* __restrict__ fb = B.fb + eb * BLK;
+
+    // m0: the walk's first shell and its window (RadialShell.jl:484-554)
+    int m0 = 1, mupp0 = 1;
+    bool live = valid;
+    if (valid) {
+        m0 = first_r2_gt(a.shell_r2, 2, m, ir2min);
+        if (m0 > m) m0 = m;
+        bool tail = false;  // no crossing within the hunt radius
+        if (fb[m0] >= fcrit) {
+            if (scross > 0) m0 = scross;
+            else tail = true;
+        } else {
+            bool found = false;
+            for (int mp = m0 - 1 > 1 ? m0 - 1 : 1; mp >= 1; --mp) {
+                if (fb[mp] >= fcrit) {
+                    found = true;
+                    break;
+                }
+                m0 = mp;
+            }
+            live = found;
+        }
+        mupp0 = tail ? m : B.win[3 * m0];
+        if (m0 == 1) live = false;
+    }
+    const int mlow0 = B.win[3 * m0 + 2];
+
+    // ---- walk: step 0 is m0 itself (no collapse test), step i shell m0 - i ----
+    bool hit_row = false;
+    int mc = 0;  // m0 of the collapse
+    double zvir1 = -1.0, zvir1p = -1.0, Frhoh = 0.0;
+    KS last = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, prev = last, carry = last;
+    double zcarry = -1.0;
+    for (int i0 = 0;; i0 += W) {
+        const int mp = m0 - (i0 + l);
+        const bool on = live && mp >= 1;
+        if (__ballot(on) == 0ull) break;
+        int mlow = 1, mupp = 0;
+        if (on) {
+            mlow = min(mlow0, B.win[3 * mp + 2]);
+            mupp = (i0 + l == 0 || mupp0 <= B.win[3 * mp + 1]) ? mupp0 : B.win[3 * mp];
+        }
+        const KS kk = kstrain_row<W>(a, B, eb, mp, mlow, mupp, on);
+        double zv = -1.0, Fr = 0.0;
+        if (on) {
+            double lam[3], e_mp, p_mp;
+            eig_ks(kk, lam);
+            ev_from_lam(lam, &Fr, &e_mp, &p_mp);
+            const double Fb = fb[mp];
+            if (i0 + l > 0 && Fb > 0.0) {
+                const double poe = e_mp < 1e-5 ? 0.0 : p_mp / e_mp;
+                zv = interp3(a.ct, log10(Fb), e_mp, poe);
+            }
+        }
+        const bool hit = on && i0 + l > 0 && zv >= ZZon;
+        const uint64_t hits = (__ballot(hit) >> row0) & (W == 64 ? ~0ull : ((1ull << W) - 1ull));
+        const int hl = hits ? __ffsll((unsigned long long)hits) - 1 : 0;
+        const KS kl = shfl_ks(kk, row0 + hl);
+        const double zl = __shfl(zv, row0 + hl), fl = __shfl(Fr, row0 + hl);
+        const int pl = row0 + (hl > 0 ? hl - 1 : 0);
+        KS kp = shfl_ks(kk, pl);
+        double zp = __shfl(zv, pl);
+        pick_ks(kp, carry, hl == 0);
+        zp = hl == 0 ? zcarry : zp;
+        const bool take = hits != 0 && live;
+        pick_ks(last, kl, take);
+        pick_ks(prev, kp, take);
+        zvir1p = take ? zl : zvir1p;
+        zvir1 = take ? zp : zvir1;
+        Frhoh = take ? fl : Frhoh;
+        if (take) {
+            mc = m0 - (i0 + hl) + 1;
+            hit_row = true;
+            live = false;
+        }
+        carry = shfl_ks(kk, row0 + W - 1);
+        zcarry = __shfl(zv, row0 + W - 1);
+    }
+
+    double RTHL = 0.0;
+    const double dZvir = zvir1p - zvir1;
+    if (hit_row) {
+        if (zvir1 > 0.0 && dZvir != 0.0) {
+            const double RTHL3 = cube(rad[mc - 1]) + (cube(rad[mc]) - cube(rad[mc - 1])) *
+                                                         (zvir1p - ZZon) / dZvir;
+            RTHL = pow(RTHL3, 1.0 / 3.0);
+        } else {
+            RTHL = rad[mc - 1];
+        }
+        if (RTHL <= 0.0) hit_row = false;
+    }
+    if (valid && l == 0) {
+        if (T.res.nshells_used) T.res.nshells_used[p] = stop;
+        if (T.res.crossing_shell) T.res.crossing_shell[p] = scross;
+        if (T.res.bracket) T.res.bracket[p] = 0;
+        B.cross[T.base + p] = hit_row ? mc : 0;  // what block_sbar_kernel reads
+        if (!hit_row) {
+            write_no_collapse(T, p);
+            if (a.paint) a.paint[T.base + p] = -1;
+        }
+    }
+    if (__ballot(hit_row) == 0ull) return;
+    if (!hit_row) {
+        mc = 2;
+        RTHL = 1.0;
+    }
+
+    const double RTHL3 = cube(RTHL);
+    const double RTHL5 = RTHL3 * RTHL * RTHL;
+    const double rad3p = cube(rad[mc - 1]);
+    const double rad3 = cube(rad[mc]);
+    const double drad3 = rad3 - rad3p;
+    const double Fbm = hit_row ? fb[mc - 1] : 0.0, Fb0 = hit_row ? fb[mc] : 0.0;
+    double Fbarx;
+    KS fin;  // interpolated strain and gradients
+    if (zvir1 > 0.0 && drad3 != 0.0) {
+        const double frac = (RTHL3 - rad3p) / drad3;
+        Fbarx = Fbm + frac * (Fb0 - Fbm);
+        fin.E11 = last.E11 + frac * (prev.E11 - last.E11);
+        fin.E12 = last.E12 + frac * (prev.E12 - last.E12);
+        fin.E13 = last.E13 + frac * (prev.E13 - last.E13);
+        fin.E22 = last.E22 + frac * (prev.E22 - last.E22);
+        fin.E23 = last.E23 + frac * (prev.E23 - last.E23);
+        fin.E33 = last.E33 + frac * (prev.E33 - last.E33);
+        fin.g0 = last.g0 + frac * (prev.g0 - last.g0);
+        fin.g1 = last.g1 + frac * (prev.g1 - last.g1);
+        fin.g2 = last.g2 + frac * (prev.g2 - last.g2);
+        fin.f0 = last.f0 + frac * (prev.f0 - last.f0);
+        fin.f1 = last.f1 + frac * (prev.f1 - last.f1);
+        fin.f2 = last.f2 + frac * (prev.f2 - last.f2);
+    } else {
+        Fbarx = Fbm;
+        fin = prev;
+        fin.E11 = last.E11; fin.E12 = last.E12; fin.E13 = last.E13;
+        fin.E22 = last.E22; fin.E23 = last.E23; fin.E33 = last.E33;
+    }
+    const double tr = fin.E11 + fin.E22 + fin.E33;
+    if (tr != 0.0) {
+        const double sc = Fbarx / tr;
+        fin.E11 *= sc; fin.E12 *= sc; fin.E13 *= sc;
+        fin.E22 *= sc; fin.E23 *= sc; fin.E33 *= sc;
+    }
+
+    // ---- task 0: eigenvalues of the final strain; 1: filter-scale gradients; 2 .. 11: the
+    // formation redshift's radii (RadialShell.jl:801-859; variant B gives 0) ----
+    const bool half = a.variant != HNT_VARIANT_B && RTHL / 1.0 >= 3.0;
+    double zh = a.variant == HNT_VARIANT_B ? 0.0 : -1.0;
+    double lamf[3] = {0, 0, 0}, e_f = 0.0, p_f = 0.0;
+    const int ntask = half ? 12 : 2;
+    for (int t0 = 0; t0 < 12; t0 += W) {
+        const int t = t0 + l;
+        const bool on = hit_row && t < ntask;
+        if (__ballot(on) == 0ull) break;
+        int mp = 1, mlow = 1, mupp = 0;
+        const bool strain = on && t > 0;
+        if (strain && t == 1) {
+            rf_window(a, Rf, mp, mlow, mupp);
+        } else if (strain) {
+            const double rcur = RTHL * pow((double)(t - 2) / 9.0 * 0.5 + 0.5, 1.0 / 3.0);
+            mupp = 1;
+            if (m - 1 >= 2) {
+                const int f = first_gt(rad, 2, m - 1, rcur + 2.0);
+                mupp = f <= m - 1 ? f : m - 1;
+            }
+            double rl = rcur - 2.0;
+            if (rl < 0.0) rl = 0.0;
+            const int fl = first_gt(rad, 1, m - 1, rl);
+            mlow = fl <= m - 1 ? fl : 1;
+            if (m - 1 >= 1) {
+                const int f = first_gt(rad, 1, m - 1, rcur);
+                mp = f <= m - 1 ? f : m - 1;
+            }
+        }
+        const KS kr = kstrain_row<W>(a, B, eb, mp, mlow, mupp, strain);
+        if (on && t == 1) {
+            const int64_t o3 = (int64_t)p * 3;
+            T.res.gradpkrf[o3] = kr.g0;
+            T.res.gradpkrf[o3 + 1] = kr.g1;
+            T.res.gradpkrf[o3 + 2] = kr.g2;
+        } else if (on) {
+            const KS ke = t == 0 ? fin : kr;
+            double lam[3], Fr, ev, pv;
+            eig_ks(ke, lam);
+            ev_from_lam(lam, &Fr, &ev, &pv);
+            if (t == 0) {
+                lamf[0] = lam[0]; lamf[1] = lam[1]; lamf[2] = lam[2];
+                e_f = ev;
+                p_f = pv;
+            } else {
+                const double Fb = fb[mp];
+                const double poe = ev < 1e-5 ? 0.0 : pv / ev;
+                double zr = -1.0;
+                if (Fb > 0.0) zr = interp3(a.ct, log10(Fb), ev, poe);
+                const double zs = zr - 1.0;
+                if (zs > zh) zh = zs;
+            }
+        }
+    }
+#pragma unroll
+    for (int d = 1; d < W; d <<= 1) {
+        const double o = __shfl_xor(zh, d, W);
+        if (o > zh) zh = o;
+    }
+    if (!hit_row) return;
+
+    const hnt_results& R = T.res;
+    const int64_t o3 = (int64_t)p * 3;
+    if (l == 0) {
+        double Srb = 0.0, rad5p = 0.0;
+        if (mc > 2)
+            for (int mp = 2; mp <= mc - 1; ++mp) {
+                const double rad5 = pow5(rad[mp]);
+                Srb += 0.5 * (fb[mp - 1] + fb[mp]) * (rad5 - rad5p);
+                rad5p = rad5;
+            }
+        if (zvir1 > 0.0 && dZvir != 0.0) Srb += 0.5 * (Fbm + Fbarx) * (RTHL5 - rad5p);
+        if (Fbarx * RTHL5 > 0.0) Srb /= (Fbarx * RTHL5);
+        const int sR = first_gt(rad, 1, a.NS, RTHL) - 1;
+        if (a.paint) a.paint[T.base + p] = T.mask ? a.shell_r2[sR - 1] : -1;
+        double F11 = last.E11, F12 = last.E12, F13 = last.E13, F22 = last.E22, F23 = last.E23,
+               F33 = last.E33;
+        if (a.variant == HNT_VARIANT_A || Frhoh != 0.0) {
+            const double sc2 = Fbarx / Frhoh;
+            F11 *= sc2; F12 *= sc2; F13 *= sc2; F22 *= sc2; F23 *= sc2; F33 *= sc2;
+        }
+        R.RTHL[p] = RTHL;
+        R.Fbarx[p] = Fbarx;
+        R.e_v[p] = e_f;
+        R.p_v[p] = p_f;
+        R.Srb[p] = Srb;
+        R.d2F[p] = T.has_lapd ? block_d2f(a, T, ci, cj, ck, sR) : 0.0;
+        R.zvir_half[p] = zh;
+        double* sm = R.strain + (int64_t)p * 9;
+        sm[0] = F11; sm[1] = F12; sm[2] = F13;
+        sm[3] = F12; sm[4] = F22; sm[5] = F23;
+        sm[6] = F13; sm[7] = F23; sm[8] = F33;
+        R.eigs[o3] = lamf[0]; R.eigs[o3 + 1] = lamf[1]; R.eigs[o3 + 2] = lamf[2];
+        R.gradpk[o3] = fin.g0; R.gradpk[o3 + 1] = fin.g1; R.gradpk[o3 + 2] = fin.g2;
+        R.gradpkf[o3] = fin.f0; R.gradpkf[o3 + 1] = fin.f1; R.gradpkf[o3 + 2] = fin.f2;
+    }
+}
+
+// ------------------------------------------------------------------ crossing pass by rows
+// The crossing pass for few peaks: W lanes per peak, each summing one shell's delta, W shells
+// at a time; the Fbar recurrence then runs over their sums in order (every lane alike).  The
+// same sums and recurrence as crossing_kernel, which keeps a lane per peak: with tens of
+// thousands of wavefronts it wastes no shell beyond the crossing, but with few its time is
+// that of the deepest peak's whole chain of cells.
+template <int W>
+__global__ __launch_bounds__(64) void crossing_rows_kernel(SAArgs a, int32_t* __restrict__ stop_out,
+                                                           int32_t* __restrict__ cross_out) {
+    constexpr int NR = 64 / W;
+    const int lane = threadIdx.x, l = lane & (W - 1), row0 = lane & ~(W - 1);
+    const int64_t s0 = (int64_t)blockIdx.x * NR;
+    if (s0 >= a.ngroups * 64) return;
+    const TileDev& T = a.tiles[a.gtile[s0 >> 6]];
+    const int p = a.slot[s0 + lane / W];
+    const bool valid = p >= 0;
+    const int m = a.NS - 1;
+    int ci = 1, cj = 1, ck = 1, ir2min = 0;
+    double fcrit = 0.0, Rf = 0.0;
+    if (valid) {
+        ci = T.pi[p];
+        cj = T.pj[p];
+        ck = T.pk[p];
+        ir2min = T.ir2min[p];
+        Rf = T.Rf[p];
+        fcrit = T.fcrit ? T.fcrit[p] : T.fcrit_s;
+    }
+    const int64_t c0 = (int64_t)(ci - 1) + (cj - 1) * T.s1 + (ck - 1) * T.s2;
+    double Fprev = valid ? (double)T.delta[c0] : 0.0;
+    double dFbarp = Fprev;
+    bool active = valid, past = false;
+    int scross = 0;
+    for (int sb = 2; sb <= m; sb += W) {
+        if (__ballot(active) == 0ull) break;
+        const int s = sb + l;
+        double F = 0.0;
+        int64_t nin = 0;
+        // the shells of this batch that leave the grid are summed with the check
+        const bool out = ball_outside(T, ci, cj, ck, (int)a.rad[min(sb + W - 1, m)]);
+        if (active && s <= m) {
+            const int st = a.shell_start[s - 1], nc = a.shell_count[s - 1];
+            if (!out) cross_shell_hbm<false>(a, T, st, nc, ci, cj, ck, c0, F, nin);
+            else cross_shell_hbm<true>(a, T, st, nc, ci, cj, ck, c0, F, nin);
+        }
+        const int nin32 = (int)nin;
+        for (int j = 0; j < W && sb + j <= m; ++j) {
+            const double Fj = __shfl(F, row0 + j);
+            const int nj = __shfl(nin32, row0 + j);
+            if (active)
+                cross_step(a, sb + j, Fj, nj, ir2min, fcrit, Fprev, dFbarp, past, active, scross);
+        }
+    }
+    if (!valid || l != 0) return;
+    stop_out[T.base + p] = crossing_stop(a, Rf, scross);
+    cross_out[T.base + p] = scross;
+}
+
+// Chunk boundaries of a schedule too large for one profile buffer: boundary c is the start
+// (sorted position) of the brick holding the first peak whose profile begins at or after
+// block c * cap; out[2 c] the position, out[2 c + 1] its first block.
+__global__ void chunk_bounds_kernel(const uint64_t* __restrict__ keys,
+                                    const int64_t* __restrict__ off, int64_t ntot, int shift,
+                                    int64_t cap, int nchunk, int64_t* __restrict__ out) {
+    const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (c >= nchunk) return;
+    int64_t lo = 0, hi = ntot;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (off[mid] < (int64_t)c * cap) lo = mid + 1;
+        else hi = mid;
+    }
+    if (lo < ntot) {
+        const uint64_t brick = keys[lo] >> shift;
+        int64_t l2 = 0, h2 = lo;
+        while (l2 < h2) {
+            const int64_t mid = (l2 + h2) >> 1;
+            if ((keys[mid] >> shift) < brick) l2 = mid + 1;
+            else h2 = mid;
+        }
+        lo = l2;
+    }
+    out[2 * c] = lo;
+    out[2 * c + 1] = lo < ntot ? off[lo] : -1;
+}
