@@ -106,7 +106,7 @@ struct Arena {
 struct SAWork {
     DevBuf recs, keys_a, keys_b, vals_a, vals_b, cub_tmp, slots, gtiles, tiles, tilemeta, stops,
         feats, prof, queue, flag, skip, paint, cross, bcnt, boff, bbase, slots2,
-        slots3, brick, far;
+        slots3, brick, far, walk;
     std::vector<TileDev> tile_host;
     std::vector<int64_t> meta_host;
     bool own_tables = false;

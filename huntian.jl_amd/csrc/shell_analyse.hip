@@ -2006,14 +2006,14 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     int32_t* stops = (int32_t*)W.stops.p;
     int32_t* cross = (int32_t*)W.cross.p;
     const bool few = ntot < (1 << 17);
-    if (few) {
-        hipLaunchKernelGGL(crossing_rows_kernel<16>, dim3((unsigned)(ngroups * 16)), dim3(64), 0, st,
-                           A, stops, cross);
-    } else {
-        const int64_t G8 = (ngroups + 7) / 8;
-        hipLaunchKernelGGL(crossing_kernel, dim3((unsigned)(8 * G8)), dim3(64), 0, st, A, G8,
-                           stops, cross);
-    }
+    const auto row_grid = [](int64_t groups, int w) { return (unsigned)(8 * ((groups * w + 7) / 8)); };
+    const uint32_t* cell8 = (const uint32_t*)TT.cell8.p;
+    if (few)
+        hipLaunchKernelGGL(crossing_rows_kernel<16>, dim3(row_grid(ngroups, 16)), dim3(64), 0, st, A,
+                           cell8, stops, cross);
+    else
+        hipLaunchKernelGGL(crossing_rows_kernel<4>, dim3(row_grid(ngroups, 4)), dim3(64), 0, st, A,
+                           cell8, stops, cross);
     std::vector<const int32_t*> prim((size_t)ntiles);
     for (int t = 0; t < ntiles; ++t) {
         prim[t] = stops + meta[t];
@@ -2130,9 +2130,8 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     B.cell8 = (const uint32_t*)TT.cell8.p;
     B.rinv = (const double*)TT.rinv.p;
     B.win = (const int32_t*)TT.win.p;
-    double* q = (double*)W.prof.p;
-    for (int f = 0; f < BLK_FIELDS; ++f) B.line[f] = q + (int64_t)f * cap * 4 * BLK;
-    B.fb = q + (int64_t)BLK_FIELDS * cap * 4 * BLK;
+    B.prof = (double*)W.prof.p;
+    B.fb = B.prof + cap * BLK_LINES;
     // sorted position -> slot: a tile's slots start at a multiple of 64
     auto slot_of = [&](int64_t at) {
         int t = 0;
@@ -2155,6 +2154,10 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
                                     hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(BrickLds)));
     }
     const size_t lds = (size_t)nbmax * 8 + (size_t)(nbmax + 1) * 4;
+    HNT_TRY(reserve(ctx, W.walk, (size_t)ngroups * 64 * (sizeof(WalkState) + 4) + 4));
+    WalkState* ws = (WalkState*)W.walk.p;
+    int32_t* half = (int32_t*)(ws + ngroups * 64);
+    int32_t* hcnt = half + ngroups * 64;
     for (size_t c = 0; c + 1 < pos.size(); ++c) {
         B.e0 = first[c];
         B.ne = first[c + 1] - first[c];
@@ -2184,13 +2187,21 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
         hipLaunchKernelGGL(block_fbar_kernel, dim3((unsigned)ng), dim3(64), 0, st, A, B, g0);
         SAArgs A2 = A;
         A2.slot = slot2;
+        const int64_t nsl = ng * 64;
+        hipLaunchKernelGGL(fill_i32, dim3(1), dim3(64), 0, st, hcnt, (int64_t)1, 0);
+        const auto rows = [&](int w) { return dim3(row_grid(ng, w)); };
         if (few)
-            hipLaunchKernelGGL(radial_rows_kernel<16>, dim3((unsigned)(8 * ((ng * 16 + 7) / 8))),
-                               dim3(64), 0, st, A2, B, s0, ng * 64);
+            hipLaunchKernelGGL(walk_rows_kernel<16>, rows(16), dim3(64), 0, st, A2, B, s0, nsl, ws);
         else
-            hipLaunchKernelGGL(radial_rows_kernel<4>, dim3((unsigned)(8 * ((ng * 4 + 7) / 8))),
-                               dim3(64), 0, st, A2, B, s0, ng * 64);
-        hipLaunchKernelGGL(block_sbar_kernel, dim3((unsigned)ng, 3), dim3(64), 0, st, A, B, g0);
+            hipLaunchKernelGGL(walk_rows_kernel<4>, rows(4), dim3(64), 0, st, A2, B, s0, nsl, ws);
+        hipLaunchKernelGGL(finish_rows_kernel, rows(4), dim3(64), 0, st, A2, B, s0, nsl,
+                           (const WalkState*)ws, half, hcnt);
+        if (A.variant != HNT_VARIANT_B)
+            hipLaunchKernelGGL(half_rows_kernel,
+                               dim3((unsigned)std::min<int64_t>(nsl / 4, 16 * ctx->num_cus)), dim3(64), 0,
+                               st, A2, B, s0, (const WalkState*)ws, (const int32_t*)half,
+                               (const int32_t*)hcnt);
+        hipLaunchKernelGGL(sbar_rows_kernel, dim3(rows(4).x, 3), dim3(64), 0, st, A, B, s0, nsl);
     }
     stage_end(ctx, HNT_STAGE_SA_KERNEL);
     stage_begin(ctx, HNT_STAGE_SA_MASK);

@@ -12,17 +12,19 @@
 // them: no cell records are written.
 //
 // Measured against the lane-per-peak kernel with its records (same bits): shell analysis of the
-// 1024^3 tile 327 -> 264 ms, of the 512^3 tile 51.6 -> 32.5 ms, of a 128^3 tile 7.9 -> 1.5 ms, of a
-// 40^3 tile 1.37 -> 0.43 ms, of 24 tiles of 96^3 to 256^3 37 -> 26 ms.
+// 1024^3 tile 327 -> 225 ms, of the 512^3 tile 51.6 -> 27.3 ms, of a 128^3 tile 7.9 -> 1.38 ms, of a
+// 40^3 tile 1.33 -> 0.44 ms, of 24 tiles of 96^3 to 256^3 37.6 -> 21.6 ms.
 //
-// A block's sums are five 128-byte lines, one per field (delta, its transpose, psi_1 xyz),
-// four doubles per shell: {F, G0, G1, G2}, {H0, H1, H2, -}, {S, R0, R1, R2} x 3; G, H and R
-// divided by the shell's radius.  Shell s of a peak is entry 4 base + s (entry 0 unused).
+// A block's sums are five 128-byte lines side by side, one per field (delta, its transpose,
+// psi_1 xyz), four doubles per shell: {F, G0, G1, G2}, {H0, H1, H2, -}, {S, R0, R1, R2} x 3;
+// G, H and R divided by the shell's radius.  Shell s of a peak is in its block s / 4 (the
+// first block's shell 0 is unused).  What reads them takes four lanes per peak, a shell each: a
+// line is one peak's four lanes' 128 bytes, fetched once.
 
 constexpr int BLK = 4;          // shells per block
 constexpr int BLK_FIELDS = 5;   // lines per block
-// doubles of a block: five lines of 4 shells x 4 doubles, and Fbar of its 4 shells
-constexpr int BLK_DOUBLES = BLK_FIELDS * 4 * BLK + BLK;
+constexpr int BLK_LINES = BLK_FIELDS * 4 * BLK;  // doubles of a block's lines
+constexpr int BLK_DOUBLES = BLK_LINES + BLK;     // ... and Fbar of its 4 shells
 
 struct BlockArgs {
     const int32_t* stop;   // per global peak id: last shell of the gather
@@ -30,13 +32,18 @@ struct BlockArgs {
                            // logic on, the first shell beyond RTHL's, 0 = no collapse
     const int64_t* base;   // per global peak id: first block of its profile
     int64_t e0, ne;        // blocks [e0, e0 + ne) are the ones of this launch
-    double* line[BLK_FIELDS];
+    double* prof;          // [BLK_LINES ne] the blocks' lines
     double* fb;            // [4 ne] Fbar of each shell
     const uint32_t* cell8; // offsets of every table cell: three signed bytes
     const double* rinv;    // 1 / rad of each shell
     const int32_t* win;    // per shell s: last m1 with rad < rad[s] + 2, last with <=, first
                            // with rad > rad[s] - 2 (not below 0)
 };
+
+// Shell s of the profile that starts at block eb: its doubles of field f are at 4 BLK f.
+__device__ __forceinline__ double* entry_of(const BlockArgs& B, int64_t eb, int s) {
+    return B.prof + (eb + (s >> 2)) * BLK_LINES + (s & 3) * 4;
+}
 
 __device__ __forceinline__ int blocks_of(int stop) { return (stop >> 2) + 1; }
 
@@ -202,7 +209,7 @@ __device__ __forceinline__ void brick_items(BrickLds& L, int tot, int* ctr,
         const int it = L.item[t], q = it & 255, s = it >> 8;
         // LDS byte address of the peak's cell in the box
         const uint32_t c0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)L.box + 4u * cen[q];
-        double* out = line + ((int64_t)L.base[q] * BLK + s) * 4;
+        double* out = line + ((int64_t)L.base[q] + (s >> 2)) * BLK_LINES + (s & 3) * 4;
         double A = 0.0, A0 = 0.0, A1 = 0.0, A2 = 0.0;
         if (s == 1) {
             if (PLAIN) A = (double)box_at(c0, 0);
@@ -349,8 +356,8 @@ __global__ __launch_bounds__(BR_T) void gather_bricks_kernel(SAArgs a, BlockArgs
             else stage_box<VEC4>(L.box, src[f], T.n, ox, oy, oz, T.s1, T.s2);
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
-            if (f == 0) brick_items<false>(L, tot, &L.ctr[0], L.cenT, B.line[1]);
-            else brick_items<true>(L, tot, &L.ctr[f], L.cen, B.line[f == 1 ? 0 : f]);
+            if (f == 0) brick_items<false>(L, tot, &L.ctr[0], L.cenT, B.prof + 4 * BLK);
+            else brick_items<true>(L, tot, &L.ctr[f], L.cen, B.prof + 4 * BLK * (f == 1 ? 0 : f));
             __syncthreads();
         }
         __syncthreads();
@@ -482,7 +489,7 @@ __global__ __launch_bounds__(FAR_T) void gather_far_kernel(SAArgs a, BlockArgs B
             A0 = div_rad(A0, r, y);
             A1 = div_rad(A1, r, y);
             A2 = div_rad(A2, r, y);
-            double* o = B.line[f] + (eb * BLK + s) * 4;
+            double* o = entry_of(B, eb, s) + 4 * BLK * f;
             if (tr) store4(o, A0, A1, A2, 0.0);
             else store4(o, A, A0, A1, A2);
         }
@@ -664,12 +671,12 @@ __global__ __launch_bounds__(256) void gather_blocks_kernel(SAArgs a, BlockArgs 
                                   &A.R10, &A.R11, &A.R12, &A.R20, &A.R21, &A.R22})
                     *v = div_rad(*v, r, y);
             }
-            const int64_t o = (e * BLK + u) * 4;
-            store4(B.line[0] + o, A.F, A.G0, A.G1, A.G2);
-            store4(B.line[1] + o, A.H0, A.H1, A.H2, 0.0);
-            store4(B.line[2] + o, A.S0, A.R00, A.R01, A.R02);
-            store4(B.line[3] + o, A.S1, A.R10, A.R11, A.R12);
-            store4(B.line[4] + o, A.S2, A.R20, A.R21, A.R22);
+            double* o = B.prof + e * BLK_LINES + u * 4;
+            store4(o, A.F, A.G0, A.G1, A.G2);
+            store4(o + 16, A.H0, A.H1, A.H2, 0.0);
+            store4(o + 32, A.S0, A.R00, A.R01, A.R02);
+            store4(o + 48, A.S1, A.R10, A.R11, A.R12);
+            store4(o + 64, A.S2, A.R20, A.R21, A.R22);
         }
     }
 }
@@ -701,7 +708,7 @@ __global__ __launch_bounds__(64) void block_fbar_kernel(SAArgs a, BlockArgs B, i
     const int stop = B.stop[T.base + p];
     const int ci = T.pi[p], cj = T.pj[p], ck = T.pk[p];
     const bool out = ball_outside(T, ci, cj, ck, (int)a.rad[stop]);
-    const double* L = B.line[0] + eb * BLK * 4;
+    const double* L = B.prof + eb * BLK_LINES;
     double* fb = B.fb + eb * BLK;
     // the four sums of a block's line together, the next line's on their way meanwhile (shell by
     // shell, with 32 wavefronts per CU, every sum fetched its line anew)
@@ -714,7 +721,7 @@ __global__ __launch_bounds__(64) void block_fbar_kernel(SAArgs a, BlockArgs B, i
         for (int u = 0; u < BLK; ++u) F[u] = Fn[u];
         if (s0 + BLK <= stop) {
 #pragma unroll
-            for (int u = 0; u < BLK; ++u) Fn[u] = L[(s0 + BLK + u) * 4];
+            for (int u = 0; u < BLK; ++u) Fn[u] = L[(s0 / BLK + 1) * BLK_LINES + u * 4];
         }
 #pragma unroll
         for (int u = 0; u < BLK; ++u) {
@@ -732,69 +739,124 @@ __global__ __launch_bounds__(64) void block_fbar_kernel(SAArgs a, BlockArgs B, i
     }
 }
 
-// Sbar and Sbar2 of the collapsed peaks: the sums of psi_1 (from the profile) and psi_2 over
-// shells 1 .. mc - 1, added shell by shell, over their cells.  The psi_2 sums are needed here
-// only and up to there, so they are gathered here, a lane per peak and component (workgroup y),
-// rather than with every shell of every peak.
-__global__ __launch_bounds__(64) void block_sbar_kernel(SAArgs a, BlockArgs B, int64_t g0) {
-    const int64_t g = g0 + blockIdx.x;
-    const int l = blockIdx.y;
-    const TileDev& T = a.tiles[a.gtile[g]];
-    const int p = a.slot[g * 64 + threadIdx.x];
-    if (p < 0) return;
-    const int64_t eb = B.base[T.base + p] - B.e0;
-    if (eb < 0 || eb >= B.ne) return;
-    const int mc = B.cross[T.base + p];
-    if (mc <= 0) return;
-    const int ci = T.pi[p], cj = T.pj[p], ck = T.pk[p];
-    const bool out = ball_outside(T, ci, cj, ck, (int)a.rad[mc - 1]);
-    const int64_t c0 = (int64_t)(ci - 1) + (cj - 1) * T.s1 + (ck - 1) * T.s2;
-    const double* __restrict__ L = B.line[2 + l] + eb * BLK * 4;
-    const float* __restrict__ e2 = l == 0 ? T.eta2x : (l == 1 ? T.eta2y : T.eta2z);
+// v of lane S of each four lanes.
+template <int S>
+__device__ __forceinline__ double quad_of(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), S * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), S * 0x55, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// Rows of a launch: slots [slot0, slot0 + nslot), NR = 64 / W per wavefront, contiguous runs per
+// XCD.  False: this wavefront has no slot.
+template <int W>
+__device__ __forceinline__ bool row_slot(int64_t nslot, int64_t& first) {
+    constexpr int NR = 64 / W;
+    const int64_t per = (int64_t)gridDim.x >> 3;
+    first = ((int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3)) * NR;
+    return first < nslot;
+}
+
+// The sum of f over shell s around cell (ci, cj, ck), in the reference's order, and the number
+// of its cells inside the grid; out: some may lie outside.  No sum without f.
+__device__ __forceinline__ void shell_sum(const SAArgs& a, const uint32_t* __restrict__ cell8,
+                                          const TileDev& T, const float* __restrict__ f, int s,
+                                          int ci, int cj, int ck, int64_t c0, bool out, double& A,
+                                          int& nin) {
+    const int st = a.shell_start[s - 1], nc = a.shell_count[s - 1];
     const int s1 = (int)T.s1, s2 = (int)T.s2;
-    double cS = L[4], cT = T.has_eta2 ? 0.0 + (double)e2[c0] : 0.0, cN = 1.0;
     auto off = [&](uint32_t w) {
         return c0 + (byte_of(w, 0) + byte_of(w, 1) * s1 + byte_of(w, 2) * s2);
     };
-    for (int s = 2; s <= mc - 1; ++s) {
-        const int st = a.shell_start[s - 1], nc = a.shell_count[s - 1];
-        double A = 0.0;
-        int nin = nc;
-        if (!out) {
-            if (T.has_eta2) {
-                int c = 0;
-                for (; c + 8 <= nc; c += 8) {
-                    float v[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) v[u] = e2[off(B.cell8[st + c + u])];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) A += (double)v[u];
-                }
-                if (c < nc) {  // up to seven more, loaded together
-                    float v[7];
-#pragma unroll
-                    for (int u = 0; u < 7; ++u) v[u] = e2[off(B.cell8[st + min(c + u, nc - 1)])];
-#pragma unroll
-                    for (int u = 0; u < 7; ++u)
-                        if (c + u < nc) A += (double)v[u];
-                }
-            }
-        } else {
-            nin = 0;
-            for (int c = 0; c < nc; ++c) {
-                const uint32_t w = B.cell8[st + c];
-                const int i1 = ci + byte_of(w, 0), i2 = cj + byte_of(w, 1), i3 = ck + byte_of(w, 2);
-                if (i1 < 1 || i1 > T.n || i2 < 1 || i2 > T.n || i3 < 1 || i3 > T.n) continue;
-                nin += 1;
-                if (T.has_eta2) A += (double)e2[off(w)];
-            }
+    A = 0.0;
+    if (out) {
+        nin = 0;
+        for (int c = 0; c < nc; ++c) {
+            const uint32_t w = cell8[st + c];
+            const int i1 = ci + byte_of(w, 0), i2 = cj + byte_of(w, 1), i3 = ck + byte_of(w, 2);
+            if (i1 < 1 || i1 > T.n || i2 < 1 || i2 > T.n || i3 < 1 || i3 > T.n) continue;
+            nin += 1;
+            if (f) A += (double)f[off(w)];
         }
-        if (nin > 0) {
-            cN += (double)nin;
-            cS += L[s * 4];
-            cT += A;
-        }
+        return;
     }
+    nin = nc;
+    if (!f) return;
+    int c = 0;
+    for (; c + 8 <= nc; c += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = f[off(cell8[st + c + u])];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) A += (double)v[u];
+    }
+    if (c < nc) {  // up to seven more, loaded together
+        float v[7];
+#pragma unroll
+        for (int u = 0; u < 7; ++u) v[u] = f[off(cell8[st + min(c + u, nc - 1)])];
+#pragma unroll
+        for (int u = 0; u < 7; ++u)
+            if (c + u < nc) A += (double)v[u];
+    }
+}
+
+// Sbar and Sbar2 of the collapsed peaks: the sums of psi_1 (from the profile) and psi_2 over
+// shells 1 .. mc - 1, added shell by shell, over their cells.  The psi_2 sums are needed here
+// only and up to there, so they are gathered here rather than with every shell of every peak:
+// four lanes per peak and component (workgroup y), a shell each (one lane per peak: 3.3 -> 1.9 ms
+// for the 512^3 tile; 64 peaks' psi_2 rows per wavefront did not stay in the caches, 19 % hits).
+__global__ __launch_bounds__(64) void sbar_rows_kernel(SAArgs a, BlockArgs B, int64_t slot0,
+                                                       int64_t nslot) {
+    constexpr int W = 4;
+    const int lane = threadIdx.x, q = lane & (W - 1), l = blockIdx.y;
+    int64_t first;
+    if (!row_slot<W>(nslot, first)) return;
+    const TileDev& T = a.tiles[a.gtile[(slot0 + first) >> 6]];
+    const int p = a.slot[slot0 + first + lane / W];
+    int64_t eb = -1;
+    int mc = 0;
+    if (p >= 0) {
+        eb = B.base[T.base + p] - B.e0;
+        if (eb >= 0 && eb < B.ne) mc = B.cross[T.base + p];
+    }
+    const bool on = mc > 0;
+    if (__ballot(on) == 0ull) return;
+    int ci = 1, cj = 1, ck = 1;
+    bool out = false;
+    const float* __restrict__ e2 = l == 0 ? T.eta2x : (l == 1 ? T.eta2y : T.eta2z);
+    double cS = 0.0, cT = 0.0, cN = 1.0;
+    int64_t c0 = 0;
+    if (on) {
+        ci = T.pi[p];
+        cj = T.pj[p];
+        ck = T.pk[p];
+        out = ball_outside(T, ci, cj, ck, (int)a.rad[mc - 1]);
+        c0 = (int64_t)(ci - 1) + (cj - 1) * T.s1 + (ck - 1) * T.s2;
+        cS = entry_of(B, eb, 1)[4 * BLK * (2 + l)];
+        cT = T.has_eta2 ? 0.0 + (double)e2[c0] : 0.0;
+    }
+    for (int sb = 2; __ballot(sb <= mc - 1) != 0ull; sb += W) {
+        const int s = sb + q;
+        double A = 0.0, S = 0.0;
+        int nin = 0;
+        if (s <= mc - 1) {
+            S = entry_of(B, eb, s)[4 * BLK * (2 + l)];
+            shell_sum(a, B.cell8, T, T.has_eta2 ? e2 : nullptr, s, ci, cj, ck, c0, out, A, nin);
+        }
+        const double N = (double)nin;
+        auto take = [&](double n, double sv, double av) {
+            if (n > 0.0) {
+                cN += n;
+                cS += sv;
+                cT += av;
+            }
+        };
+        take(quad_of<0>(N), quad_of<0>(S), quad_of<0>(A));
+        take(quad_of<1>(N), quad_of<1>(S), quad_of<1>(A));
+        take(quad_of<2>(N), quad_of<2>(S), quad_of<2>(A));
+        take(quad_of<3>(N), quad_of<3>(S), quad_of<3>(A));
+    }
+    if (!on || q != 0) return;
     if (cN > 0.0) {
         cS /= cN;
         cT /= cN;
@@ -807,60 +869,117 @@ __global__ __launch_bounds__(64) void block_sbar_kernel(SAArgs a, BlockArgs B, i
 // ------------------------------------------------------------------ radial logic by rows
 // W lanes per peak (a row): the walk's kernel_strain, eigenvalues and table lookup at shell mp
 // depend on mp only, not on the shells before it, so the row evaluates W shells at once and
-// takes the first that collapses; every lane of the row reads the same profile entry, once for
-// W steps.  The formation redshift's ten radii, the final strain's eigenvalues and the
-// filter-scale gradients are one more batch or three.
+// takes the first that collapses.  The walk needs the strain alone; what else a collapsed peak's
+// record holds is worked out afterwards (finish_rows_kernel) from the two shells on either
+// side of the collapse, and the formation redshift, which one halo in eight has, by
+// half_rows_kernel: in one kernel the walk held 222 registers, two wavefronts per SIMD, and
+// waited for its loads (512^3 tile, ms: 7.8; walk, finish and half 2.9 + 2.5 + 1.0; with four
+// lanes reading a block's lines and handing them round, 2.5 + 2.1 + 0.9.  Loading the next block
+// ahead costs a wavefront per SIMD: 2.7 + 2.3 + 0.8).  Four lanes for many peaks (median walk 6
+// shells): two, eight and sixteen took 4, 29 and 95 % longer; sixteen where the peaks would not
+// fill the CUs.
 
-// kernel_strain of a row: lane l's shell mp with window [mlow, mupp], for lanes with `on`;
-// eb = first block of the row's peak.  The sums run over the shells in ascending order, as
-// kstrain's.
+// The weights of shell mp (kernel_strain): its shells lo .. hi within [mlow, mupp] and the first
+// weight; the row's range of them.
+struct RowWin {
+    const double* w;
+    int lo, hi, rlo, rhi;
+};
 template <int W>
+__device__ __forceinline__ RowWin row_win(const SAArgs& a, int mp, int mlow, int mupp, bool on) {
+    RowWin r;
+    const int mpc = on ? mp : 1;
+    const int lo0 = a.kidx[3 * mpc], hi0 = a.kidx[3 * mpc + 1];
+    r.w = a.kw + (a.kidx[3 * mpc + 2] - lo0);
+    r.lo = on ? (mlow > lo0 ? mlow : lo0) : 0x7fff;
+    r.hi = on ? (mupp < hi0 ? mupp : hi0) : -1;
+    r.rlo = r.lo;
+    r.rhi = r.hi;
+#pragma unroll
+    for (int d = 1; d < W; d <<= 1) {
+        r.rlo = min(r.rlo, __shfl_xor(r.rlo, d, W));
+        r.rhi = max(r.rhi, __shfl_xor(r.rhi, d, W));
+    }
+    return r;
+}
+
+// The lines of a block, one shell per lane of four.
+template <bool STRAIN_ONLY>
+struct Entry {
+    double g0, g1, g2, f0, f1, f2, x0, x1, x2, y0, y1, y2, z0, z1, z2;
+    __device__ __forceinline__ void load(const double* __restrict__ q) {
+        if (!STRAIN_ONLY) {
+            g0 = q[1];
+            const double2 gb = *reinterpret_cast<const double2*>(q + 2);
+            g1 = gb.x; g2 = gb.y;
+            const double2 ha = *reinterpret_cast<const double2*>(q + 16);
+            f0 = ha.x; f1 = ha.y;
+            f2 = q[18];
+        }
+        x0 = q[33];
+        y0 = q[49];
+        z0 = q[65];
+        const double2 x = *reinterpret_cast<const double2*>(q + 34);
+        const double2 y = *reinterpret_cast<const double2*>(q + 50);
+        const double2 z = *reinterpret_cast<const double2*>(q + 66);
+        x1 = x.x; x2 = x.y;
+        y1 = y.x; y2 = y.y;
+        z1 = z.x; z2 = z.y;
+    }
+    template <int S>
+    __device__ __forceinline__ void add(KS& r, const RowWin& w, int m1) const {
+        const double X0 = quad_of<S>(x0), X1 = quad_of<S>(x1), X2 = quad_of<S>(x2);
+        const double Y0 = quad_of<S>(y0), Y1 = quad_of<S>(y1), Y2 = quad_of<S>(y2);
+        const double Z0 = quad_of<S>(z0), Z1 = quad_of<S>(z1), Z2 = quad_of<S>(z2);
+        double G0 = 0, G1 = 0, G2 = 0, F0 = 0, F1 = 0, F2 = 0;
+        if (!STRAIN_ONLY) {
+            G0 = quad_of<S>(g0); G1 = quad_of<S>(g1); G2 = quad_of<S>(g2);
+            F0 = quad_of<S>(f0); F1 = quad_of<S>(f1); F2 = quad_of<S>(f2);
+        }
+        if (m1 >= w.lo && m1 <= w.hi) {
+            const double wt = w.w[m1], hw = 0.5 * wt;
+            if (!STRAIN_ONLY) {
+                r.g0 += wt * G0;
+                r.g1 += wt * G1;
+                r.g2 += wt * G2;
+                r.f0 += wt * F0;
+                r.f1 += wt * F1;
+                r.f2 += wt * F2;
+            }
+            r.E11 -= hw * (X0 + X0);
+            r.E12 -= hw * (X1 + Y0);
+            r.E13 -= hw * (X2 + Z0);
+            r.E22 -= hw * (Y1 + Y1);
+            r.E23 -= hw * (Y2 + Z1);
+            r.E33 -= hw * (Z2 + Z2);
+        }
+    }
+};
+
+// kernel_strain of a row: lane l's shell mp with window [mlow, mupp], for lanes with `on`; eb =
+// first block of the row's peak.  The sums run over the shells in ascending order, as kstrain's.
+// Four lanes read a block's lines, a shell each, and hand them round.
+template <int W, bool STRAIN_ONLY>
 __device__ __forceinline__ KS kstrain_row(const SAArgs& a, const BlockArgs& B, int64_t eb, int mp,
                                           int mlow, int mupp, bool on) {
     KS r = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const int mpc = on ? mp : 1;
-    const int lo0 = a.kidx[3 * mpc], hi0 = a.kidx[3 * mpc + 1];
-    const double* __restrict__ wt0 = a.kw + (a.kidx[3 * mpc + 2] - lo0);
-    const int lo = on ? (mlow > lo0 ? mlow : lo0) : 0x7fff;
-    const int hi = on ? (mupp < hi0 ? mupp : hi0) : -1;
-    int rlo = lo, rhi = hi;
-#pragma unroll
-    for (int d = 1; d < W; d <<= 1) {
-        rlo = min(rlo, __shfl_xor(rlo, d, W));
-        rhi = max(rhi, __shfl_xor(rhi, d, W));
+    const RowWin w = row_win<W>(a, mp, mlow, mupp, on);
+    const int b1 = w.rlo <= w.rhi ? w.rhi >> 2 : -1;
+    int b = w.rlo >> 2;
+    Entry<STRAIN_ONLY> cur;
+    const double* q = B.prof + (eb + b) * BLK_LINES + (threadIdx.x & 3) * 4;
+    for (; b <= b1; ++b, q += BLK_LINES) {
+        cur.load(q);
+        cur.template add<0>(r, w, 4 * b);
+        cur.template add<1>(r, w, 4 * b + 1);
+        cur.template add<2>(r, w, 4 * b + 2);
+        cur.template add<3>(r, w, 4 * b + 3);
     }
-    const int64_t o0 = eb * BLK * 4;
-    for (int m1 = rlo; m1 <= rhi; ++m1) {
-        const int64_t o = o0 + (int64_t)m1 * 4;
-        const double2 ga = *reinterpret_cast<const double2*>(B.line[0] + o);
-        const double2 gb = *reinterpret_cast<const double2*>(B.line[0] + o + 2);
-        const double2 ha = *reinterpret_cast<const double2*>(B.line[1] + o);
-        const double h2 = B.line[1][o + 2];
-        const double2 xa = *reinterpret_cast<const double2*>(B.line[2] + o);
-        const double2 xb = *reinterpret_cast<const double2*>(B.line[2] + o + 2);
-        const double2 ya = *reinterpret_cast<const double2*>(B.line[3] + o);
-        const double2 yb = *reinterpret_cast<const double2*>(B.line[3] + o + 2);
-        const double2 za = *reinterpret_cast<const double2*>(B.line[4] + o);
-        const double2 zb = *reinterpret_cast<const double2*>(B.line[4] + o + 2);
-        if (m1 >= lo && m1 <= hi) {
-            const double wt = wt0[m1], hw = 0.5 * wt;
-            r.g0 += wt * ga.y;
-            r.g1 += wt * gb.x;
-            r.g2 += wt * gb.y;
-            r.f0 += wt * ha.x;
-            r.f1 += wt * ha.y;
-            r.f2 += wt * h2;
-            r.E11 -= hw * (xa.y + xa.y);
-            r.E12 -= hw * (xb.x + ya.y);
-            r.E13 -= hw * (xb.y + za.y);
-            r.E22 -= hw * (yb.x + yb.x);
-            r.E23 -= hw * (yb.y + zb.x);
-            r.E33 -= hw * (zb.y + zb.y);
-        }
-    }
-    const double sc = mpc > 1 ? a.wRnor / a.rad[mpc] : a.aRnor;
+    const double sc = on && mp > 1 ? a.wRnor / a.rad[mp] : a.aRnor;
     r.E11 *= sc; r.E12 *= sc; r.E13 *= sc; r.E22 *= sc; r.E23 *= sc; r.E33 *= sc;
-    r.g0 *= sc; r.g1 *= sc; r.g2 *= sc; r.f0 *= sc; r.f1 *= sc; r.f2 *= sc;
+    if (!STRAIN_ONLY) {
+        r.g0 *= sc; r.g1 *= sc; r.g2 *= sc; r.f0 *= sc; r.f1 *= sc; r.f2 *= sc;
+    }
     return r;
 }
 
@@ -871,13 +990,6 @@ __device__ __forceinline__ KS shfl_ks(const KS& k, int src) {
     r.g0 = __shfl(k.g0, src); r.g1 = __shfl(k.g1, src); r.g2 = __shfl(k.g2, src);
     r.f0 = __shfl(k.f0, src); r.f1 = __shfl(k.f1, src); r.f2 = __shfl(k.f2, src);
     return r;
-}
-
-__device__ __forceinline__ void pick_ks(KS& d, const KS& s, bool c) {
-    d.E11 = c ? s.E11 : d.E11; d.E12 = c ? s.E12 : d.E12; d.E13 = c ? s.E13 : d.E13;
-    d.E22 = c ? s.E22 : d.E22; d.E23 = c ? s.E23 : d.E23; d.E33 = c ? s.E33 : d.E33;
-    d.g0 = c ? s.g0 : d.g0; d.g1 = c ? s.g1 : d.g1; d.g2 = c ? s.g2 : d.g2;
-    d.f0 = c ? s.f0 : d.f0; d.f1 = c ? s.f1 : d.f1; d.f2 = c ? s.f2 : d.f2;
 }
 
 // Running lapd sum over the cells of shells 1 .. sR: variants B and C from the centre on,
@@ -902,16 +1014,21 @@ __device__ double block_d2f(const SAArgs& a, const TileDev& T, int ci, int cj, i
     return n > 0 ? lap / (double)n : 0.0;
 }
 
+// What the walk leaves for a slot: the collapse between shells mc - 1 (zvir1p) and mc (zvir1), the
+// walk's start m0 with its window's end, and the trace at mc - 1; mc = 0 without a collapse.
+struct WalkState {
+    double zvir1, zvir1p, Frhoh;
+    int mc, m0, mupp0, pad;
+};
+
 template <int W>
-__global__ __launch_bounds__(64) void radial_rows_kernel(SAArgs a, BlockArgs B, int64_t slot0,
-                                                         int64_t nslot) {
-    constexpr int NR = 64 / W;
+__global__ __launch_bounds__(64) void walk_rows_kernel(SAArgs a, BlockArgs B, int64_t slot0,
+                                                       int64_t nslot, WalkState* __restrict__ state) {
     const int lane = threadIdx.x, l = lane & (W - 1), row0 = lane & ~(W - 1);
-    const int64_t per = (int64_t)gridDim.x >> 3;
-    const int64_t w = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if (w * NR >= nslot) return;
-    const int64_t sl = slot0 + w * NR + lane / W;
-    const TileDev& T = a.tiles[a.gtile[(slot0 + w * NR) >> 6]];
+    int64_t first;
+    if (!row_slot<W>(nslot, first)) return;
+    const int64_t sl = slot0 + first + lane / W;
+    const TileDev& T = a.tiles[a.gtile[(slot0 + first) >> 6]];
     const int p = a.slot[sl];
     int64_t eb = 0;
     bool valid = p >= 0;
@@ -920,21 +1037,14 @@ __global__ __launch_bounds__(64) void radial_rows_kernel(SAArgs a, BlockArgs B, 
         valid = eb >= 0 && eb < B.ne;
         if (!valid) eb = 0;
     }
-    if (__ballot(valid) == 0ull) return;
-    const double* __restrict__ rad = a.rad;
     const int m = a.NS - 1;
-    int ci = 1, cj = 1, ck = 1, ir2min = 0, scross = 0, stop = 1;
-    double ZZon = 0.0, fcrit = 0.0, Rf = 0.0;
+    int ir2min = 0, scross = 0;
+    double ZZon = 0.0, fcrit = 0.0;
     if (valid) {
-        ci = T.pi[p];
-        cj = T.pj[p];
-        ck = T.pk[p];
         ir2min = T.ir2min[p];
-        Rf = T.Rf[p];
         ZZon = T.ZZon ? T.ZZon[p] : T.ZZon_s;
         fcrit = T.fcrit ? T.fcrit[p] : T.fcrit_s;
         scross = B.cross[T.base + p];
-        stop = B.stop[T.base + p];
     }
     const double* __restrict__ fb = B.fb + eb * BLK;
 
@@ -964,95 +1074,143 @@ __global__ __launch_bounds__(64) void radial_rows_kernel(SAArgs a, BlockArgs B, 
     }
     const int mlow0 = B.win[3 * m0 + 2];
 
-    // ---- walk: step 0 is m0 itself (no collapse test), step i shell m0 - i ----
-    bool hit_row = false;
-    int mc = 0;  // m0 of the collapse
-    double zvir1 = -1.0, zvir1p = -1.0, Frhoh = 0.0;
-    KS last = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, prev = last, carry = last;
+    // step i is shell m0 - 1 - i; the step before the first counts as zvir -1
+    WalkState ws = {-1.0, -1.0, 0.0, 0, m0, mupp0, 0};
     double zcarry = -1.0;
     for (int i0 = 0;; i0 += W) {
-        const int mp = m0 - (i0 + l);
+        const int mp = m0 - 1 - (i0 + l);
         const bool on = live && mp >= 1;
         if (__ballot(on) == 0ull) break;
         int mlow = 1, mupp = 0;
         if (on) {
             mlow = min(mlow0, B.win[3 * mp + 2]);
-            mupp = (i0 + l == 0 || mupp0 <= B.win[3 * mp + 1]) ? mupp0 : B.win[3 * mp];
+            mupp = mupp0 <= B.win[3 * mp + 1] ? mupp0 : B.win[3 * mp];
         }
-        const KS kk = kstrain_row<W>(a, B, eb, mp, mlow, mupp, on);
+        const KS kk = kstrain_row<W, true>(a, B, eb, mp, mlow, mupp, on);
         double zv = -1.0, Fr = 0.0;
         if (on) {
             double lam[3], e_mp, p_mp;
             eig_ks(kk, lam);
             ev_from_lam(lam, &Fr, &e_mp, &p_mp);
             const double Fb = fb[mp];
-            if (i0 + l > 0 && Fb > 0.0) {
+            if (Fb > 0.0) {
                 const double poe = e_mp < 1e-5 ? 0.0 : p_mp / e_mp;
                 zv = interp3(a.ct, log10(Fb), e_mp, poe);
             }
         }
-        const bool hit = on && i0 + l > 0 && zv >= ZZon;
-        const uint64_t hits = (__ballot(hit) >> row0) & (W == 64 ? ~0ull : ((1ull << W) - 1ull));
+        const bool hit = on && zv >= ZZon;
+        const uint64_t hits = (__ballot(hit) >> row0) & ((1ull << W) - 1ull);
         const int hl = hits ? __ffsll((unsigned long long)hits) - 1 : 0;
-        const KS kl = shfl_ks(kk, row0 + hl);
         const double zl = __shfl(zv, row0 + hl), fl = __shfl(Fr, row0 + hl);
-        const int pl = row0 + (hl > 0 ? hl - 1 : 0);
-        KS kp = shfl_ks(kk, pl);
-        double zp = __shfl(zv, pl);
-        pick_ks(kp, carry, hl == 0);
-        zp = hl == 0 ? zcarry : zp;
-        const bool take = hits != 0 && live;
-        pick_ks(last, kl, take);
-        pick_ks(prev, kp, take);
-        zvir1p = take ? zl : zvir1p;
-        zvir1 = take ? zp : zvir1;
-        Frhoh = take ? fl : Frhoh;
-        if (take) {
-            mc = m0 - (i0 + hl) + 1;
-            hit_row = true;
+        const double zb = __shfl(zv, row0 + (hl > 0 ? hl - 1 : 0));
+        if (hits != 0 && live) {
+            ws.zvir1p = zl;
+            ws.Frhoh = fl;
+            ws.zvir1 = hl == 0 ? zcarry : zb;
+            ws.mc = m0 - (i0 + hl);
             live = false;
         }
-        carry = shfl_ks(kk, row0 + W - 1);
         zcarry = __shfl(zv, row0 + W - 1);
     }
+    if (!valid || l != 0) {
+        if (l == 0) state[sl - slot0].mc = 0;
+        return;
+    }
+    // RTHL > 0 (a collapse at the centre has radius 0)
+    if (ws.mc > 0) {
+        const double dZ = ws.zvir1p - ws.zvir1;
+        double R3 = cube(a.rad[ws.mc - 1]);
+        if (ws.zvir1 > 0.0 && dZ != 0.0)
+            R3 = R3 + (cube(a.rad[ws.mc]) - R3) * (ws.zvir1p - ZZon) / dZ;
+        if (R3 == 0.0) ws.mc = 0;
+    }
+    state[sl - slot0] = ws;
+    if (T.res.nshells_used) T.res.nshells_used[p] = B.stop[T.base + p];
+    if (T.res.crossing_shell) T.res.crossing_shell[p] = scross;
+    if (T.res.bracket) T.res.bracket[p] = 0;
+    B.cross[T.base + p] = ws.mc;  // what sbar_rows_kernel reads
+    if (ws.mc == 0) {
+        write_no_collapse(T, p);
+        if (a.paint) a.paint[T.base + p] = -1;
+    }
+}
 
-    double RTHL = 0.0;
-    const double dZvir = zvir1p - zvir1;
-    if (hit_row) {
-        if (zvir1 > 0.0 && dZvir != 0.0) {
-            const double RTHL3 = cube(rad[mc - 1]) + (cube(rad[mc]) - cube(rad[mc - 1])) *
-                                                         (zvir1p - ZZon) / dZvir;
-            RTHL = pow(RTHL3, 1.0 / 3.0);
-        } else {
-            RTHL = rad[mc - 1];
+__device__ __forceinline__ double walk_rthl(const SAArgs& a, const WalkState& ws, double ZZon) {
+    const double* rad = a.rad;
+    const double dZvir = ws.zvir1p - ws.zvir1;
+    if (ws.zvir1 > 0.0 && dZvir != 0.0) {
+        const double RTHL3 = cube(rad[ws.mc - 1]) + (cube(rad[ws.mc]) - cube(rad[ws.mc - 1])) *
+                                                        (ws.zvir1p - ZZon) / dZvir;
+        return pow(RTHL3, 1.0 / 3.0);
+    }
+    return rad[ws.mc - 1];
+}
+
+// The record of the collapsed peaks (RadialShell.jl:608-800) but for Sbar, Sbar2 and the
+// formation redshift: four lanes per peak take kernel_strain at mc - 1, at mc and at the filter
+// scale.  Halos of RTHL >= 3 go to `half` (hcnt of them), slot by slot.
+__global__ __launch_bounds__(64) void finish_rows_kernel(SAArgs a, BlockArgs B, int64_t slot0,
+                                                         int64_t nslot,
+                                                         const WalkState* __restrict__ state,
+                                                         int32_t* __restrict__ half,
+                                                         int32_t* __restrict__ hcnt) {
+    constexpr int W = 4;
+    const int lane = threadIdx.x, l = lane & (W - 1), row0 = lane & ~(W - 1);
+    int64_t first;
+    if (!row_slot<W>(nslot, first)) return;
+    const int64_t sl = slot0 + first + lane / W;
+    const TileDev& T = a.tiles[a.gtile[(slot0 + first) >> 6]];
+    WalkState ws = state[sl - slot0];
+    const bool on = ws.mc > 0;
+    if (__ballot(on) == 0ull) return;
+    const double* __restrict__ rad = a.rad;
+    const int p = on ? a.slot[sl] : 0;
+    const int64_t eb = on ? B.base[T.base + p] - B.e0 : 0;
+    const double* __restrict__ fb = B.fb + eb * BLK;
+    if (!on) ws.mc = 2;
+    const int mc = ws.mc;
+    const double ZZon = on ? (T.ZZon ? T.ZZon[p] : T.ZZon_s) : 0.0;
+    const double RTHL = on ? walk_rthl(a, ws, ZZon) : 1.0;
+    const double dZvir = ws.zvir1p - ws.zvir1;
+
+    int mp = 1, mlow = 1, mupp = 0;
+    if (on && l == 2) {
+        rf_window(a, T.Rf[p], mp, mlow, mupp);
+    } else if (on && l < 2) {
+        mp = mc - 1 + l;
+        mlow = min(B.win[3 * ws.m0 + 2], B.win[3 * mp + 2]);
+        mupp = (mp == ws.m0 || ws.mupp0 <= B.win[3 * mp + 1]) ? ws.mupp0 : B.win[3 * mp];
+    }
+    const KS kk = kstrain_row<W, false>(a, B, eb, mp, mlow, mupp, on && l < 3);
+    const KS last = shfl_ks(kk, row0), prev = shfl_ks(kk, row0 + 1);
+    if (on && l == 2) {
+        const int64_t o3 = (int64_t)p * 3;
+        T.res.gradpkrf[o3] = kk.g0;
+        T.res.gradpkrf[o3 + 1] = kk.g1;
+        T.res.gradpkrf[o3 + 2] = kk.g2;
+    }
+    const bool halfz = on && l == 0 && a.variant != HNT_VARIANT_B && RTHL / 1.0 >= 3.0;
+    {
+        const uint64_t hm = __ballot(halfz);
+        if (hm) {
+            int at = 0;
+            const int f = __ffsll((unsigned long long)hm) - 1;
+            if (lane == f) at = atomicAdd(hcnt, (int)__popcll(hm));
+            at = __shfl(at, f) + (int)__popcll(hm & ((1ull << lane) - 1ull));
+            if (halfz) half[at] = (int32_t)(sl - slot0);
         }
-        if (RTHL <= 0.0) hit_row = false;
     }
-    if (valid && l == 0) {
-        if (T.res.nshells_used) T.res.nshells_used[p] = stop;
-        if (T.res.crossing_shell) T.res.crossing_shell[p] = scross;
-        if (T.res.bracket) T.res.bracket[p] = 0;
-        B.cross[T.base + p] = hit_row ? mc : 0;  // what block_sbar_kernel reads
-        if (!hit_row) {
-            write_no_collapse(T, p);
-            if (a.paint) a.paint[T.base + p] = -1;
-        }
-    }
-    if (__ballot(hit_row) == 0ull) return;
-    if (!hit_row) {
-        mc = 2;
-        RTHL = 1.0;
-    }
+    if (!on || l != 0) return;
 
     const double RTHL3 = cube(RTHL);
     const double RTHL5 = RTHL3 * RTHL * RTHL;
     const double rad3p = cube(rad[mc - 1]);
     const double rad3 = cube(rad[mc]);
     const double drad3 = rad3 - rad3p;
-    const double Fbm = hit_row ? fb[mc - 1] : 0.0, Fb0 = hit_row ? fb[mc] : 0.0;
+    const double Fbm = fb[mc - 1], Fb0 = fb[mc];
     double Fbarx;
     KS fin;  // interpolated strain and gradients
-    if (zvir1 > 0.0 && drad3 != 0.0) {
+    if (ws.zvir1 > 0.0 && drad3 != 0.0) {
         const double frac = (RTHL3 - rad3p) / drad3;
         Fbarx = Fbm + frac * (Fb0 - Fbm);
         fin.E11 = last.E11 + frac * (prev.E11 - last.E11);
@@ -1079,23 +1237,70 @@ __global__ __launch_bounds__(64) void radial_rows_kernel(SAArgs a, BlockArgs B, 
         fin.E11 *= sc; fin.E12 *= sc; fin.E13 *= sc;
         fin.E22 *= sc; fin.E23 *= sc; fin.E33 *= sc;
     }
+    double lamf[3], Frc, e_f, p_f;
+    eig_ks(fin, lamf);
+    ev_from_lam(lamf, &Frc, &e_f, &p_f);
 
-    // ---- task 0: eigenvalues of the final strain; 1: filter-scale gradients; 2 .. 11: the
-    // formation redshift's radii (RadialShell.jl:801-859; variant B gives 0) ----
-    const bool half = a.variant != HNT_VARIANT_B && RTHL / 1.0 >= 3.0;
-    double zh = a.variant == HNT_VARIANT_B ? 0.0 : -1.0;
-    double lamf[3] = {0, 0, 0}, e_f = 0.0, p_f = 0.0;
-    const int ntask = half ? 12 : 2;
-    for (int t0 = 0; t0 < 12; t0 += W) {
-        const int t = t0 + l;
-        const bool on = hit_row && t < ntask;
-        if (__ballot(on) == 0ull) break;
+    double Srb = 0.0, rad5p = 0.0;
+    if (mc > 2)
+        for (int s = 2; s <= mc - 1; ++s) {
+            const double rad5 = pow5(rad[s]);
+            Srb += 0.5 * (fb[s - 1] + fb[s]) * (rad5 - rad5p);
+            rad5p = rad5;
+        }
+    if (ws.zvir1 > 0.0 && dZvir != 0.0) Srb += 0.5 * (Fbm + Fbarx) * (RTHL5 - rad5p);
+    if (Fbarx * RTHL5 > 0.0) Srb /= (Fbarx * RTHL5);
+    const int sR = first_gt(rad, 1, a.NS, RTHL) - 1;
+    if (a.paint) a.paint[T.base + p] = T.mask ? a.shell_r2[sR - 1] : -1;
+    double F11 = last.E11, F12 = last.E12, F13 = last.E13, F22 = last.E22, F23 = last.E23,
+           F33 = last.E33;
+    if (a.variant == HNT_VARIANT_A || ws.Frhoh != 0.0) {
+        const double sc2 = Fbarx / ws.Frhoh;
+        F11 *= sc2; F12 *= sc2; F13 *= sc2; F22 *= sc2; F23 *= sc2; F33 *= sc2;
+    }
+    const hnt_results& R = T.res;
+    const int64_t o3 = (int64_t)p * 3;
+    R.RTHL[p] = RTHL;
+    R.Fbarx[p] = Fbarx;
+    R.e_v[p] = e_f;
+    R.p_v[p] = p_f;
+    R.Srb[p] = Srb;
+    R.d2F[p] = T.has_lapd ? block_d2f(a, T, T.pi[p], T.pj[p], T.pk[p], sR) : 0.0;
+    // half_rows_kernel overwrites it for the halos of its list
+    R.zvir_half[p] = a.variant == HNT_VARIANT_B ? 0.0 : -1.0;
+    double* sm = R.strain + (int64_t)p * 9;
+    sm[0] = F11; sm[1] = F12; sm[2] = F13;
+    sm[3] = F12; sm[4] = F22; sm[5] = F23;
+    sm[6] = F13; sm[7] = F23; sm[8] = F33;
+    R.eigs[o3] = lamf[0]; R.eigs[o3 + 1] = lamf[1]; R.eigs[o3 + 2] = lamf[2];
+    R.gradpk[o3] = fin.g0; R.gradpk[o3 + 1] = fin.g1; R.gradpk[o3 + 2] = fin.g2;
+    R.gradpkf[o3] = fin.f0; R.gradpkf[o3 + 1] = fin.f1; R.gradpkf[o3 + 2] = fin.f2;
+}
+
+// The formation redshift (RadialShell.jl:801-859) of the listed halos: sixteen lanes per halo, ten
+// of them a radius each.
+__global__ __launch_bounds__(64) void half_rows_kernel(SAArgs a, BlockArgs B, int64_t slot0,
+                                                       const WalkState* __restrict__ state,
+                                                       const int32_t* __restrict__ half,
+                                                       const int32_t* __restrict__ hcnt) {
+    constexpr int W = 16, NR = 64 / W;
+    const int lane = threadIdx.x, l = lane & (W - 1);
+    const int n = *hcnt, m = a.NS - 1;
+    const double* __restrict__ rad = a.rad;
+    for (int i0 = (int)blockIdx.x * NR; i0 < n; i0 += (int)gridDim.x * NR) {
+        const int i = i0 + lane / W;
+        const bool row = i < n;
+        const int64_t sl = slot0 + half[row ? i : i0];
+        const TileDev& T = a.tiles[a.gtile[sl >> 6]];
+        const int p = a.slot[sl];
+        const int64_t eb = B.base[T.base + p] - B.e0;
+        const double* __restrict__ fb = B.fb + eb * BLK;
+        const WalkState ws = state[sl - slot0];
+        const double RTHL = walk_rthl(a, ws, T.ZZon ? T.ZZon[p] : T.ZZon_s);
+        const bool on = row && l < 10;
         int mp = 1, mlow = 1, mupp = 0;
-        const bool strain = on && t > 0;
-        if (strain && t == 1) {
-            rf_window(a, Rf, mp, mlow, mupp);
-        } else if (strain) {
-            const double rcur = RTHL * pow((double)(t - 2) / 9.0 * 0.5 + 0.5, 1.0 / 3.0);
+        if (on) {
+            const double rcur = RTHL * pow((double)l / 9.0 * 0.5 + 0.5, 1.0 / 3.0);
             mupp = 1;
             if (m - 1 >= 2) {
                 const int f = first_gt(rad, 2, m - 1, rcur + 2.0);
@@ -1110,88 +1315,44 @@ __global__ __launch_bounds__(64) void radial_rows_kernel(SAArgs a, BlockArgs B, 
                 mp = f <= m - 1 ? f : m - 1;
             }
         }
-        const KS kr = kstrain_row<W>(a, B, eb, mp, mlow, mupp, strain);
-        if (on && t == 1) {
-            const int64_t o3 = (int64_t)p * 3;
-            T.res.gradpkrf[o3] = kr.g0;
-            T.res.gradpkrf[o3 + 1] = kr.g1;
-            T.res.gradpkrf[o3 + 2] = kr.g2;
-        } else if (on) {
-            const KS ke = t == 0 ? fin : kr;
+        const KS kr = kstrain_row<W, true>(a, B, eb, mp, mlow, mupp, on);
+        double zh = -1.0;
+        if (on) {
             double lam[3], Fr, ev, pv;
-            eig_ks(ke, lam);
+            eig_ks(kr, lam);
             ev_from_lam(lam, &Fr, &ev, &pv);
-            if (t == 0) {
-                lamf[0] = lam[0]; lamf[1] = lam[1]; lamf[2] = lam[2];
-                e_f = ev;
-                p_f = pv;
-            } else {
-                const double Fb = fb[mp];
-                const double poe = ev < 1e-5 ? 0.0 : pv / ev;
-                double zr = -1.0;
-                if (Fb > 0.0) zr = interp3(a.ct, log10(Fb), ev, poe);
-                const double zs = zr - 1.0;
-                if (zs > zh) zh = zs;
-            }
+            const double Fb = fb[mp];
+            const double poe = ev < 1e-5 ? 0.0 : pv / ev;
+            double zr = -1.0;
+            if (Fb > 0.0) zr = interp3(a.ct, log10(Fb), ev, poe);
+            const double zs = zr - 1.0;
+            if (zs > zh) zh = zs;
         }
-    }
 #pragma unroll
-    for (int d = 1; d < W; d <<= 1) {
-        const double o = __shfl_xor(zh, d, W);
-        if (o > zh) zh = o;
-    }
-    if (!hit_row) return;
-
-    const hnt_results& R = T.res;
-    const int64_t o3 = (int64_t)p * 3;
-    if (l == 0) {
-        double Srb = 0.0, rad5p = 0.0;
-        if (mc > 2)
-            for (int mp = 2; mp <= mc - 1; ++mp) {
-                const double rad5 = pow5(rad[mp]);
-                Srb += 0.5 * (fb[mp - 1] + fb[mp]) * (rad5 - rad5p);
-                rad5p = rad5;
-            }
-        if (zvir1 > 0.0 && dZvir != 0.0) Srb += 0.5 * (Fbm + Fbarx) * (RTHL5 - rad5p);
-        if (Fbarx * RTHL5 > 0.0) Srb /= (Fbarx * RTHL5);
-        const int sR = first_gt(rad, 1, a.NS, RTHL) - 1;
-        if (a.paint) a.paint[T.base + p] = T.mask ? a.shell_r2[sR - 1] : -1;
-        double F11 = last.E11, F12 = last.E12, F13 = last.E13, F22 = last.E22, F23 = last.E23,
-               F33 = last.E33;
-        if (a.variant == HNT_VARIANT_A || Frhoh != 0.0) {
-            const double sc2 = Fbarx / Frhoh;
-            F11 *= sc2; F12 *= sc2; F13 *= sc2; F22 *= sc2; F23 *= sc2; F33 *= sc2;
+        for (int d = 1; d < W; d <<= 1) {
+            const double o = __shfl_xor(zh, d, W);
+            if (o > zh) zh = o;
         }
-        R.RTHL[p] = RTHL;
-        R.Fbarx[p] = Fbarx;
-        R.e_v[p] = e_f;
-        R.p_v[p] = p_f;
-        R.Srb[p] = Srb;
-        R.d2F[p] = T.has_lapd ? block_d2f(a, T, ci, cj, ck, sR) : 0.0;
-        R.zvir_half[p] = zh;
-        double* sm = R.strain + (int64_t)p * 9;
-        sm[0] = F11; sm[1] = F12; sm[2] = F13;
-        sm[3] = F12; sm[4] = F22; sm[5] = F23;
-        sm[6] = F13; sm[7] = F23; sm[8] = F33;
-        R.eigs[o3] = lamf[0]; R.eigs[o3 + 1] = lamf[1]; R.eigs[o3 + 2] = lamf[2];
-        R.gradpk[o3] = fin.g0; R.gradpk[o3 + 1] = fin.g1; R.gradpk[o3 + 2] = fin.g2;
-        R.gradpkf[o3] = fin.f0; R.gradpkf[o3 + 1] = fin.f1; R.gradpkf[o3 + 2] = fin.f2;
+        if (row && l == 0) T.res.zvir_half[p] = zh;
     }
 }
 
 // ------------------------------------------------------------------ crossing pass by rows
-// The crossing pass for few peaks: W lanes per peak, each summing one shell's delta, W shells
-// at a time; the Fbar recurrence then runs over their sums in order (every lane alike).  The
-// same sums and recurrence as crossing_kernel, which keeps a lane per peak: with tens of
-// thousands of wavefronts it wastes no shell beyond the crossing, but with few its time is
-// that of the deepest peak's whole chain of cells.
+// The crossing pass: W lanes per peak, each summing one shell's delta, W shells at a time; the
+// Fbar recurrence then runs over their sums in order (every lane alike).  The same sums and
+// recurrence as crossing_kernel, which keeps a lane per peak: there a wavefront's 64 peaks walk
+// 64 different cache lines for every cell and lose them before the next cell (57 % hits), and it
+// runs as long as its deepest peak.  Four lanes: 512^3 tile 4.2 -> 2.8 ms; two and eight were
+// 12 and 7 % slower than four (a row idles beyond the crossing, at shell 7 to 12 on average);
+// sixteen for few peaks, where the time is one deep peak's chain of cells.
 template <int W>
-__global__ __launch_bounds__(64) void crossing_rows_kernel(SAArgs a, int32_t* __restrict__ stop_out,
+__global__ __launch_bounds__(64) void crossing_rows_kernel(SAArgs a,
+                                                           const uint32_t* __restrict__ cell8,
+                                                           int32_t* __restrict__ stop_out,
                                                            int32_t* __restrict__ cross_out) {
-    constexpr int NR = 64 / W;
     const int lane = threadIdx.x, l = lane & (W - 1), row0 = lane & ~(W - 1);
-    const int64_t s0 = (int64_t)blockIdx.x * NR;
-    if (s0 >= a.ngroups * 64) return;
+    int64_t s0;
+    if (!row_slot<W>(a.ngroups * 64, s0)) return;
     const TileDev& T = a.tiles[a.gtile[s0 >> 6]];
     const int p = a.slot[s0 + lane / W];
     const bool valid = p >= 0;
@@ -1215,18 +1376,15 @@ __global__ __launch_bounds__(64) void crossing_rows_kernel(SAArgs a, int32_t* __
         if (__ballot(active) == 0ull) break;
         const int s = sb + l;
         double F = 0.0;
-        int64_t nin = 0;
+        int nin = 0;
         // the shells of this batch that leave the grid are summed with the check
         const bool out = ball_outside(T, ci, cj, ck, (int)a.rad[min(sb + W - 1, m)]);
         if (active && s <= m) {
-            const int st = a.shell_start[s - 1], nc = a.shell_count[s - 1];
-            if (!out) cross_shell_hbm<false>(a, T, st, nc, ci, cj, ck, c0, F, nin);
-            else cross_shell_hbm<true>(a, T, st, nc, ci, cj, ck, c0, F, nin);
+            shell_sum(a, cell8, T, T.delta, s, ci, cj, ck, c0, out, F, nin);
         }
-        const int nin32 = (int)nin;
         for (int j = 0; j < W && sb + j <= m; ++j) {
             const double Fj = __shfl(F, row0 + j);
-            const int nj = __shfl(nin32, row0 + j);
+            const int nj = __shfl(nin, row0 + j);
             if (active)
                 cross_step(a, sb + j, Fj, nj, ir2min, fcrit, Fprev, dFbarp, past, active, scross);
         }
