@@ -111,13 +111,13 @@ __device__ __forceinline__ void dft(float2 (&v)[R]) {
 // One Stockham stage of radix R on `ncol` columns of length L held in LDS (column c at
 // buf + c * LS): butterfly j of a column reads x[j + r L/R], twiddles by W^(r k L/(Ns R)),
 // k = j mod Ns, and writes x[(j/Ns) Ns R + k + r Ns].  All reads precede all writes.
-// Row-major LDS layout of the direct-load column passes (C = 8 or 4 columns): element i of
+// Row-major LDS layout of the direct-load column passes (C = 16, 8 or 4 columns): element i of
 // column c at (i + i / (128 / C)) * C + c, i.e. rows of C complex (8 C bytes) in blocks of
 // 128 / C rows (1 KB, what one wavefront's 16-byte direct loads fill) with one spare row
 // after each block.
 template <int C>
 __device__ __forceinline__ int rm_slot(int c, int i) {
-    constexpr int LGC = C == 8 ? 3 : 2, LGB = 7 - LGC;
+    constexpr int LGC = C == 16 ? 4 : (C == 8 ? 3 : 2), LGB = 7 - LGC;
     return ((i + (i >> LGB)) << LGC) + c;
 }
 
@@ -134,7 +134,7 @@ __device__ __forceinline__ void stage(float2* buf, int LS, int ncol, int lgL, in
     // column-major (RMC = 0): a thread's butterflies run down one column; row-major (RMC
     // columns): the column index is the fastest, so RMC lanes read or write one row
     constexpr bool RM = RMC != 0;
-    constexpr int LGRM = RMC == 8 ? 3 : 2;
+    constexpr int LGRM = RMC == 16 ? 4 : (RMC == 8 ? 3 : 2);
     auto at = [&](int c, int i) -> float2& {
         if constexpr (RM) return buf[rm_slot<RMC>(c, i)];
         else return buf[c * LS + pad(i)];
@@ -344,34 +344,39 @@ __global__ __launch_bounds__(NT, WAVES) void fft_cols(
     }
 }
 
-// fft_cols for 1024-point columns, 8 per workgroup, and 2048-point columns, 4 per
-// workgroup, reading rows [0, r1) with r1 a multiple of 128 / C (the rest are zero): the
+// fft_cols for 128- to 512-point columns, 16 per workgroup, 1024-point columns, 8, and 2048-point
+// columns, 4, reading rows [0, r1) with r1 a multiple of 128 / C (the rest are zero): the
 // spectrum goes from HBM straight into LDS (16-byte direct loads, no registers held), so a
-// workgroup has all of its 64 KB in flight at once instead of two elements per thread.  Each wavefront load fills one 1 KB
+// workgroup has all of its 64 KB in flight at once instead of two elements per thread.
+// 512 points: the 2LPT of a 512^3 tile's 20 inverse passes 6.3 -> 5.0 ms (4.6 TB/s; 8 columns, i.e.
+// half lines, 5.1), the isolated convolution of a 256^3 tile's 8 1.89 -> 1.47 ms.  Each wavefront load fills one 1 KB
 // block of the row-major layout (rm_slot<C>): lane l brings columns 2 (l % (C/2)) and
 // 2 (l % (C/2)) + 1 of row (128/C) b + l / (C/2).  The operator's table entries are loaded
 // into registers meanwhile and the operator is applied in LDS, element by element as the
 // register path does, so the values are the same bit for bit.
 template <int L, int C>
 struct DirectShape {
-    static constexpr int LGL = L == 2048 ? 11 : 10, LGC = C == 8 ? 3 : 2;
+    static constexpr int LGL = L == 2048 ? 11 : L == 1024 ? 10 : L == 512 ? 9 : L == 256 ? 8 : 7;
+    static constexpr int LGC = C == 16 ? 4 : (C == 8 ? 3 : 2);
+    static constexpr int NT = C * L / 8;        // threads: a radix-8 butterfly each
     static constexpr int ROWS = 128 / C;        // rows per 1 KB block
     static constexpr int NB = L / ROWS;         // blocks
     static constexpr int LDS = NB * (ROWS + 1) * C;  // float2, a spare row per block
-    static_assert((L == 1024 && C == 8) || (L == 2048 && C == 4), "direct column shapes");
+    // Twiddles the Stockham stages read: index (k << (lgL - lgNs - lgR)) with k < Ns is below
+    // L / R of the last stage, i.e. below 32 (128 = 8 4 4), 64 (256 = 8 8 4, 512 = 8 8 8), 256
+    // (1024 = 8 8 4 4) and 512 (2048 = 8 8 8 4).
+    static constexpr int TW = L >= 1024 ? 512 : 128;
+    static_assert((1 << LGL) == L && L >= TW && NT >= TW / 2 && NT <= 1024, "direct column shapes");
 };
-// Twiddles the Stockham stages read: index (k << (lgL - lgNs - lgR)) with k < Ns is below
-// L / R of the last stage, i.e. below 256 (1024 = 8 8 4 4) and 512 (2048 = 8 8 8 4).
-constexpr int DIRECT_TW = 512;
-template <bool INV, int NT, int WAVES, int L, int C>
-__global__ __launch_bounds__(NT, WAVES) void fft_cols_direct(
+template <bool INV, int L, int C>
+__global__ __launch_bounds__(C * L / 8, 8) void fft_cols_direct(
     const float2* in, float2* out, int64_t strideA, int64_t strideB, int nx, int gx,
     int ntiles, int b0, int r1, int w0, int w1, FftOp op, const float2* __restrict__ W) {
     using S = DirectShape<L, C>;
-    constexpr int lgL = S::LGL, LGC = S::LGC, NB = S::NB, ROWS = S::ROWS;
+    constexpr int lgL = S::LGL, LGC = S::LGC, NB = S::NB, ROWS = S::ROWS, NT = S::NT;
     constexpr int EPT = C * L / NT;  // elements per thread
     __shared__ float2 buf[S::LDS];
-    __shared__ float2 tw[DIRECT_TW];  // the twiddles, read by every butterfly of the stages
+    __shared__ float2 tw[S::TW];  // the twiddles, read by every butterfly of the stages
     const int per = (ntiles + 7) >> 3;
     const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if (tile >= ntiles) return;
@@ -379,9 +384,9 @@ __global__ __launch_bounds__(NT, WAVES) void fft_cols_direct(
     const int b = b0 + tile / gx;
     const int64_t boff = (int64_t)b * strideB;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // the twiddles (4 KB) into LDS with the first four wavefronts' first direct loads: the
+    // the twiddles into LDS with the first wavefronts' first direct loads: the
     // stages then read them from LDS instead of waiting on L2 at every stage
-    if (wave < DIRECT_TW / 128)
+    if (wave < S::TW / 128)
         __builtin_amdgcn_global_load_lds(
             W + 128 * wave + 2 * lane, (__attribute__((address_space(3))) void*)(tw + 128 * wave),
             16, 0, 0);
@@ -417,7 +422,7 @@ __global__ __launch_bounds__(NT, WAVES) void fft_cols_direct(
         // the first radix-8 stage (span 1, no twiddles) with the operator applied to its
         // inputs as they are read: thread (c, j) takes elements j + (L/8) r of column c, the
         // very elements whose table entries it loaded (t[r])
-        static_assert(EPT == 8 && NT == 1024, "one radix-8 butterfly per thread");
+        static_assert(EPT == 8, "one radix-8 butterfly per thread");
         const int c = (int)threadIdx.x & (C - 1), j = (int)threadIdx.x >> LGC, x = x0 + c;
         float2 v[8];
 #pragma unroll
@@ -444,46 +449,110 @@ __global__ __launch_bounds__(NT, WAVES) void fft_cols_direct(
 // Forward x pass: rows (iy, iz) of a w^3 real field (iy, iz < w), zero-extended to L = 2M,
 // into rows of the (M + 1) x L x L half spectrum.  z[m] = x[2m] + i x[2m + 1], Z = FFT_M(z),
 // X[k] = E[k] + W_L^k O[k] with E = (Z[k] + conj Z[M-k]) / 2, O = (Z[k] - conj Z[M-k]) / 2i.
+// A wavefront takes 64-element pieces of the workgroup's rows, so that a piece's row (and its
+// place in the field) is the same for all lanes: the row divisions are the scalar unit's (per
+// element they and the twiddles' L2 reads bounded the row passes, with 4-byte loads and stores
+// of neighbouring reals: 512^3 forward 0.42 -> 0.29 ms, 1024^3 3.1 -> 1.9, inverse 1.62 -> 1.22).
+// `pairs`: w is even and f 8-byte aligned.  The twiddles of the stages lie in LDS.
+constexpr int ROW_TW = 256;  // entries the stages read: below M / 4 (1024 = 8 8 4 4)
+constexpr int ROW_U = SMALL_DATA / SMALL_T;  // pieces per wavefront
 __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_r2c(
-    const float* __restrict__ f, int w, int lgM, int lgG, float2* __restrict__ spec,
+    const float* __restrict__ f, int w, int lgM, int lgG, int pairs, float2* __restrict__ spec,
     const float2* __restrict__ WM, const float2* __restrict__ WL) {
     __shared__ float2 buf[SMALL_LDS];
+    __shared__ float2 tw[ROW_TW];
     const int M = 1 << lgM, G = 1 << lgG, LS = padded_len(M), L = 2 * M, nk = M + 1;
     const int row0 = (int)blockIdx.x * G;
     const int nrows = w * w;
-    // two elements per step, both loads issued before either is used
-    for (int e0 = threadIdx.x; e0 < G * M; e0 += 2 * SMALL_T) {
-        float2 v[2];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int lgP = lgM > 6 ? lgM - 6 : 0;  // pieces per row
+    if ((int)threadIdx.x < min(M, ROW_TW)) tw[threadIdx.x] = WM[threadIdx.x];
+    float2 v[ROW_U];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = e0 + u * SMALL_T;
-            const int g = e >> lgM, m = e & (M - 1), row = row0 + g;
-            v[u] = make_float2(0.0f, 0.0f);
-            if (e < G * M && row < nrows) {
-                const float* src = f + (int64_t)row * w;
-                const int x = 2 * m;
-                v[u] = make_float2(x < w ? src[x] : 0.0f, x + 1 < w ? src[x + 1] : 0.0f);
+    for (int u = 0; u < ROW_U; ++u) {
+        const int piece = wave + u * (SMALL_T / 64), g = piece >> lgP;
+        const int m = ((piece & ((1 << lgP) - 1)) << 6) + lane, x = 2 * m;
+        v[u] = make_float2(0.0f, 0.0f);
+        if (g < G && row0 + g < nrows && m < M) {
+            const float* src = f + (int64_t)(row0 + g) * w;
+            if (pairs) {
+                if (x < w) v[u] = *reinterpret_cast<const float2*>(src + x);
+            } else {
+                if (x < w) v[u].x = src[x];
+                if (x + 1 < w) v[u].y = src[x + 1];
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < ROW_U; ++u) {
+        const int piece = wave + u * (SMALL_T / 64), g = piece >> lgP;
+        const int m = ((piece & ((1 << lgP) - 1)) << 6) + lane;
+        if (g < G && m < M) buf[g * LS + pad(m)] = v[u];
+    }
+    __syncthreads();
+    stockham<false, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, tw);
+    for (int g = wave; g < G; g += SMALL_T / 64) {
+        const int row = row0 + g;
+        if (row >= nrows) break;
+        const int iz = row / w, iy = row - iz * w;
+        float2* __restrict__ dst = spec + (int64_t)fft_pitch(L) * iy + fft_plane(L) * iz;
+        for (int k = lane; k < nk; k += 64) {
+            const float2 zk = buf[g * LS + pad(k & (M - 1))];
+            const float2 zm = buf[g * LS + pad((M - k) & (M - 1))];
+            const float2 ev = make_float2((zk.x + zm.x) * 0.5f, (zk.y - zm.y) * 0.5f);
+            // (zk - conj zm) / 2i
+            const float2 od = make_float2((zk.y + zm.y) * 0.5f, -(zk.x - zm.x) * 0.5f);
+            const float2 t = ctw<false>(od, WL[k]);
+            dst[k] = cadd(ev, t);
+        }
+    }
+}
+
+// The kept part of the inverse x pass's rows, from their FFTs in LDS; `pairs`: s and n even, out
+// 8-byte aligned.
+__device__ __forceinline__ void store_rows(const float2* buf, int LS, int G, int row0, int nrows,
+                                           int s, int n, float scale, int mode, float coef,
+                                           int pairs, float* __restrict__ out) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (pairs) {
+        const int np = (n / 2 + 63) >> 6;  // pieces of 64 pairs per row
+        float2 old[ROW_U];
+        if (mode != 0) {
+#pragma unroll
+            for (int u = 0; u < ROW_U; ++u) {
+                const int piece = wave + u * (SMALL_T / 64), g = piece / np;
+                const int j = ((piece - g * np) << 6) + lane;
+                if (g < G && row0 + g < nrows && j < n / 2)
+                    old[u] = *reinterpret_cast<const float2*>(out + (int64_t)(row0 + g) * n + 2 * j);
             }
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = e0 + u * SMALL_T;
-            if (e < G * M) buf[(e >> lgM) * LS + pad(e & (M - 1))] = v[u];
+        for (int u = 0; u < ROW_U; ++u) {
+            const int piece = wave + u * (SMALL_T / 64), g = piece / np;
+            const int j = ((piece - g * np) << 6) + lane;
+            if (g < G && row0 + g < nrows && j < n / 2) {
+                const float2 z = buf[g * LS + pad((s >> 1) + j)];
+                float2 v = make_float2(z.x * scale, z.y * scale);
+                if (mode != 0)
+                    v = make_float2(old[u].x - (v.x * v.x) * coef, old[u].y - (v.y * v.y) * coef);
+                *reinterpret_cast<float2*>(out + (int64_t)(row0 + g) * n + 2 * j) = v;
+            }
         }
+        return;
     }
-    __syncthreads();
-    stockham<false, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, WM);
-    for (int e = threadIdx.x; e < G * nk; e += SMALL_T) {
-        const int g = e / nk, k = e - g * nk, row = row0 + g;
-        if (row >= nrows) continue;
-        const int iy = row % w, iz = row / w;
-        const float2 zk = buf[g * LS + pad(k & (M - 1))];
-        const float2 zm = buf[g * LS + pad((M - k) & (M - 1))];
-        const float2 ev = make_float2((zk.x + zm.x) * 0.5f, (zk.y - zm.y) * 0.5f);
-        // (zk - conj zm) / 2i
-        const float2 od = make_float2((zk.y + zm.y) * 0.5f, -(zk.x - zm.x) * 0.5f);
-        const float2 t = ctw<false>(od, WL[k]);
-        spec[k + (int64_t)fft_pitch(L) * iy + fft_plane(L) * iz] = cadd(ev, t);
+    for (int g = wave; g < G; g += SMALL_T / 64) {
+        const int row = row0 + g;
+        if (row >= nrows) break;
+        for (int xo = lane; xo < n; xo += 64) {
+            const int xx = s + xo;
+            const float2 zz = buf[g * LS + pad(xx >> 1)];
+            const float v = ((xx & 1) ? zz.y : zz.x) * scale;
+            const int64_t o = (int64_t)row * n + xo;
+            if (mode == 0) out[o] = v;
+            else out[o] = out[o] - (v * v) * coef;
+        }
     }
 }
 
@@ -494,33 +563,40 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_r2c(
 // x[2m + 1] = Im z[m].
 __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r(
     const float2* __restrict__ spec, int lgM, int lgG, int s, int n, float scale, int mode,
-    float coef, float* __restrict__ out, const float2* __restrict__ WM,
+    float coef, int pairs, float* __restrict__ out, const float2* __restrict__ WM,
     const float2* __restrict__ WL) {
     __shared__ float2 buf[SMALL_LDS];
-    const int M = 1 << lgM, G = 1 << lgG, LS = padded_len(M), L = 2 * M, nk = M + 1;
+    __shared__ float2 tw[ROW_TW];
+    const int M = 1 << lgM, G = 1 << lgG, LS = padded_len(M), L = 2 * M;
     const int row0 = (int)blockIdx.x * G;
     const int nrows = n * n;
-    // two elements per step, both loads issued before either is used
-    for (int e0 = threadIdx.x; e0 < G * nk; e0 += 2 * SMALL_T) {
-        float2 v[2];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int lgP = lgM > 6 ? lgM - 6 : 0;  // pieces per row
+    if ((int)threadIdx.x < min(M, ROW_TW)) tw[threadIdx.x] = WM[threadIdx.x];
+    {
+        float2 v[ROW_U], nyq = make_float2(0.0f, 0.0f);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = e0 + u * SMALL_T;
-            const int g = e / nk, k = e - g * nk, row = row0 + g;
+        for (int u = 0; u < ROW_U; ++u) {
+            const int piece = wave + u * (SMALL_T / 64), g = piece >> lgP;
+            const int k = ((piece & ((1 << lgP) - 1)) << 6) + lane;
             v[u] = make_float2(0.0f, 0.0f);
-            if (e < G * nk && row < nrows) {
-                const int iy = s + row % n, iz = s + row / n;
-                v[u] = spec[k + (int64_t)fft_pitch(L) * iy + fft_plane(L) * iz];
+            if (g < G && row0 + g < nrows && k < M) {
+                const int jz = (row0 + g) / n, jy = row0 + g - jz * n;
+                v[u] = spec[k + (int64_t)fft_pitch(L) * (s + jy) + fft_plane(L) * (s + jz)];
             }
+        }
+        if ((int)threadIdx.x < G && row0 + (int)threadIdx.x < nrows) {
+            const int row = row0 + threadIdx.x, jz = row / n, jy = row - jz * n;
+            nyq = spec[M + (int64_t)fft_pitch(L) * (s + jy) + fft_plane(L) * (s + jz)];
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = e0 + u * SMALL_T;
-            if (e < G * nk) {
-                const int g = e / nk;
-                buf[g * LS + pad(e - g * nk)] = v[u];
-            }
+        for (int u = 0; u < ROW_U; ++u) {
+            const int piece = wave + u * (SMALL_T / 64), g = piece >> lgP;
+            const int k = ((piece & ((1 << lgP) - 1)) << 6) + lane;
+            if (g < G && k < M) buf[g * LS + pad(k)] = v[u];
         }
+        if ((int)threadIdx.x < G) buf[threadIdx.x * LS + pad(M)] = nyq;
     }
     __syncthreads();
     // untwist into Z (registers first: Z[k] needs X[M - k] of the same row)
@@ -550,38 +626,35 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r(
         if (e < G * M) buf[(e >> lgM) * LS + pad(e & (M - 1))] = z[q];
     }
     __syncthreads();
-    stockham<true, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, WM);
-    for (int e = threadIdx.x; e < G * n; e += SMALL_T) {
-        const int g = e / n, xo = e - g * n, row = row0 + g;
-        if (row >= nrows) continue;
-        const int xx = s + xo;
-        const float2 zz = buf[g * LS + pad(xx >> 1)];
-        const float v = ((xx & 1) ? zz.y : zz.x) * scale;
-        const int64_t o = (int64_t)row * n + xo;
-        if (mode == 0) out[o] = v;
-        else out[o] = out[o] - (v * v) * coef;
-    }
+    stockham<true, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, tw);
+    store_rows(buf, LS, G, row0, nrows, s, n, scale, mode, coef, pairs, out);
 }
 
-// fft_rows_c2r for L = 1024 (M = 512, 8 rows per workgroup) and L = 2048 (M = 1024, 4
-// rows) with the rows loaded straight into LDS: each row's first M coefficients as M / 128
+// fft_rows_c2r for L = 512 (M = 256, 16 rows per workgroup; 0.50 -> 0.25 ms for 512^3 with the
+// pieces of store_rows), L = 1024 (M = 512, 8 rows) and L = 2048 (M = 1024, 4 rows) with the rows loaded straight into LDS: each row's first M coefficients as M / 128
 // 1 KB direct loads into an unpadded staging layout (row g at g P, as in the spectrum), the
 // Nyquist coefficient X[M] by an ordinary load; the untwist reads the staging layout and
 // writes the padded FFT layout over it after a barrier.  Same arithmetic as fft_rows_c2r,
 // so the same values bit for bit.
 template <int LGM>
 __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r_direct(
-    const float2* __restrict__ spec, int s, int n, float scale, int mode, float coef,
+    const float2* __restrict__ spec, int s, int n, float scale, int mode, float coef, int pairs,
     float* __restrict__ out, const float2* __restrict__ WM, const float2* __restrict__ WL) {
     constexpr int lgM = LGM, M = 1 << LGM, G = SMALL_DATA / M, L = 2 * M, P = fft_pitch(L);
     constexpr int Q = M / 128, LGQ = LGM - 7;  // 1 KB chunks per row
-    static_assert((LGM == 9 || LGM == 10) && G * padded_len(M) <= SMALL_LDS, "row shapes");
+    static_assert(LGM >= 8 && LGM <= 10 && G * padded_len(M) <= SMALL_LDS, "row shapes");
     static_assert(G * P <= SMALL_LDS, "staging rows fit the FFT buffer");
     __shared__ float2 buf[SMALL_LDS];
+    __shared__ float2 tw[ROW_TW];
     const int LS = padded_len(M);
     const int row0 = (int)blockIdx.x * G;
     const int nrows = n * n;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;  // 8 wavefronts
+    const int lane = threadIdx.x & 63;  // 8 wavefronts
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (wave < ROW_TW / 128)
+        __builtin_amdgcn_global_load_lds(
+            WM + 128 * wave + 2 * lane, (__attribute__((address_space(3))) void*)(tw + 128 * wave),
+            16, 0, 0);
     // 32 chunks (G rows x Q) over the 8 wavefronts
     for (int u = wave; u < Q * G; u += SMALL_T / 64) {
         const int g = u >> LGQ, q = u & (Q - 1);
@@ -626,17 +699,8 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r_direct(
         buf[(e >> lgM) * LS + pad(e & (M - 1))] = z[q];
     }
     __syncthreads();
-    stockham<true, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, WM);
-    for (int e = threadIdx.x; e < G * n; e += SMALL_T) {
-        const int g = e / n, xo = e - g * n, row = row0 + g;
-        if (row >= nrows) continue;
-        const int xx = s + xo;
-        const float2 zz = buf[g * LS + pad(xx >> 1)];
-        const float v = ((xx & 1) ? zz.y : zz.x) * scale;
-        const int64_t o = (int64_t)row * n + xo;
-        if (mode == 0) out[o] = v;
-        else out[o] = out[o] - (v * v) * coef;
-    }
+    stockham<true, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, tw);
+    store_rows(buf, LS, G, row0, nrows, s, n, scale, mode, coef, pairs, out);
 }
 
 // sqrt P per (ix, |iy|, |iz|) of the transfer: the (L/2 + 1)^3 table the inverse z pass reads
@@ -702,17 +766,29 @@ void launch_cols(hipStream_t st, int L, unsigned gx, int nb, const float2* in, f
                  int w1, const FftOp& op, const float2* W, bool direct = false) {
     const int lgC = cols_lgC(L);
     const int LS = cols_ls(L, 1 << lgC);
-    if (direct && r0 == 0 && r1 <= L && r1 % 16 == 0 && L == 1024 && lgC == 3) {
-        hipLaunchKernelGGL((fft_cols_direct<INV, BIG_T, 8, 1024, 8>), dim3(cols_grid(gx, nb)),
-                           dim3(BIG_T), 0, st, in, out, strideA, strideB, nx, (int)gx,
-                           (int)gx * nb, b0, r1, w0, w1, op, W);
-        return;
-    }
-    if (direct && r0 == 0 && r1 <= L && r1 % 32 == 0 && L == 2048 && lgC == 2) {
-        hipLaunchKernelGGL((fft_cols_direct<INV, BIG_T, 8, 2048, 4>), dim3(cols_grid(gx, nb)),
-                           dim3(BIG_T), 0, st, in, out, strideA, strideB, nx, (int)gx,
-                           (int)gx * nb, b0, r1, w0, w1, op, W);
-        return;
+    if (direct && r0 == 0 && r1 <= L) {
+        bool done = true;
+        const auto launch = [&](auto shape) {
+            using S = decltype(shape);
+            constexpr int C = 1 << S::LGC;
+            const unsigned g = (unsigned)((nx + C - 1) / C);
+            if (r1 % S::ROWS != 0) {
+                done = false;
+                return;
+            }
+            hipLaunchKernelGGL((fft_cols_direct<INV, 1 << S::LGL, C>), dim3(cols_grid(g, nb)),
+                               dim3(S::NT), 0, st, in, out, strideA, strideB, nx, (int)g,
+                               (int)g * nb, b0, r1, w0, w1, op, W);
+        };
+        switch (L) {
+            case 128: launch(DirectShape<128, 16>{}); break;
+            case 256: launch(DirectShape<256, 16>{}); break;
+            case 512: launch(DirectShape<512, 16>{}); break;
+            case 1024: launch(DirectShape<1024, 8>{}); break;
+            case 2048: launch(DirectShape<2048, 4>{}); break;
+            default: done = false;
+        }
+        if (done) return;
     }
     if (cols_big(L))
         hipLaunchKernelGGL((fft_cols<INV, BIG_T, BIG_LDS, BIG_DATA, 8>), dim3(cols_grid(gx, nb)), dim3(BIG_T),
@@ -766,7 +842,8 @@ hnt_status fft_forward(hnt_ctx* ctx, const float* f, int w, int L, float2* spec)
     const int lgG = rows_lgG(M);
     const int64_t rows = (int64_t)w * w;
     hipLaunchKernelGGL(fft_rows_r2c, dim3((unsigned)((rows + (1 << lgG) - 1) >> lgG)),
-                       dim3(SMALL_T), 0, st, f, w, ilog2(M), lgG, spec, WM, WL);
+                       dim3(SMALL_T), 0, st, f, w, ilog2(M), lgG, w % 2 == 0 && ((uintptr_t)f & 7) == 0, spec,
+                       WM, WL);
     FftOp none;
     const int lgC = cols_lgC(L);
     const unsigned gx = (unsigned)((nk + (1 << lgC) - 1) >> lgC);
@@ -799,21 +876,28 @@ hnt_status fft_inverse(hnt_ctx* ctx, const float2* spec, float2* work, int L, in
                       s + n, none, WL, ctx->fft_direct != 0);
     const int lgG = rows_lgG(M);
     const int64_t rows = (int64_t)n * n;
+    const int pairs = s % 2 == 0 && n % 2 == 0 && ((uintptr_t)out & 7) == 0;
+    if (ctx->fft_direct && L == 512 && lgG == 4) {
+        hipLaunchKernelGGL(fft_rows_c2r_direct<8>, dim3((unsigned)((rows + 15) >> 4)),
+                           dim3(SMALL_T), 0, st, (const float2*)work, s, n, scale, mode, coef,
+                           pairs, out, WM, WL);
+        return HNT_OK;
+    }
     if (ctx->fft_direct && L == 1024 && lgG == 3) {
         hipLaunchKernelGGL(fft_rows_c2r_direct<9>, dim3((unsigned)((rows + 7) >> 3)),
                            dim3(SMALL_T), 0, st, (const float2*)work, s, n, scale, mode, coef,
-                           out, WM, WL);
+                           pairs, out, WM, WL);
         return HNT_OK;
     }
     if (ctx->fft_direct && L == 2048 && lgG == 2) {
         hipLaunchKernelGGL(fft_rows_c2r_direct<10>, dim3((unsigned)((rows + 3) >> 2)),
                            dim3(SMALL_T), 0, st, (const float2*)work, s, n, scale, mode, coef,
-                           out, WM, WL);
+                           pairs, out, WM, WL);
         return HNT_OK;
     }
     hipLaunchKernelGGL(fft_rows_c2r, dim3((unsigned)((rows + (1 << lgG) - 1) >> lgG)),
                        dim3(SMALL_T), 0, st, (const float2*)work, ilog2(M), lgG, s, n, scale,
-                       mode, coef, out, WM, WL);
+                       mode, coef, pairs, out, WM, WL);
     return HNT_OK;
 }
 

@@ -99,8 +99,8 @@ hnt_status hnt_ctx_get_profile(hnt_ctx* ctx, double* ms, int64_t* calls, int32_t
  *  FFT:          transforms of the field-synthesis entries.  0 (default): the library's own
  *                FFTs for power-of-two sizes 8..2048 (hipFFT otherwise); 1: hipFFT always.
  *                Both are Float32 transforms; results differ by their rounding.
- *  FFT_DIRECT:   1 (default): the library's 1024- and 2048-point column passes (reading
- *                whole 1 KB blocks of rows, the rest zero) and its 1024- and 2048-point
+ *  FFT_DIRECT:   1 (default): the library's 128- to 2048-point column passes (reading
+ *                whole 1 KB blocks of rows, the rest zero) and its 512- to 2048-point
  *                complex-to-real row passes load straight into LDS (no registers held, a
  *                workgroup's 64 KB in flight at once); 0: through registers, two elements
  *                per thread at a time.  Speed only: the results are the same bit for bit.
