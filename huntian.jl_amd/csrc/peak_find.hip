@@ -407,17 +407,24 @@ __device__ __forceinline__ float window32(double k2, double Rf, int wsmooth) {
 // written: 0.54 GB of table instead of 8.6 GB of spectrum traffic per filter at 1024^3.
 // The table is laid out as the z pass reads it, |kz| fastest: entry az + nk (ix + nk ay).
 // One workgroup per (kx, |ky|) row of the table: blockIdx.x + nk blockIdx.y is
-// ix + nk ay for ix < nk, ay < nk (no 64-bit division per element).
+// ix + nk ay for ix < nk, ay < nk (no 64-bit division per element).  (kx, ky, kz) and (ky, kx, kz)
+// have the same k^2, kx^2 + ky^2 being the same sum, so the workgroups with kx <= ky evaluate the
+// window (FP64 sin and cos, what bounds this kernel) and write it to both rows: 0.61 -> 0.34 ms
+// per filter at 1024^3.
 __global__ __launch_bounds__(256) void fb_wtable(int n, double dk, double Rf, int wsmooth,
                                                  float* __restrict__ w) {
     const int nk = n / 2 + 1;
     const int ix = (int)blockIdx.x, ay = (int)blockIdx.y;
+    if (ix > ay) return;
     const double kx = (double)ix * dk, ky = (double)ay * dk;
     float* row = w + (int64_t)nk * (ix + (int64_t)nk * ay);
+    float* mirror = w + (int64_t)nk * (ay + (int64_t)nk * ix);
     for (int az = threadIdx.x; az < nk; az += 256) {
         const double kz = (double)az * dk;
         const double k2 = kx * kx + ky * ky + kz * kz;
-        row[az] = k2 != 0.0 ? window32(k2, Rf, wsmooth) : 1.0f;
+        const float v = k2 != 0.0 ? window32(k2, Rf, wsmooth) : 1.0f;
+        row[az] = v;
+        mirror[az] = v;
     }
 }
 
