@@ -462,7 +462,7 @@ static void release_scratch(hnt_ctx* ctx) {
                       &ctx->fs_base, &ctx->fs_work, &ctx->fs_aux, &ctx->fs_tab})
         release(*b);
     MergeBufs& m = ctx->mg;
-    for (DevBuf* b : {&m.a, &m.b, &m.c, &m.d, &m.rank, &m.cidx, &m.cstart, &m.cnt, &m.off, &m.e1,
+    for (DevBuf* b : {&m.a, &m.b, &m.c, &m.d, &m.rank, &m.cidx, &m.cstart, &m.off, &m.e1,
                       &m.e2, &m.e3, &m.e4, &m.state, &m.instart, &m.dv, &m.pk, &m.pv, &m.newr,
                       &m.pos, &m.prank, &m.ext})
         release(*b);

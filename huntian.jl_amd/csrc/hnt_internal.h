@@ -75,7 +75,7 @@ struct TileDev {
 // scratch of hnt_merge_catalog: sort keys and permutations, ranks, the cell hash,
 // containment edges, decision states, overlap pairs, volume deficits, new radii
 struct MergeBufs {
-    DevBuf a, b, c, d, rank, cidx, cstart, cnt, off, e1, e2, e3, e4, state, instart, dv, pk,
+    DevBuf a, b, c, d, rank, cidx, cstart, off, e1, e2, e3, e4, state, instart, dv, pk,
         pv, newr, pos, prank, ext;
 };
 

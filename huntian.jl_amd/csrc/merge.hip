@@ -126,90 +126,6 @@ __global__ void merge_gather(const float* __restrict__ rec, int64_t N, int nf,
     prank[p] = rank[m];
 }
 
-// Visit the positions of the halos in the cells within +-dcell of (xi, yi, zi)'s cell, in the
-// reference's order: cells by dz, dy, dx; within a cell by descending catalog index.
-template <class F>
-__device__ __forceinline__ void for_neighbours(const Grid& g, double xi, double yi, double zi,
-                                               int dcell, F&& f) {
-    const int ci = cell_of(xi, g.ox, g.cell, g.nc), cj = cell_of(yi, g.oy, g.cell, g.nc),
-              ck = cell_of(zi, g.oz, g.cell, g.nc);
-    for (int dz = -dcell; dz <= dcell; ++dz) {
-        const int jz = ck + dz;
-        if (jz < 1 || jz > g.nc) continue;
-        for (int dy = -dcell; dy <= dcell; ++dy) {
-            const int jy = cj + dy;
-            if (jy < 1 || jy > g.nc) continue;
-            const int64_t row = (int64_t)g.nc * ((jy - 1) + (int64_t)g.nc * (jz - 1));
-            for (int dx = -dcell; dx <= dcell; ++dx) {
-                const int jx = ci + dx;
-                if (jx < 1 || jx > g.nc) continue;
-                const int64_t c = (jx - 1) + row;
-                const int32_t e = g.cell_start[c + 1];
-                for (int32_t q = g.cell_start[c]; q < e; ++q) f((int64_t)q);
-            }
-        }
-    }
-}
-
-// Containment edges p -> q: rank q > rank p and |x_q - x_p| < r_p (lagrangian_exclusion!,
-// Exclusion.jl:110-131).  write == 0 counts, write == 1 fills from off[p].
-__global__ void merge_edges(Grid g, int write, int64_t* __restrict__ cnt,
-                            const int64_t* __restrict__ off, int32_t* __restrict__ src,
-                            int32_t* __restrict__ dst) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= g.N) return;
-    const float4 me = g.pos[p];
-    const double xi = me.x, yi = me.y, zi = me.z, ri = me.w;
-    const int dcell = (int)ceil(ri / g.cell);
-    const int32_t rkp = g.prank[p];
-    int64_t n = 0, w = write ? off[p] : 0;
-    for_neighbours(g, xi, yi, zi, dcell, [&](int64_t q) {
-        if (g.prank[q] <= rkp) return;  // also q == p
-        const float4 o = g.pos[q];
-        const double dx = (double)o.x - xi, dy = (double)o.y - yi, dz = (double)o.z - zi;
-        const double dist = sqrt(dx * dx + dy * dy + dz * dz);
-        if (dist < ri) {
-            if (write) {
-                src[w] = (int32_t)p;
-                dst[w] = (int32_t)q;
-                ++w;
-            } else {
-                ++n;
-            }
-        }
-    });
-    if (!write) cnt[p] = n;
-}
-
-// One round of decisions: state 0 undecided, 1 alive, 2 dead.  in_start / in_src: containers
-// of each halo (CSR by position).
-__global__ void merge_round(int64_t N, const int64_t* __restrict__ in_start,
-                            const int32_t* __restrict__ in_src, uint8_t* __restrict__ state,
-                            unsigned long long* __restrict__ undecided) {
-    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= N || state[j] != 0) return;
-    bool all_dead = true;
-    for (int64_t e = in_start[j]; e < in_start[j + 1]; ++e) {
-        const uint8_t s = state[in_src[e]];
-        if (s == 1) {
-            state[j] = 2;
-            return;
-        }
-        if (s != 2) all_dead = false;
-    }
-    if (all_dead) state[j] = 1;
-    else atomicAdd(undecided, 1ull);
-}
-
-// start[j] = first entry of halo j in entries sorted by halo (key >> shift), j = 0 .. N
-template <class K>
-__global__ void merge_csr(const K* __restrict__ sorted, int64_t E, int64_t N, int shift,
-                          int64_t* __restrict__ start) {
-    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j > N) return;
-    start[j] = j == N ? E : lower_bound(sorted, E, (K)((K)j << shift));
-}
-
 // sphere_overlap (Exclusion.jl:86-101): caps (v1, v2) cut from spheres r1, r2 at distance d
 __device__ __forceinline__ void sphere_overlap(double d, double r1, double r2, double& v1,
                                                double& v2) {
@@ -222,48 +138,156 @@ __device__ __forceinline__ void sphere_overlap(double d, double r1, double r2, d
     v2 = (M_PI / 3.0) * (h2 * h2) * (3.0 * r2 - h2);
 }
 
-// Overlapping survivor pairs (p larger by rank) of volume_reduction! (Exclusion.jl:163-180).
-// Every pair gives two caps: the one cut from the smaller halo q, keyed (q << 32 | rank p),
-// and p's own, keyed (p << 32 | N + q).  Sorted by key, a halo's caps come in the reference's
-// order: those cut by larger halos in their rank order, then its own in its cell-scan order
-// (cells by dz, dy, dx, descending catalog index within a cell = ascending position q).
-// mode 0 counts two entries per pair; mode 1 writes them from off[p].
-__global__ void merge_pairs(Grid g, int mode, const uint8_t* __restrict__ state,
-                            int fortran_ties, int64_t* __restrict__ cnt,
-                            const int64_t* __restrict__ off, uint64_t* __restrict__ keys,
-                            double* __restrict__ vals) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= g.N) return;
-    if (state[p] != 1) {
-        if (mode == 0) cnt[p] = 0;  // the scan reads every count: none may be left over
+// The neighbour scans: SCAN_W lanes per halo p, a row of cells (fixed y and z) each.  A row's cells
+// are consecutive, so its halos are one run of positions; every halo of lower rank than p that
+// passes the test is listed in LDS and the workgroup's list is then written out together, behind
+// one atomic on the count.  The order of the entries does not matter: the containment edges are
+// sorted by contained halo and only asked whether any or all of a halo's containers live, and
+// the caps' keys are all different.  Entries beyond `cap` are counted only; the caller makes room
+// and scans again.  (One thread per halo, looking every cell up, counting in one scan and
+// writing in a second: 8.0 + 1.9 ms for 2 M halos, most of it the threads with large radii and
+// hundreds of cells; now 1.3 + 0.4 ms.  Lanes per halo: edges, mostly 9 rows, 2, 4, 8, 16: 0.60,
+// 0.57, 0.78, 1.51 ms; pairs, 25 rows and more, 4, 8, 16: 1.40, 1.34, 1.54 ms.)
+//
+// Edges (PAIRS = false; lagrangian_exclusion!, Exclusion.jl:110-131): |x_q - x_p| < r_p.
+//
+// Pairs (volume_reduction!, Exclusion.jl:163-180): survivors whose spheres overlap (the others'
+// rank is -1 by then).  Every pair
+// gives two caps: the one cut from the smaller halo q, keyed (q << lb | rank p), and p's own,
+// keyed (p << lb | N + q), lb the bits of 2 N.  Sorted by key, a halo's caps come in the
+// reference's order: those cut by larger halos in their rank order, then its own in its
+// cell-scan order (cells by dz, dy, dx, descending catalog index within a cell = ascending
+// position q).
+constexpr int EDGE_W = 4, PAIR_W = 8, SCAN_LIST = 2048;
+
+struct ScanOut {
+    int64_t cap;                 // edges or pairs
+    unsigned long long* count;
+    int32_t *src, *dst;          // edges
+    uint64_t* keys;              // pairs: two entries each
+    double* vals;
+    int lb, fortran_ties;
+};
+
+template <bool PAIRS>
+__device__ __forceinline__ void scan_emit(const Grid& g, const ScanOut& o, int64_t e, int p, int q) {
+    if (e >= o.cap) return;
+    if (!PAIRS) {
+        o.src[e] = p;
+        o.dst[e] = q;
         return;
     }
-    const float4 me = g.pos[p];
-    const double xi = me.x, yi = me.y, zi = me.z, ri = me.w;
-    const int dcell = (int)ceil(2.0 * ri / g.cell);
-    const int32_t rkp = g.prank[p];
-    int64_t n = 0, w = mode == 1 ? off[p] : 0;
-    for_neighbours(g, xi, yi, zi, dcell, [&](int64_t q) {
-        if (g.prank[q] <= rkp || state[q] != 1) return;
-        const float4 o = g.pos[q];
-        const double rj = o.w;
-        const double ex = (double)o.x - xi, ey = (double)o.y - yi, ez = (double)o.z - zi;
-        const double d = sqrt(ex * ex + ey * ey + ez * ez);
-        if (!(d < ri + rj)) return;
-        if (mode == 0) {
-            n += 2;
-            return;
+    const float4 me = g.pos[p], ot = g.pos[q];
+    const double ri = me.w, rj = ot.w;
+    const double ex = (double)ot.x - (double)me.x, ey = (double)ot.y - (double)me.y,
+                 ez = (double)ot.z - (double)me.z;
+    const double d = sqrt(ex * ex + ey * ey + ez * ez);
+    double v1, v2;
+    sphere_overlap(d, ri, rj, v1, v2);
+    const double wgt = (o.fortran_ties && rj == ri) ? 2.0 : 1.0;
+    o.keys[2 * e] = ((uint64_t)q << o.lb) | (uint32_t)g.prank[p];
+    o.vals[2 * e] = wgt * v2;
+    o.keys[2 * e + 1] = ((uint64_t)p << o.lb) | (uint64_t)(g.N + q);
+    o.vals[2 * e + 1] = wgt * v1;
+}
+
+template <bool PAIRS>
+__global__ __launch_bounds__(MB) void merge_scan(Grid g, ScanOut o) {
+    constexpr int SCAN_W = PAIRS ? PAIR_W : EDGE_W;
+    __shared__ int2 list[SCAN_LIST];
+    __shared__ int listed;
+    __shared__ unsigned long long base;
+    const int tid = threadIdx.x, lane = tid & (SCAN_W - 1);
+    const int64_t p = (int64_t)blockIdx.x * (MB / SCAN_W) + tid / SCAN_W;
+    if (tid == 0) listed = 0;
+    __syncthreads();
+    const int32_t rkp = p < g.N ? g.prank[p] : -1;
+    if (rkp >= 0) {
+        const float4 me = g.pos[p];
+        const double xi = me.x, yi = me.y, zi = me.z, ri = me.w;
+        const int dcell = (int)ceil((PAIRS ? 2.0 * ri : ri) / g.cell);
+        const int ci = cell_of(xi, g.ox, g.cell, g.nc), cj = cell_of(yi, g.oy, g.cell, g.nc),
+                  ck = cell_of(zi, g.oz, g.cell, g.nc);
+        const int x0 = max(1, ci - dcell), x1 = min(g.nc, ci + dcell);
+        const int y0 = max(1, cj - dcell), ny = min(g.nc, cj + dcell) - y0 + 1;
+        const int z0 = max(1, ck - dcell), nz = min(g.nc, ck + dcell) - z0 + 1;
+        const int rows = dcell >= 0 ? ny * nz : 0;
+        for (int r = lane; r < rows; r += SCAN_W) {
+            const int dz = r / ny;
+            const int64_t row = (int64_t)g.nc * ((y0 + r - dz * ny - 1) + (int64_t)g.nc * (z0 + dz - 1));
+            const int32_t e = g.cell_start[row + x1];
+            for (int32_t q = g.cell_start[row + x0 - 1]; q < e; q += 4) {
+                int32_t rk[4];
+                float4 ot[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    rk[u] = g.prank[min(q + u, e - 1)];
+                    ot[u] = g.pos[min(q + u, e - 1)];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (q + u >= e || rk[u] <= rkp) continue;  // also q + u == p
+                    const double dx = (double)ot[u].x - xi, dy = (double)ot[u].y - yi,
+                                 dw = (double)ot[u].z - zi;
+                    const double d = sqrt(dx * dx + dy * dy + dw * dw);
+                    if (!(d < (PAIRS ? ri + (double)ot[u].w : ri))) continue;
+                    const int at = atomicAdd(&listed, 1);
+                    if (at < SCAN_LIST) list[at] = make_int2((int)p, q + u);
+                    else scan_emit<PAIRS>(g, o, (int64_t)atomicAdd(o.count, 1ull), (int)p, q + u);
+                }
+            }
         }
-        double v1, v2;
-        sphere_overlap(d, ri, rj, v1, v2);
-        const double wgt = (fortran_ties && rj == ri) ? 2.0 : 1.0;
-        keys[w] = ((uint64_t)q << 32) | (uint32_t)rkp;
-        vals[w] = wgt * v2;
-        keys[w + 1] = ((uint64_t)p << 32) | (uint32_t)(g.N + q);
-        vals[w + 1] = wgt * v1;
-        w += 2;
-    });
-    if (mode == 0) cnt[p] = n;
+    }
+    __syncthreads();
+    const int n = min(listed, SCAN_LIST);
+    if (n == 0) return;
+    if (tid == 0) base = atomicAdd(o.count, (unsigned long long)n);
+    __syncthreads();
+    for (int i = tid; i < n; i += MB)
+        scan_emit<PAIRS>(g, o, (int64_t)base + i, list[i].x, list[i].y);
+}
+
+// One round of decisions: state 0 undecided, 1 alive, 2 dead.  in_start / in_src: containers
+// of each halo (CSR by position).  The first round, before anything is decided, only asks for
+// halos without containers.  *undecided becomes 1 if any halo stays so: a store per workgroup (an
+// atomic count per wavefront took 0.3 ms of each of the first two rounds at 2 M halos).
+__global__ __launch_bounds__(MB) void merge_round(int64_t N, int first,
+                                                  const int64_t* __restrict__ in_start,
+                                                  const int32_t* __restrict__ in_src,
+                                                  uint8_t* __restrict__ state,
+                                                  unsigned long long* __restrict__ undecided) {
+    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    bool open = false;
+    if (j < N && state[j] == 0) {
+        const int64_t e0 = in_start[j], e1 = in_start[j + 1];
+        uint8_t mine = 1;  // unless a container is alive or undecided
+        if (first) mine = e0 == e1 ? 1 : 0;
+        else
+            for (int64_t e = e0; e < e1 && mine != 2; ++e) {
+                const uint8_t s = state[in_src[e]];
+                if (s == 1) mine = 2;
+                else if (s == 0) mine = 0;
+            }
+        if (mine != 0) state[j] = mine;
+        open = mine == 0;
+    }
+    if (__syncthreads_or(open) && threadIdx.x == 0) *undecided = 1ull;
+}
+
+// start[j] = first entry of halo j in entries sorted by halo (key >> shift), j = 0 .. N
+template <class K>
+__global__ void merge_csr(const K* __restrict__ sorted, int64_t E, int64_t N, int shift,
+                          int64_t* __restrict__ start) {
+    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (j > N) return;
+    start[j] = j == N ? E : lower_bound(sorted, E, (K)((K)j << shift));
+}
+
+// Dead halos leave the neighbour scan: rank -1.
+__global__ void merge_live_rank(int64_t N, const uint8_t* __restrict__ state,
+                                int32_t* __restrict__ prank) {
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < N && state[p] != 1) prank[p] = -1;
 }
 
 // dV[j] = halo j's caps summed in the reference's order (entries sorted by key; one thread
@@ -447,13 +471,15 @@ extern "C" hnt_status hnt_merge_catalog(hnt_ctx* ctx, const float* records, int6
     HNT_TRY(reserve(ctx, B.prank, (size_t)N * 4));
     int32_t* idx = (int32_t*)B.cidx.p;
     int32_t* desc = pb;  // free perm buffer
+    int cbits = 1;
+    while (((int64_t)1 << cbits) < ncell) ++cbits;
     hipLaunchKernelGGL(merge_iota, dim3(nblk(N)), dim3(MB), 0, st, desc, N, 1);
     hipLaunchKernelGGL(merge_cell_keys, dim3(nblk(N)), dim3(MB), 0, st, records, N, nfields, G,
                        (const int32_t*)desc, ka);
     {
         size_t t = ctx->cub_tmp.bytes;
         HNT_HIP(hipcub::DeviceRadixSort::SortPairs(ctx->cub_tmp.p, t, ka, kb, desc, idx, (int)N,
-                                                   0, 32, st));
+                                                   0, cbits, st));
     }
     hipLaunchKernelGGL(merge_cell_start, dim3(nblk(ncell + 1)), dim3(MB), 0, st,
                        (const uint32_t*)kb, N, ncell, (int32_t*)B.cstart.p);
@@ -465,29 +491,31 @@ extern "C" hnt_status hnt_merge_catalog(hnt_ctx* ctx, const float* records, int6
     G.cell_start = (const int32_t*)B.cstart.p;
 
     // ---- exclusion: containment edges, CSR by contained halo, decision rounds ----
-    HNT_TRY(reserve(ctx, B.cnt, (size_t)(N + 1) * 8));
     HNT_TRY(reserve(ctx, B.off, (size_t)(N + 1) * 8));
-    int64_t* cnt = (int64_t*)B.cnt.p;
     int64_t* off = (int64_t*)B.off.p;
-    hipLaunchKernelGGL(merge_edges, dim3(nblk(N)), dim3(MB), 0, st, G, 0, cnt, nullptr, nullptr,
-                       nullptr);
-    size_t tmp3 = 0;
-    HNT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp3, cnt, off, (int)(N + 1), st));
-    if (tmp3 > ctx->cub_tmp.bytes) HNT_TRY(reserve(ctx, ctx->cub_tmp, tmp3));
-    HNT_HIP(hipMemsetAsync(cnt + N, 0, 8, st));
-    {
-        size_t t = ctx->cub_tmp.bytes;
-        HNT_HIP(hipcub::DeviceScan::ExclusiveSum(ctx->cub_tmp.p, t, cnt, off, (int)(N + 1), st));
-    }
+    HNT_TRY(reserve(ctx, ctx->small, 64));
+    unsigned long long* count = (unsigned long long*)ctx->small.p;
+    const auto scan_grid = [&](int w) { return dim3((unsigned)((N + MB / w - 1) / (MB / w))); };
+    // entries of a scan: room for one per halo (up to 2^24) or what an earlier call had; more are
+    // counted, and scanned again with room for all
+    const int64_t guess = std::min<int64_t>(N, 1 << 24);
+    int bits = 1;
+    while (((int64_t)1 << bits) < 2 * N) ++bits;  // of 2 N
     int64_t E = 0;
-    HNT_HIP(hipMemcpyAsync(&E, off + N, 8, hipMemcpyDeviceToHost, st));
-    HNT_HIP(hipStreamSynchronize(st));
-    HNT_REQUIRE(E < (1LL << 31), "hnt_merge_catalog: %lld containment pairs", (long long)E);
-    const size_t ebytes = (size_t)std::max<int64_t>(E, 1) * 4;
-    HNT_TRY(reserve(ctx, B.e1, ebytes));
-    HNT_TRY(reserve(ctx, B.e2, ebytes));
-    HNT_TRY(reserve(ctx, B.e3, ebytes));
-    HNT_TRY(reserve(ctx, B.e4, ebytes));
+    for (int64_t want = std::max<int64_t>(guess, (int64_t)(B.e4.bytes / 4));;) {
+        HNT_TRY(reserve(ctx, B.e1, (size_t)want * 4));
+        HNT_TRY(reserve(ctx, B.e2, (size_t)want * 4));
+        HNT_TRY(reserve(ctx, B.e3, (size_t)want * 4));
+        HNT_TRY(reserve(ctx, B.e4, (size_t)want * 4));
+        HNT_HIP(hipMemsetAsync(count, 0, 8, st));
+        ScanOut o{want, count, (int32_t*)B.e1.p, (int32_t*)B.e2.p, nullptr, nullptr, bits, 0};
+        hipLaunchKernelGGL(merge_scan<false>, scan_grid(EDGE_W), dim3(MB), 0, st, G, o);
+        HNT_HIP(hipMemcpyAsync(&E, count, 8, hipMemcpyDeviceToHost, st));
+        HNT_HIP(hipStreamSynchronize(st));
+        HNT_REQUIRE(E < (1LL << 31), "hnt_merge_catalog: %lld containment pairs", (long long)E);
+        if (E <= want) break;
+        want = E;
+    }
     HNT_TRY(reserve(ctx, B.state, (size_t)N));
     HNT_TRY(reserve(ctx, B.instart, (size_t)(N + 1) * 8));
     uint8_t* state = (uint8_t*)B.state.p;
@@ -495,32 +523,32 @@ extern "C" hnt_status hnt_merge_catalog(hnt_ctx* ctx, const float* records, int6
     int64_t* in_start = (int64_t*)B.instart.p;
     int32_t* in_src = (int32_t*)B.e3.p;
     if (E > 0) {
-        hipLaunchKernelGGL(merge_edges, dim3(nblk(N)), dim3(MB), 0, st, G, 1, nullptr,
-                           (const int64_t*)off, (int32_t*)B.e1.p, (int32_t*)B.e2.p);
         size_t t = 0;
         HNT_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, t, (int32_t*)nullptr,
                                                    (int32_t*)nullptr, (int32_t*)nullptr,
-                                                   (int32_t*)nullptr, (int)E, 0, 32, st));
+                                                   (int32_t*)nullptr, (int)E, 0, bits, st));
         if (t > ctx->cub_tmp.bytes) HNT_TRY(reserve(ctx, ctx->cub_tmp, t));
         t = ctx->cub_tmp.bytes;
         // keys: contained halo, values: container
         HNT_HIP(hipcub::DeviceRadixSort::SortPairs(ctx->cub_tmp.p, t, (int32_t*)B.e2.p,
                                                    (int32_t*)B.e4.p, (int32_t*)B.e1.p, in_src,
-                                                   (int)E, 0, 32, st));
+                                                   (int)E, 0, bits, st));
         hipLaunchKernelGGL(merge_csr<int32_t>, dim3(nblk(N + 1)), dim3(MB), 0, st,
                            (const int32_t*)B.e4.p, E, N, 0, in_start);
     } else {
         HNT_HIP(hipMemsetAsync(in_start, 0, (size_t)(N + 1) * 8, st));
     }
-    HNT_TRY(reserve(ctx, ctx->small, 64));
-    unsigned long long* und = (unsigned long long*)ctx->small.p;
-    for (int round = 0;; ++round) {
-        HNT_REQUIRE(round <= N, "hnt_merge_catalog: exclusion did not settle");
-        HNT_HIP(hipMemsetAsync(und, 0, 8, st));
-        hipLaunchKernelGGL(merge_round, dim3(nblk(N)), dim3(MB), 0, st, N,
-                           (const int64_t*)in_start, (const int32_t*)in_src, state, und);
+    // four rounds per look at the count of undecided halos (a round without any costs a few
+    // microseconds, a look some sixty)
+    constexpr int ROUNDS = 4;
+    for (int64_t round = 0;; round += ROUNDS) {
+        HNT_REQUIRE(round <= N + ROUNDS, "hnt_merge_catalog: exclusion did not settle");
+        HNT_HIP(hipMemsetAsync(count, 0, 8 * ROUNDS, st));
+        for (int u = 0; u < ROUNDS; ++u)
+            hipLaunchKernelGGL(merge_round, dim3(nblk(N)), dim3(MB), 0, st, N,
+                               round == 0 && u == 0, (const int64_t*)in_start, (const int32_t*)in_src, state, count + u);
         unsigned long long left = 0;
-        HNT_HIP(hipMemcpyAsync(&left, und, 8, hipMemcpyDeviceToHost, st));
+        HNT_HIP(hipMemcpyAsync(&left, count + ROUNDS - 1, 8, hipMemcpyDeviceToHost, st));
         HNT_HIP(hipStreamSynchronize(st));
         if (left == 0) break;
     }
@@ -529,38 +557,39 @@ extern "C" hnt_status hnt_merge_catalog(hnt_ctx* ctx, const float* records, int6
     HNT_TRY(reserve(ctx, B.dv, (size_t)N * 8));
     double* dV = (double*)B.dv.p;
     if (volume_reduction) {
-        hipLaunchKernelGGL(merge_pairs, dim3(nblk(N)), dim3(MB), 0, st, G, 0,
-                           (const uint8_t*)state, fortran_ties, cnt, nullptr, nullptr, nullptr);
-        HNT_HIP(hipMemsetAsync(cnt + N, 0, 8, st));
-        {
-            size_t t = ctx->cub_tmp.bytes;
-            HNT_HIP(hipcub::DeviceScan::ExclusiveSum(ctx->cub_tmp.p, t, cnt, off, (int)(N + 1),
-                                                     st));
+        hipLaunchKernelGGL(merge_live_rank, dim3(nblk(N)), dim3(MB), 0, st, N,
+                           (const uint8_t*)state, (int32_t*)B.prank.p);
+        int64_t P = 0;  // cap entries, two per overlapping pair
+        uint64_t *pk0 = nullptr, *pk1 = nullptr;
+        double *pv0 = nullptr, *pv1 = nullptr;
+        for (int64_t want = std::max<int64_t>(guess, (int64_t)(B.pv.bytes / 32));;) {
+            HNT_TRY(reserve(ctx, B.pk, (size_t)want * 32));
+            HNT_TRY(reserve(ctx, B.pv, (size_t)want * 32));
+            pk0 = (uint64_t*)B.pk.p;
+            pk1 = pk0 + 2 * want;
+            pv0 = (double*)B.pv.p;
+            pv1 = pv0 + 2 * want;
+            HNT_HIP(hipMemsetAsync(count, 0, 8, st));
+            ScanOut o{want, count, nullptr, nullptr, pk0, pv0, bits, fortran_ties};
+            hipLaunchKernelGGL(merge_scan<true>, scan_grid(PAIR_W), dim3(MB), 0, st, G, o);
+            HNT_HIP(hipMemcpyAsync(&P, count, 8, hipMemcpyDeviceToHost, st));
+            HNT_HIP(hipStreamSynchronize(st));
+            P *= 2;
+            HNT_REQUIRE(P < (1LL << 31), "hnt_merge_catalog: %lld cap entries (2 per overlapping "
+                        "pair)", (long long)P);
+            if (P <= 2 * want) break;
+            want = P / 2;
         }
-        int64_t P = 0;
-        HNT_HIP(hipMemcpyAsync(&P, off + N, 8, hipMemcpyDeviceToHost, st));
-        HNT_HIP(hipStreamSynchronize(st));
-        HNT_REQUIRE(P < (1LL << 31), "hnt_merge_catalog: %lld cap entries (2 per overlapping "
-                    "pair)", (long long)P);
         if (P > 0) {
-            HNT_TRY(reserve(ctx, B.pk, (size_t)P * 8 * 2));
-            HNT_TRY(reserve(ctx, B.pv, (size_t)P * 8 * 2));
-            uint64_t* pk0 = (uint64_t*)B.pk.p;
-            uint64_t* pk1 = pk0 + P;
-            double* pv0 = (double*)B.pv.p;
-            double* pv1 = pv0 + P;
-            hipLaunchKernelGGL(merge_pairs, dim3(nblk(N)), dim3(MB), 0, st, G, 1,
-                               (const uint8_t*)state, fortran_ties, nullptr,
-                               (const int64_t*)off, pk0, pv0);
             size_t t = 0;
             HNT_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, t, pk0, pk1, pv0, pv1, (int)P, 0,
-                                                       64, st));
+                                                       2 * bits - 1, st));
             if (t > ctx->cub_tmp.bytes) HNT_TRY(reserve(ctx, ctx->cub_tmp, t));
             t = ctx->cub_tmp.bytes;
             HNT_HIP(hipcub::DeviceRadixSort::SortPairs(ctx->cub_tmp.p, t, pk0, pk1, pv0, pv1,
-                                                       (int)P, 0, 64, st));
+                                                       (int)P, 0, 2 * bits - 1, st));
             hipLaunchKernelGGL(merge_csr<uint64_t>, dim3(nblk(N + 1)), dim3(MB), 0, st,
-                               (const uint64_t*)pk1, P, N, 32, in_start);
+                               (const uint64_t*)pk1, P, N, bits, in_start);
             hipLaunchKernelGGL(merge_incoming, dim3(nblk(N)), dim3(MB), 0, st,
                                (const double*)pv1, (const int64_t*)in_start, N, dV);
         } else {
