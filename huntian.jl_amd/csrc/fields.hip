@@ -301,9 +301,25 @@ __device__ __forceinline__ void stencil(int g, int block, int M, float w[4], int
 // mod1(start_a + l, N)), computed once per call: Catmull-Rom weights w[a * nmesh + l] and
 // coarse indices idx[a * nmesh + l].  Every row of the tile shares the x stencils, every
 // plane the y ones.
+// For fs_tricubic_runs (nprod != 0) also the 64 products ((wx wy) wz) of every position
+// (qx, qy, qz) in a coarse cell, i.e. of the tile's first block^3 cells, [4 z + y][x] each: entry
+// qx + block (qy + block qz) of wp.
 __global__ void fs_tricubic_axes(int M, int N, int block, int i0, int j0, int k0, int nmesh,
-                                 float4* __restrict__ w, int4* __restrict__ idx) {
+                                 float4* __restrict__ w, int4* __restrict__ idx, int nprod,
+                                 float4* __restrict__ wp) {
     const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (t < nprod) {
+        const int b = t & 3, c = (t >> 2) & 3, q = t >> 4, m = block - 1;
+        const int qz = q / (block * block), qy = (q / block) & m;
+        float wx[4], wy[4], wz[4];
+        int ii[4];
+        stencil(mod1(i0 + (q & m), N), block, M, wx, ii);
+        stencil(mod1(j0 + qy, N), block, M, wy, ii);
+        stencil(mod1(k0 + qz, N), block, M, wz, ii);
+        const float y = b == 0 ? wy[0] : b == 1 ? wy[1] : b == 2 ? wy[2] : wy[3];
+        const float z = c == 0 ? wz[0] : c == 1 ? wz[1] : c == 2 ? wz[2] : wz[3];
+        wp[t] = make_float4(wx[0] * y * z, wx[1] * y * z, wx[2] * y * z, wx[3] * y * z);
+    }
     if (t >= 3 * nmesh) return;
     const int axis = t / nmesh, l = t - axis * nmesh;
     const int s = axis == 0 ? i0 : (axis == 1 ? j0 : k0);
@@ -435,6 +451,68 @@ __global__ __launch_bounds__(FT) void fs_tricubic_tab(const float* __restrict__ 
                     val += w.w * cv[c][b][3];
                 }
             o[li] = val;
+        }
+    }
+}
+
+// fs_tricubic_tab's values for tiles of several coarse cells a side: the lanes of a wavefront are
+// runs of `block` cells with the same x indices, in rows of one position (qy, qz) in their
+// coarse cells, so that all lanes need the same 64 products at every step.  They come by scalar
+// loads and enter the multiplications from scalar registers; a lane keeps its run's 64 coarse
+// values.  What bounds it is the 64 multiplications and 64 additions of a cell (54 us for
+// 256^3 cells; fused forms would round otherwise): 92 us, with the products in LDS, read by 16
+// loads of 16 bytes per cell, 151 us.
+// q0: first cell whose x indices differ from the cell before; cxn: runs per row.
+template <bool VEC>
+__global__ __launch_bounds__(FT) void fs_tricubic_runs(const float* __restrict__ coarse, int M,
+                                                       int nmesh, int lgb, int q0, int cxn, int cyn,
+                                                       const int4* __restrict__ si,
+                                                       const float* wp, float* __restrict__ out) {
+    const int block = 1 << lgb, m = block - 1;
+    const int qy = (int)blockIdx.y & m, qz = (int)blockIdx.y >> lgb;
+    const int item = (int)(blockIdx.x * FT + threadIdx.x);
+    const int cx = item % cxn, r = item / cxn, jy = r % cyn, jz = r / cyn;
+    const int lj = qy + (jy << lgb), lk = qz + (jz << lgb);
+    const int base = (cx << lgb) + q0 - (q0 > 0 ? block : 0);
+    if (jz >= cyn || lj >= nmesh || lk >= nmesh || base >= nmesh) return;
+    float cv[4][4][4];
+    {
+        const int4 xs4 = si[max(base, 0)], ys4 = si[nmesh + lj], zs4 = si[2 * nmesh + lk];
+        const int xs[4] = {xs4.x, xs4.y, xs4.z, xs4.w}, ys[4] = {ys4.x, ys4.y, ys4.z, ys4.w},
+                  zs[4] = {zs4.x, zs4.y, zs4.z, zs4.w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const float* cy = coarse + (int64_t)M * M * zs[c] + (int64_t)M * ys[b];
+#pragma unroll
+                for (int a = 0; a < 4; ++a) cv[c][b][a] = cy[xs[a]];
+            }
+    }
+    float* o = out + ((int64_t)lk * nmesh + lj) * nmesh + base;
+    const __attribute__((address_space(4))) float* wq =
+        (const __attribute__((address_space(4))) float*)wp + (((int)blockIdx.y << lgb) << 6);
+    for (int t = 0; t < block; t += 4) {
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const __attribute__((address_space(4))) float* w = wq + (((q0 + t + u) & m) << 6);
+            float val = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) val += w[16 * c + 4 * b + a] * cv[c][b][a];
+            v[u] = val;
+        }
+        if (VEC) {  // every four cells inside or outside together
+            if (base + t >= 0 && base + t < nmesh)
+                *reinterpret_cast<float4*>(o + t) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (base + t + u >= 0 && base + t + u < nmesh) o[t + u] = v[u];
         }
     }
 }
@@ -775,12 +853,37 @@ extern "C" hnt_status hnt_interpolate_to_tile(hnt_ctx* ctx, const float* coarse,
     HNT_REQUIRE(std::max(i0, std::max(j0, k0)) + nmesh < (1LL << 31),
                 "hnt_interpolate_to_tile: tile start beyond Int32");
     // the three axes' stencils: 3 nmesh x (float4 weights + int4 indices)
-    HNT_TRY(reserve(ctx, ctx->fs_tab, (size_t)3 * nmesh * 32));
+    const bool pow2 = (block & (block - 1)) == 0 && block <= TRI_MAXB && nmesh >= block;
+    // runs of cells, unless a position (qy, qz) has too few of them to fill a wavefront or the
+    // tile is too small to pay for the products (us per call, table in LDS / runs: 64 cells a
+    // side in blocks of 8 39 / 42, 96 in 16 53 / 42, 128 in 32 96 / 79, 256 in 32 272 / 145)
+    const bool runs = pow2 && ctx->tricubic_tab && block >= 4 && nmesh >= 4 * block && nmesh >= 96;
+    const size_t nprod = runs ? (size_t)block * block * block * 16 : 0;  // float4
+    HNT_TRY(reserve(ctx, ctx->fs_tab, (size_t)3 * nmesh * 32 + nprod * sizeof(float4)));
     float4* sw = (float4*)ctx->fs_tab.p;
     int4* si = (int4*)(sw + 3 * (size_t)nmesh);
-    hipLaunchKernelGGL(fs_tricubic_axes, dim3((unsigned)((3 * nmesh + 255) / 256)), dim3(256), 0,
-                       ctx->stream, M, N, block, (int)i0, (int)j0, (int)k0, nmesh, sw, si);
-    if ((block & (block - 1)) == 0 && block <= TRI_MAXB && nmesh >= block && ctx->tricubic_tab)
+    float4* wp = (float4*)(si + 3 * (size_t)nmesh);
+    const size_t nsetup = std::max((size_t)3 * nmesh, nprod);
+    hipLaunchKernelGGL(fs_tricubic_axes, dim3((unsigned)((nsetup + 255) / 256)), dim3(256), 0,
+                       ctx->stream, M, N, block, (int)i0, (int)j0, (int)k0, nmesh, sw, si,
+                       (int)nprod, wp);
+    if (runs) {
+        int lgb = 0;
+        while ((1 << lgb) < block) ++lgb;
+        // global cell g (1-based) starts a run where g - 1/2 passes an odd multiple of block / 2
+        const int q0 = (int)(((1 - i0 - block / 2) % block + block) % block);
+        const int cyn = (nmesh + block - 1) / block;
+        const int cxn = (nmesh - q0 + block - 1) / block + (q0 > 0 ? 1 : 0);
+        const dim3 grid((unsigned)(((int64_t)cxn * cyn * cyn + FT - 1) / FT),
+                        (unsigned)(block * block));
+        const bool vec = q0 % 4 == 0 && nmesh % 4 == 0 && ((uintptr_t)tile & 15) == 0;
+        const auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(FT), 0, ctx->stream, coarse, M, nmesh, lgb, q0, cxn,
+                               cyn, (const int4*)si, (const float*)wp, tile);
+        };
+        if (vec) launch(fs_tricubic_runs<true>);
+        else launch(fs_tricubic_runs<false>);
+    } else if (pow2 && ctx->tricubic_tab)
         hipLaunchKernelGGL(fs_tricubic_tab, dim3(grid_rows((int64_t)nmesh * nmesh)), dim3(FT), 0,
                            ctx->stream, coarse, M, nmesh, block, (const float4*)sw,
                            (const int4*)si, tile);
