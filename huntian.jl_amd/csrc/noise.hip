@@ -52,8 +52,10 @@ __device__ inline void gauss_pair(uint64_t seed, uint64_t pair, double& g1, doub
     const double u2 = ((double)(r1 >> 11) + 1.0) * 1.1102230246251565e-16;
     const double r = sqrt(-2.0 * log(u1));
     const double th = 6.283185307179586 * u2;  // 2 pi (Float64) times u2
-    g1 = r * cos(th);
-    g2 = r * sin(th);
+    double sn, cs;
+    sincos(th, &sn, &cs);
+    g1 = r * cs;
+    g2 = r * sn;
 }
 
 // The Gaussian of global cell idx0 (0-based linear index), in FP64.
@@ -64,63 +66,79 @@ __device__ inline double gauss_at(uint64_t seed, uint64_t idx0) {
 }
 
 // mod1(x, N) - 1: the 0-based periodic index of 1-based x
-__device__ __forceinline__ int64_t wrap0(int64_t x, int64_t N) {
+inline int64_t wrap0(int64_t x, int64_t N) {
     const int64_t m = (x - 1) % N;
     return m < 0 ? m + N : m;
 }
 
-// Cells (li, lj, lk) of a side^3 region whose first cell is global (i0, j0, k0) (1-based,
-// wrapped): out = Float32(gauss), or with coarse, Float32(gauss) - coarse[block cell] * inv.
+// Cells (li, lj, lk) of a side^3 region whose first cell is global (i0, j0, k0) (0-based, wrapped):
+// out = Float32(gauss), or with coarse, Float32(gauss) - coarse[block cell] * inv.
 // For an even N the two cells of a pair are neighbours along x in one row (the parity of a
 // cell's global index is that of its wrapped x index), so one thread takes a pair: the
 // region's row is cut into pairs from the parity of its first cell, a lone cell at either
-// end.  An odd N takes one cell per thread.
-__device__ __forceinline__ void region_store(int64_t e, int64_t gi, int64_t gj, int64_t gk,
-                                             double g, const float* __restrict__ coarse, int M,
-                                             int64_t block, float inv, float* __restrict__ out) {
+// end.  An odd N takes one cell per thread.  Workgroups (x, lk) cover plane lk.  T: unsigned, as
+// wide as the grid's coordinates ask for (64-bit divisions, twelve per pair, took as long as
+// the Gaussians: 256^3 cells 180 -> 103 us).
+template <class T>
+__device__ __forceinline__ void region_store(int64_t e, T ci, T cj, T ck, double g,
+                                             const float* __restrict__ coarse, int M, float inv,
+                                             float* __restrict__ out) {
     const float fine = (float)g;
     if (!coarse) {
         out[e] = fine;
         return;
     }
-    const int64_t ci = gi / block, cj = gj / block, ck = gk / block;
     const float mean = coarse[ci + (int64_t)M * (cj + (int64_t)M * ck)] * inv;
     out[e] = fine - mean;
 }
 
-__global__ __launch_bounds__(256) void region_noise_kernel(uint64_t seed, int64_t N,
-                                                           int64_t i0, int64_t j0, int64_t k0,
+template <class T>
+__global__ __launch_bounds__(256) void region_noise_kernel(uint64_t seed, T N, T i0, T j0, T k0,
                                                            int side, const float* __restrict__ coarse,
-                                                           int M, int64_t block, float inv,
+                                                           int M, T block, float inv,
                                                            float* __restrict__ out) {
     const bool paired = (N & 1) == 0;
-    const int64_t gi0 = wrap0(i0, N);                  // global x of the row's first cell
-    const int shift = paired ? (int)(gi0 & 1) : 0;     // 1: the first cell ends a pair
-    const int per_row = paired ? (side + shift + 1) / 2 : side;
-    const int64_t rows = (int64_t)side * side, total = rows * per_row;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int t = (int)(e % per_row);
-        const int64_t row = e / per_row;
-        const int lj = (int)(row % side), lk = (int)(row / side);
-        const int64_t gj = wrap0(j0 + lj, N), gk = wrap0(k0 + lk, N);
-        const int64_t obase = (int64_t)side * row;
-        if (!paired) {
-            const int64_t gi = wrap0(i0 + t, N);
-            region_store(obase + t, gi, gj, gk,
-                         gauss_at(seed, (uint64_t)(gi + gj * N + gk * N * N)), coarse, M,
-                         block, inv, out);
-            continue;
-        }
-        const int la = 2 * t - shift;  // the pair's even-index cell, maybe outside the row
-        const int64_t gi = wrap0(i0 + (la >= 0 ? la : la + 1), N) - (la >= 0 ? 0 : 1);
-        const uint64_t idx0 = (uint64_t)(gi + gj * N + gk * N * N);  // even
-        double g1, g2;
-        gauss_pair(seed, idx0 >> 1, g1, g2);
-        if (la >= 0) region_store(obase + la, gi, gj, gk, g1, coarse, M, block, inv, out);
-        if (la + 1 < side)
-            region_store(obase + la + 1, gi + 1, gj, gk, g2, coarse, M, block, inv, out);
+    const int shift = paired ? (int)(i0 & 1) : 0;     // 1: the first cell ends a pair
+    const unsigned per_row = paired ? (side + shift + 1) / 2 : side;
+    const unsigned e = blockIdx.x * 256 + threadIdx.x;
+    const unsigned lj = e / per_row, t = e - lj * per_row, lk = blockIdx.y;
+    if (lj >= (unsigned)side) return;
+    auto wrap = [&](T g) { return g < N ? g : g % N; };
+    const T gj = wrap(j0 + lj), gk = wrap(k0 + lk);
+    const T cj = coarse ? gj / block : 0, ck = coarse ? gk / block : 0;
+    const int64_t obase = (int64_t)side * (lj + (int64_t)side * lk);
+    const uint64_t row0 = (uint64_t)N * (gj + (uint64_t)N * gk);
+    if (!paired) {
+        const T gi = wrap(i0 + t);
+        region_store<T>(obase + t, coarse ? gi / block : 0, cj, ck, gauss_at(seed, gi + row0), coarse,
+                        M, inv, out);
+        return;
     }
+    const int la = 2 * (int)t - shift;  // the pair's even-index cell, maybe outside the row
+    const T gi = wrap(i0 - shift + 2 * (T)t);  // even
+    double g1, g2;
+    gauss_pair(seed, (gi + row0) >> 1, g1, g2);
+    T ci = coarse ? gi / block : 0;
+    if (la >= 0) region_store<T>(obase + la, ci, cj, ck, g1, coarse, M, inv, out);
+    if (coarse && gi + 1 - ci * block == block) ++ci;
+    if (la + 1 < side) region_store<T>(obase + la + 1, ci, cj, ck, g2, coarse, M, inv, out);
+}
+
+// i0, j0, k0: 1-based, not wrapped
+void launch_region_noise(hipStream_t st, uint64_t seed, int64_t N, int64_t i0, int64_t j0, int64_t k0,
+                         int side, const float* coarse, int M, int64_t block, float inv, float* out) {
+    const int64_t gi = wrap0(i0, N), gj = wrap0(j0, N), gk = wrap0(k0, N);
+    const int shift = (N & 1) == 0 ? (int)(gi & 1) : 0;
+    const int64_t per_row = (N & 1) == 0 ? (side + shift + 1) / 2 : side;
+    const dim3 grid((unsigned)((per_row * side + 255) / 256), (unsigned)side);
+    if (N < (1LL << 31))  // with the region's side, at most 16384
+        hipLaunchKernelGGL(region_noise_kernel<uint32_t>, grid, dim3(256), 0, st, seed, (uint32_t)N,
+                           (uint32_t)gi, (uint32_t)gj, (uint32_t)gk, side, coarse, M,
+                           (uint32_t)block, inv, out);
+    else
+        hipLaunchKernelGGL(region_noise_kernel<uint64_t>, grid, dim3(256), 0, st, seed, (uint64_t)N,
+                           (uint64_t)gi, (uint64_t)gj, (uint64_t)gk, side, coarse, M,
+                           (uint64_t)block, inv, out);
 }
 
 // Coarse cell (I, J, K): the FP64 sum of its block^3 fine Gaussians in the reference's loop
@@ -176,9 +194,7 @@ extern "C" hnt_status hnt_tile_noise(hnt_ctx* ctx, int32_t it, int32_t jt, int32
     const int64_t i0 = (int64_t)(it - 1) * nsub + 1 - nbuff;
     const int64_t j0 = (int64_t)(jt - 1) * nsub + 1 - nbuff;
     const int64_t k0 = (int64_t)(kt - 1) * nsub + 1 - nbuff;
-    const int64_t total = (int64_t)nmesh * nmesh * nmesh;
-    hipLaunchKernelGGL(region_noise_kernel, dim3(grid_for(total)), dim3(256), 0, ctx->stream,
-                       seed, N, i0, j0, k0, nmesh, nullptr, 1, (int64_t)1, 0.0f, out);
+    launch_region_noise(ctx->stream, seed, N, i0, j0, k0, nmesh, nullptr, 1, 1, 0.0f, out);
     HNT_HIP(hipGetLastError());
     return finish_call(ctx, "hnt_tile_noise");
 }
@@ -220,9 +236,7 @@ extern "C" hnt_status hnt_extended_residual(hnt_ctx* ctx, int32_t it, int32_t jt
     // Float32(1 / sqrt(Float64(block)^3)): the block mean from the coarse block sum
     const double b = (double)block;
     const float inv = (float)(1.0 / sqrt(b * b * b));
-    const int64_t total = (int64_t)side * side * side;
-    hipLaunchKernelGGL(region_noise_kernel, dim3(grid_for(total)), dim3(256), 0, ctx->stream,
-                       seed, N, i0, j0, k0, side, coarse, M, block, inv, out);
+    launch_region_noise(ctx->stream, seed, N, i0, j0, k0, side, coarse, M, block, inv, out);
     HNT_HIP(hipGetLastError());
     return finish_call(ctx, "hnt_extended_residual");
 }
