@@ -17,8 +17,8 @@
 //             (DPP lane shifts along i, then three rows), and the k direction keeps the last
 //             planes' maxima in registers (no LDS).  One barrier per plane keeps the
 //             workgroup's wavefronts on the same plane, so the cache lines they share (halo
-//             columns and rows) come from HBM once: 1.45x the field bytes at 1024^3, against
-//             2.1x for free-running wavefronts.  A peak is written to the claim array
+//             columns and rows) come from HBM once: with 32 planes 1.45x the field bytes at
+//             1024^3, against 2.1x for free-running wavefronts.  A peak is written to the claim array
 //             (filter index; 255 = none) by the one lane owning the cell; a per-lane bitset
 //             marks cells masked or already taken by an earlier filter.
 //  pf_count   per 4096-cell chunk of the claim array (inner-cube scan order k, j, i): peaks
@@ -34,8 +34,13 @@
 namespace {
 
 // pf_mark geometry: a wavefront owns OI = 62 consecutive i (its 64 lanes load i-1 .. i+62),
-// TJ rows of j and TK planes of k; a workgroup is WI x WJ wavefronts along i and j.
-constexpr int OI = 62, TJ = 8, TK = 32, WI = 4, WJ = 2;
+// TJ rows of j and TK planes of k; a workgroup is WI x WJ wavefronts along i and j.  TK: two halo
+// planes for every TK, but a workgroup's planes follow one another, so few of them are what
+// fills the CUs (the inner 144^3 of a 192^3 tile is 45 workgroups at 32 planes).  16 filters at
+// 192^3, 16 fields at 512^3, 24 filters at 1024^3, ms: 32 planes 0.95, 1.84, 19.5; 16 0.55, 1.77,
+// 20.8; 8 0.24, 1.70, 18.5; 4 0.28, 1.74, 34.0 (its one claim word does not need the rotation:
+// the compiler unrolls into 255 registers).
+constexpr int OI = 62, TJ = 8, TK = 8, WI = 4, WJ = 2;
 constexpr int PF_THREADS = 64 * WI * WJ;
 constexpr int CHUNK = 4096;
 constexpr uint8_t NONE = 255, BLOCKED = 254;  // claim of a cell: filter index, or these
@@ -432,12 +437,12 @@ __global__ __launch_bounds__(256) void fb_window(const float2* __restrict__ spec
                                                  float2* __restrict__ out, int n, double dk,
                                                  double Rf, int wsmooth, float inv_n3) {
     const int nk = n / 2 + 1, nyq = n / 2;
-    const int64_t total = (int64_t)nk * (nyq + 1) * (nyq + 1);
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        const int ix = (int)(e % nk);
-        const int64_t rem = e / nk;
-        const int ay = (int)(rem % (nyq + 1)), az = (int)(rem / (nyq + 1));  // |ky|, |kz| / dk
+    // 32 bits: the transforms here are of less than 2^31 reals
+    const unsigned total = (unsigned)nk * (nyq + 1) * (nyq + 1);
+    for (unsigned e = blockIdx.x * blockDim.x + threadIdx.x; e < total; e += gridDim.x * blockDim.x) {
+        const unsigned rem = e / (unsigned)nk;
+        const int ix = (int)(e - rem * nk);
+        const int az = (int)(rem / (unsigned)(nyq + 1)), ay = (int)(rem - az * (nyq + 1));  // |k| / dk
         const double kx = (double)ix * dk, ky = (double)ay * dk, kz = (double)az * dk;
         const double k2 = kx * kx + ky * ky + kz * kz;
         float w32 = 1.0f;
