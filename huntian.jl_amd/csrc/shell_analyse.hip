@@ -2168,6 +2168,13 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
         const int64_t h0 = bricks ? 0 : g0, hn = bricks ? ngroups : ng;
         const int shares = (int)std::min<int64_t>(8, std::max<int64_t>(1, 2048 / hn));
         SAArgs A1 = A;
+        const bool beyond = bricks && TT.near_shells < A.NS - 1;  // shells no brick holds
+        const auto far = [&](int f) {
+            hipLaunchKernelGGL(gather_far_kernel,
+                               dim3((unsigned)(std::max(8, ctx->num_cus / 8 * 8) * FAR_WG)), dim3(FAR_T),
+                               0, st, A, B, (const int64_t*)W.far.p, (const int32_t*)far_cnt,
+                               TT.near_shells, f);
+        };
         if (bricks) {
             const dim3 grid((unsigned)((maxbr + 511) / 512 * 512));
             if (vec4)
@@ -2176,10 +2183,8 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
             else
                 hipLaunchKernelGGL(gather_bricks_kernel<false>, grid, dim3(BR_T), sizeof(BrickLds), st,
                                    A1, B, K);
-            for (int f = 0; f < BLK_FIELDS; ++f)
-                hipLaunchKernelGGL(gather_far_kernel, dim3((unsigned)(std::max(8, ctx->num_cus / 8 * 8) * FAR_WG)),
-                                   dim3(FAR_T), 0, st, A1, B, (const int64_t*)W.far.p,
-                                   (const int32_t*)far_cnt, TT.near_shells, f);
+            if (beyond)
+                for (int f : {0, 2, 3, 4}) far(f);
             A1.slot = far_slot;
         }
         hipLaunchKernelGGL(gather_blocks_kernel, dim3((unsigned)(8 * ((hn * shares + 7) / 8))),
@@ -2194,6 +2199,7 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
             hipLaunchKernelGGL(walk_rows_kernel<16>, rows(16), dim3(64), 0, st, A2, B, s0, nsl, ws);
         else
             hipLaunchKernelGGL(walk_rows_kernel<4>, rows(4), dim3(64), 0, st, A2, B, s0, nsl, ws);
+        if (beyond) far(1);
         hipLaunchKernelGGL(finish_rows_kernel, rows(4), dim3(64), 0, st, A2, B, s0, nsl,
                            (const WalkState*)ws, half, hcnt);
         if (A.variant != HNT_VARIANT_B)
