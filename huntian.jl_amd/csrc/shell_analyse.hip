@@ -1872,6 +1872,7 @@ __device__ __forceinline__ int isqrt_floor(int v) {
     return h;
 }
 
+// Workgroup y takes its share of a group's 64 peaks, one halo after another.
 __global__ __launch_bounds__(64) void paint_mask_kernel(SAArgs a, int64_t G8) {
     const int64_t g = (int64_t)(blockIdx.x & 7) * G8 + (blockIdx.x >> 3);
     if (g >= a.ngroups) return;
@@ -1884,7 +1885,8 @@ __global__ __launch_bounds__(64) void paint_mask_kernel(SAArgs a, int64_t G8) {
     const int mi = myr2 >= 0 ? T.pi[myp] : 0, mj = myr2 >= 0 ? T.pj[myp] : 0;
     const int mk = myr2 >= 0 ? T.pk[myp] : 0;
     const int n = T.n, nb = a.nbuff;
-    for (int k = 0; k < 64; ++k) {
+    const int share = 64 / (int)gridDim.y, k0 = (int)blockIdx.y * share;
+    for (int k = k0; k < k0 + share; ++k) {
         const int r2 = __builtin_amdgcn_readlane(myr2, k);
         if (r2 < 0) continue;
         const int ci = __builtin_amdgcn_readlane(mi, k), cj = __builtin_amdgcn_readlane(mj, k);
@@ -1962,7 +1964,9 @@ void launch_repacks(hipStream_t st, const std::vector<RepackJob>& jobs) {
 void launch_paint(hipStream_t st, const LaunchDesc& d) {
     if (!d.A.paint) return;
     const int64_t G8 = (d.A.ngroups + 7) / 8;
-    hipLaunchKernelGGL(paint_mask_kernel, dim3((unsigned)(8 * G8)), dim3(64), 0, st, d.A, G8);
+    // groups that would not fill the CUs are shared out (128^3 tile 64 -> 16 us)
+    const unsigned shares = d.A.ngroups < 2048 ? 16 : 1;
+    hipLaunchKernelGGL(paint_mask_kernel, dim3((unsigned)(8 * G8), shares), dim3(64), 0, st, d.A, G8);
 }
 
 void launch_main(hipStream_t st, const LaunchDesc& d) {
@@ -2005,7 +2009,10 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     }
     int32_t* stops = (int32_t*)W.stops.p;
     int32_t* cross = (int32_t*)W.cross.p;
-    const bool few = ntot < (1 << 17);
+    // few: the time is the deepest peaks' chains, not the work (sixteen lanes per peak, fields side by
+    // side, the first order throughout; ms with and without: 60 k peaks 1.92 / 2.33, 130 k
+    // 2.36 / 2.67, 180 k 3.71 / 3.95, 300 k 4.42 / 4.51)
+    const bool few = ntot < (1 << 18);
     const auto row_grid = [](int64_t groups, int w) { return (unsigned)(8 * ((groups * w + 7) / 8)); };
     const uint32_t* cell8 = (const uint32_t*)TT.cell8.p;
     if (few)
@@ -2029,44 +2036,37 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     size_t tmp = 0;
     HNT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, cnt, off, (int)ntot, st));
     HNT_TRY(reserve(ctx, W.cub_tmp, tmp > 0 ? tmp : 16));
-    // bricks of 16^3 cells with their peaks, and the peaks they do not gather entirely, unless
-    // the tiles hold only a few peaks per brick (staging a brick costs about as much as the
-    // direct gather of five peaks)
+    // bricks of 16^3 cells with their peaks, and the peaks they do not gather entirely (also where
+    // a brick has one peak: against the gather from the fields, 1000 peaks of a 256^3 tile take
+    // 1.09 instead of 1.22 ms, 16 000 of a 512^3 tile 5.0 instead of 8.5)
     int64_t vol = 0;
     for (int t = 0; t < ntiles; ++t) {
         const int64_t b = (W.tile_host[t].n + BR_CORE - 1) / BR_CORE;
         vol += batches[t].npeaks > 0 ? b * b * b : 0;
     }
-    const bool bricks = ntot >= 4 * vol;
     const int64_t maxbr = std::min(vol, ntot);
-    int32_t* far_slot = (int32_t*)W.slots.p;
-    int32_t* far_cnt = nullptr;
-    BrickArgs K{};
-    if (bricks) {
-        HNT_TRY(reserve(ctx, W.brick, (size_t)(maxbr + 1) * 8 + (size_t)maxbr * 4 + 8 + (size_t)ntiles * 4));
-        HNT_TRY(reserve(ctx, W.far, (size_t)ntot * 8));
-        HNT_TRY(reserve(ctx, W.slots3, (size_t)ngroups * 64 * 4));
-        int64_t* bstart = (int64_t*)W.brick.p;
-        int32_t* btile = (int32_t*)(bstart + maxbr + 1);
-        int32_t* bcount = btile + maxbr;
-        int32_t* fcnt = bcount + 1;
-        far_slot = (int32_t*)W.slots3.p;
-        hipLaunchKernelGGL(brick_head_kernel, dim3(nb), dim3(256), 0, st, keys, ntot, 11 + 3 * 4, cnt);
-        size_t tb = W.cub_tmp.bytes;
-        HNT_HIP(hipcub::DeviceScan::ExclusiveSum(W.cub_tmp.p, tb, cnt, off, (int)ntot, st));
-        hipLaunchKernelGGL(brick_list_kernel, dim3(nb), dim3(256), 0, st, keys, cnt,
-                           (const int64_t*)off, ntot, bstart, btile, bcount);
-        far_cnt = fcnt;
-        hipLaunchKernelGGL(fill_i32, dim3((unsigned)((ntiles + 256) / 256)), dim3(256), 0, st, fcnt,
-                           (int64_t)ntiles + 1, 0);
-        hipLaunchKernelGGL(fill_i32, dim3((unsigned)((ngroups * 64 + 255) / 256)), dim3(256), 0, st,
-                           far_slot, ngroups * 64, -1);
-        hipLaunchKernelGGL(far_list_kernel, dim3(nb), dim3(256), 0, st, A.tiles, keys, vals, stops,
-                           A.rad, ntot, TT.near_shells, (const int64_t*)W.tilemeta.p + ntiles, fcnt,
-                           far_slot, (int64_t*)W.far.p);
-        K = BrickArgs{bstart, btile, bcount, vals, (const uint2*)TT.brick_tab.p,
-                      (const uint8_t*)TT.near_order.p, TT.near_cells, TT.near_shells};
-    }
+    HNT_TRY(reserve(ctx, W.brick, (size_t)(maxbr + 1) * 8 + (size_t)maxbr * 4 + 8 + (size_t)ntiles * 4));
+    HNT_TRY(reserve(ctx, W.far, (size_t)ntot * 8));
+    HNT_TRY(reserve(ctx, W.slots3, (size_t)ngroups * 64 * 4));
+    int64_t* bstart = (int64_t*)W.brick.p;
+    int32_t* btile = (int32_t*)(bstart + maxbr + 1);
+    int32_t* bcount = btile + maxbr;
+    int32_t* fcnt = bcount + 1;
+    int32_t* far_slot = (int32_t*)W.slots3.p;
+    hipLaunchKernelGGL(brick_head_kernel, dim3(nb), dim3(256), 0, st, keys, ntot, 11 + 3 * 4, cnt);
+    size_t tb = W.cub_tmp.bytes;
+    HNT_HIP(hipcub::DeviceScan::ExclusiveSum(W.cub_tmp.p, tb, cnt, off, (int)ntot, st));
+    hipLaunchKernelGGL(brick_list_kernel, dim3(nb), dim3(256), 0, st, keys, cnt,
+                       (const int64_t*)off, ntot, bstart, btile, bcount);
+    hipLaunchKernelGGL(fill_i32, dim3((unsigned)((ntiles + 256) / 256)), dim3(256), 0, st, fcnt,
+                       (int64_t)ntiles + 1, 0);
+    hipLaunchKernelGGL(fill_i32, dim3((unsigned)((ngroups * 64 + 255) / 256)), dim3(256), 0, st,
+                       far_slot, ngroups * 64, -1);
+    hipLaunchKernelGGL(far_list_kernel, dim3(nb), dim3(256), 0, st, A.tiles, keys, vals, stops,
+                       A.rad, ntot, TT.near_shells, (const int64_t*)W.tilemeta.p + ntiles, fcnt,
+                       far_slot, (int64_t*)W.far.p);
+    BrickArgs K{bstart, btile, bcount, vals, (const uint2*)TT.brick_tab.p,
+                  (const uint8_t*)TT.near_order.p, TT.near_cells, TT.near_shells};
     // profile offsets in the first order
     hipLaunchKernelGGL(block_count_kernel, dim3(nb), dim3(256), 0, st, vals, stops, ntot, cnt);
     tmp = W.cub_tmp.bytes;
@@ -2146,13 +2146,11 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
         for (const float* f : {T.delta, T.etax, T.etay, T.etaz})
             vec4 = vec4 && ((uintptr_t)f & 15) == 0;
     }
-    if (bricks) {
-        // more than the default 64 KB of LDS per workgroup
-        HNT_HIP(hipFuncSetAttribute((const void*)gather_bricks_kernel<true>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(BrickLds)));
-        HNT_HIP(hipFuncSetAttribute((const void*)gather_bricks_kernel<false>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(BrickLds)));
-    }
+    // more than the default 64 KB of LDS per workgroup
+    HNT_HIP(hipFuncSetAttribute((const void*)gather_bricks_kernel<true>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(BrickLds)));
+    HNT_HIP(hipFuncSetAttribute((const void*)gather_bricks_kernel<false>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(BrickLds)));
     const size_t lds = (size_t)nbmax * 8 + (size_t)(nbmax + 1) * 4;
     HNT_TRY(reserve(ctx, W.walk, (size_t)ngroups * 64 * (sizeof(WalkState) + 4) + 4));
     WalkState* ws = (WalkState*)W.walk.p;
@@ -2164,35 +2162,38 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
         const int64_t s0 = slot_of(pos[c]) & ~(int64_t)63;
         const int64_t s1 = c + 2 == pos.size() ? ngroups * 64 : slot_of(pos[c + 1]);
         const int64_t g0 = s0 >> 6, ng = (s1 - s0 + 63) >> 6;
-        // (the far peaks' slots are in no chunk's order: every launch looks through all of them)
-        const int64_t h0 = bricks ? 0 : g0, hn = bricks ? ngroups : ng;
-        const int shares = (int)std::min<int64_t>(8, std::max<int64_t>(1, 2048 / hn));
-        SAArgs A1 = A;
-        const bool beyond = bricks && TT.near_shells < A.NS - 1;  // shells no brick holds
+        const bool beyond = TT.near_shells < A.NS - 1;  // shells no brick holds
         const auto far = [&](int f) {
             hipLaunchKernelGGL(gather_far_kernel,
-                               dim3((unsigned)(std::max(8, ctx->num_cus / 8 * 8) * FAR_WG)), dim3(FAR_T),
-                               0, st, A, B, (const int64_t*)W.far.p, (const int32_t*)far_cnt,
-                               TT.near_shells, f);
+                               dim3((unsigned)(std::max(8, ctx->num_cus / 8 * 8) * FAR_WG),
+                                    f < 0 ? BLK_FIELDS - 1 : 1), dim3(FAR_T), 0, st, A, B,
+                               (const int64_t*)W.far.p, (const int32_t*)fcnt, TT.near_shells, f);
         };
-        if (bricks) {
-            const dim3 grid((unsigned)((maxbr + 511) / 512 * 512));
-            if (vec4)
-                hipLaunchKernelGGL(gather_bricks_kernel<true>, grid, dim3(BR_T), sizeof(BrickLds), st,
-                                   A1, B, K);
-            else
-                hipLaunchKernelGGL(gather_bricks_kernel<false>, grid, dim3(BR_T), sizeof(BrickLds), st,
-                                   A1, B, K);
-            if (beyond)
-                for (int f : {0, 2, 3, 4}) far(f);
-            A1.slot = far_slot;
-        }
-        hipLaunchKernelGGL(gather_blocks_kernel, dim3((unsigned)(8 * ((hn * shares + 7) / 8))),
-                           dim3(256), lds, st, A1, B, h0, hn, shares);
-        hipLaunchKernelGGL(block_fbar_kernel, dim3((unsigned)ng), dim3(64), 0, st, A, B, g0);
+        // a workgroup per field where that still leaves every one a CU (40^3 tile 48 -> 36 us;
+        // at 128^3, 216 bricks, listing the items five times costs more: 208 -> 276)
+        const dim3 grid((unsigned)((maxbr + 511) / 512 * 512),
+                        maxbr * BLK_FIELDS <= ctx->num_cus ? BLK_FIELDS : 1);
+        if (vec4)
+            hipLaunchKernelGGL(gather_bricks_kernel<true>, grid, dim3(BR_T), sizeof(BrickLds), st, A, B, K);
+        else
+            hipLaunchKernelGGL(gather_bricks_kernel<false>, grid, dim3(BR_T), sizeof(BrickLds), st, A, B, K);
+        if (beyond && few) far(-1);
+        else if (beyond)
+            for (int f : {0, 2, 3, 4}) far(f);
+        // the peaks whose balls leave the grid are in no chunk's order: every launch looks
+        // through all of them
+        SAArgs A1 = A;
+        A1.slot = far_slot;
+        const int shares = (int)std::min<int64_t>(8, std::max<int64_t>(1, 2048 / ngroups));
+        hipLaunchKernelGGL(gather_blocks_kernel, dim3((unsigned)(8 * ((ngroups * shares + 7) / 8))),
+                           dim3(256), lds, st, A1, B, (int64_t)0, ngroups, shares);
         SAArgs A2 = A;
         A2.slot = slot2;
         const int64_t nsl = ng * 64;
+        if (few)
+            hipLaunchKernelGGL(fbar_rows_kernel, dim3(row_grid(ng, 16)), dim3(64), 0, st, A, B, s0, nsl);
+        else
+            hipLaunchKernelGGL(block_fbar_kernel, dim3((unsigned)ng), dim3(64), 0, st, A, B, g0);
         hipLaunchKernelGGL(fill_i32, dim3(1), dim3(64), 0, st, hcnt, (int64_t)1, 0);
         const auto rows = [&](int w) { return dim3(row_grid(ng, w)); };
         if (few)

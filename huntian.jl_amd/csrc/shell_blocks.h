@@ -252,7 +252,8 @@ template <bool VEC4>
 __global__ __launch_bounds__(BR_T) void gather_bricks_kernel(SAArgs a, BlockArgs B, BrickArgs K) {
     extern __shared__ char lds_raw[];
     BrickLds& L = *reinterpret_cast<BrickLds*>(lds_raw);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // runs of 64 bricks (a 64^3 brick) per XCD in turn
     const int j = (int)(blockIdx.x >> 3);
     const int k = (((j >> 6) << 3) + (int)(blockIdx.x & 7)) * 64 + (j & 63);
@@ -269,6 +270,9 @@ __global__ __launch_bounds__(BR_T) void gather_bricks_kernel(SAArgs a, BlockArgs
               oz = ((T.pk[p0] - 1) & ~(BR_CORE - 1)) - BR_H;
     const int nsh = K.nsh;  // shells 1 .. nsh
     constexpr int NW = BR_PK / 64;
+    // lane i's: the i-th shell by falling number of cells (read one by one as they are wanted, each
+    // was a trip to the cache in a chain of 55)
+    const int order = lane < nsh ? (int)K.order[lane] : 0;
     for (int s = tid; s <= nsh + 1; s += BR_T) {
         // table start of shell s, s = nsh + 1 the end of the last one
         L.sstart[s] = (uint16_t)(s < 1 ? 0 : s <= nsh ? a.shell_start[s - 1] : K.ncell);
@@ -314,7 +318,7 @@ __global__ __launch_bounds__(BR_T) void gather_bricks_kernel(SAArgs a, BlockArgs
         np = L.np;
         if (wave < NW)
             for (int i = 0; i < nsh; ++i) {
-                const uint64_t m = __ballot(tid < np && stop >= (int)K.order[i]);
+                const uint64_t m = __ballot(tid < np && stop >= __builtin_amdgcn_readlane(order, i));
                 if (lane == 0) L.mask[i * NW + wave] = m;
             }
         __syncthreads();
@@ -343,14 +347,16 @@ __global__ __launch_bounds__(BR_T) void gather_bricks_kernel(SAArgs a, BlockArgs
             const uint64_t m = L.mask[e];
             if ((m >> lane) & 1ull) {
                 const int r = __popcll(m & ((1ull << lane) - 1ull));
-                L.item[L.pre[e] + r] = (uint16_t)(((int)K.order[e / NW] << 8) | ((e & (NW - 1)) * 64 + lane));
+                L.item[L.pre[e] + r] = (uint16_t)((__builtin_amdgcn_readlane(order, e / NW) << 8) | ((e & (NW - 1)) * 64 + lane));
             }
         }
         const int tot = L.tot;
         // the transposed delta first, then delta, psi_1 xyz through the other table
         const float* const src[BLK_FIELDS] = {T.delta, T.delta, T.etax, T.etay, T.etaz};
-        for (int f = 0; f < BLK_FIELDS && tot > 0; ++f) {
-            if (f < 2)
+        // (all of them, or the one of workgroup y)
+        const int f0 = gridDim.y > 1 ? (int)blockIdx.y : 0, f1 = gridDim.y > 1 ? f0 + 1 : BLK_FIELDS;
+        for (int f = f0; f < f1 && tot > 0; ++f) {
+            if (f < 2 || f == f0)
                 for (int c = tid; c < K.ncell; c += BR_T) L.tab[c] = K.tab[(f == 0 ? K.ncell : 0) + c];
             if (f == 0) stage_box<VEC4>(L.box, src[f], T.n, oz, ox, oy, T.s1, T.s2);
             else stage_box<VEC4>(L.box, src[f], T.n, ox, oy, oz, T.s1, T.s2);
@@ -431,7 +437,9 @@ constexpr int FAR_T = 256, FAR_WG = 4;  // workgroups per CU
 __global__ __launch_bounds__(FAR_T) void gather_far_kernel(SAArgs a, BlockArgs B,
                                                            const int64_t* __restrict__ far,
                                                            const int32_t* __restrict__ count,
-                                                           int nsh, int f) {
+                                                           int nsh, int f0) {
+    // one field, or (f0 < 0) delta and psi_1 by workgroup y
+    const int f = f0 >= 0 ? f0 : blockIdx.y == 0 ? 0 : (int)blockIdx.y + 1;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     constexpr int NWV = FAR_T / 64;
@@ -505,6 +513,7 @@ __global__ __launch_bounds__(FAR_T) void gather_far_kernel(SAArgs a, BlockArgs B
 }
 
 // ------------------------------------------------------------------ gather from the fields
+// The peaks whose balls leave the grid, read from the fields as they are.
 struct BlockSums {
     double F, G0, G1, G2, H0, H1, H2;
     double S0, S1, S2, R00, R01, R02, R10, R11, R12, R20, R21, R22;
@@ -747,14 +756,6 @@ __global__ __launch_bounds__(64) void block_fbar_kernel(SAArgs a, BlockArgs B, i
     }
 }
 
-// v of lane S of each four lanes.
-template <int S>
-__device__ __forceinline__ double quad_of(double v) {
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), S * 0x55, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), S * 0x55, 0xf, 0xf, true);
-    return __hiloint2double(hi, lo);
-}
-
 // Rows of a launch: slots [slot0, slot0 + nslot), NR = 64 / W per wavefront, contiguous runs per
 // XCD.  False: this wavefront has no slot.
 template <int W>
@@ -763,6 +764,64 @@ __device__ __forceinline__ bool row_slot(int64_t nslot, int64_t& first) {
     const int64_t per = (int64_t)gridDim.x >> 3;
     first = ((int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3)) * NR;
     return first < nslot;
+}
+
+// block_fbar_kernel for few peaks, where its time is the deepest peak's chain of loads: sixteen
+// lanes per peak, a shell each; the recurrence then runs over their quotients in order, every lane
+// alike.  128^3 tile 67 -> 50 us.
+__global__ __launch_bounds__(64) void fbar_rows_kernel(SAArgs a, BlockArgs B, int64_t slot0,
+                                                       int64_t nslot) {
+    constexpr int W = 16;
+    const int lane = threadIdx.x, l = lane & (W - 1), row0 = lane & ~(W - 1);
+    int64_t first;
+    if (!row_slot<W>(nslot, first)) return;
+    const TileDev& T = a.tiles[a.gtile[(slot0 + first) >> 6]];
+    const int p = a.slot[slot0 + first + lane / W];
+    int64_t eb = -1;
+    int stop = -1, ci = 1, cj = 1, ck = 1;
+    bool out = false;
+    if (p >= 0) {
+        eb = B.base[T.base + p] - B.e0;
+        if (eb >= 0 && eb < B.ne) {
+            stop = B.stop[T.base + p];
+            ci = T.pi[p];
+            cj = T.pj[p];
+            ck = T.pk[p];
+            out = ball_outside(T, ci, cj, ck, (int)a.rad[stop]);
+        }
+    }
+    double* fb = B.fb + (stop >= 0 ? eb : 0) * BLK;
+    double Fprev = 0.0, dFbarp = 0.0, Fn = stop >= max(l, 1) ? *entry_of(B, eb, l) : 0.0;
+    for (int sb = 0; __ballot(sb <= stop) != 0ull; sb += W) {
+        const int s = sb + l;
+        const double F = Fn;
+        if (s + W <= stop) Fn = *entry_of(B, eb, s + W);
+        double dF = 0.0, Fb = 0.0;
+        if (s >= 2 && s <= stop) {
+            const int nin = shell_cells_in(a, T, s, ci, cj, ck, out);
+            dF = nin > 0 ? F / (double)nin : 0.0;
+        }
+        if (sb == 0) Fprev = dFbarp = __shfl(F, row0 + 1);
+        for (int j = 0; j < W; ++j) {
+            const double dFbar = __shfl(dF, row0 + j);
+            const int t = sb + j;
+            if (t >= 2 && t <= stop) {
+                const double rad3p = cube(a.rad[t - 1]), rad3 = cube(a.rad[t]);
+                Fprev = (rad3p * Fprev + 0.5 * (dFbarp + dFbar) * (rad3 - rad3p)) / rad3;
+                dFbarp = dFbar;
+            }
+            if (j == l) Fb = Fprev;
+        }
+        if (s <= (stop | 3) && stop >= 0) fb[s] = Fb;
+    }
+}
+
+// v of lane S of each four lanes.
+template <int S>
+__device__ __forceinline__ double quad_of(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), S * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), S * 0x55, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
 }
 
 // The sum of f over shell s around cell (ci, cj, ck), in the reference's order, and the number
