@@ -34,19 +34,25 @@
 namespace {
 
 // pf_mark geometry: a wavefront owns OI = 62 consecutive i (its 64 lanes load i-1 .. i+62),
-// TJ rows of j and TK planes of k; a workgroup is WI x WJ wavefronts along i and j.  TK: two halo
-// planes for every TK, but a workgroup's planes follow one another, so few of them are what
-// fills the CUs (the inner 144^3 of a 192^3 tile is 45 workgroups at 32 planes).  16 filters at
-// 192^3, 16 fields at 512^3, 24 filters at 1024^3, ms: 32 planes 0.95, 1.84, 19.5; 16 0.55, 1.77,
-// 20.8; 8 0.24, 1.70, 18.5; 4 0.28, 1.74, 34.0 (its one claim word does not need the rotation:
-// the compiler unrolls into 255 registers).
-constexpr int OI = 62, TJ = 8, TK = 8, WI = 4, WJ = 2;
+// TJ rows of j and TK planes of k; a workgroup is WI x WJ wavefronts along i and j.  There are two
+// halo planes for every TK, but a workgroup's planes follow one another, so few of them are
+// what fills the CUs (the inner 144^3 of a 192^3 tile is 45 workgroups at 32 planes): TK_FEW.
+// 16 filters at 192^3, 16 fields at 512^3, 24 filters at 1024^3, one by one, ms: 32 planes 0.95,
+// 1.84, 19.5; 16 0.55, 1.77, 20.8; 8 0.24, 1.70, 18.5; 4 0.28, 1.74, 34.0 (its one claim word
+// does not need the rotation: the compiler unrolls into 255 registers).  TK_MANY for many large
+// fields in one launch, whose workgroups are fields apart by the time a neighbour's planes are
+// wanted again, which then come from HBM: hnt_peak_find, ms with 8 / 32 planes, of 4 fields of
+// 1024^3 (17 GB) 5.3 / 5.9, 16 of 640^3 (17 GB) 4.10 / 4.16, 16 of 768^3 (29 GB) 6.8 / 6.6, 24 of
+// 1024^3 (103 GB) 26.8 / 23.2.
+constexpr int OI = 62, TJ = 8, WI = 4, WJ = 2, TK_FEW = 8, TK_MANY = 32;
+constexpr int64_t MANY_BYTES = 24LL << 30;
 constexpr int PF_THREADS = 64 * WI * WJ;
 constexpr int CHUNK = 4096;
 constexpr uint8_t NONE = 255, BLOCKED = 254;  // claim of a cell: filter index, or these
 // Word 3 of a raw (stride 0) buffer resource on CDNA: 32-bit data format, no swizzle.
 constexpr int BUF_DWORD3 = 0x00020000;
-static_assert(TJ * 4 == 32 && TK % 4 == 0, "claim bits: one 32-bit word per 4 planes of TJ=8");
+static_assert(TJ * 4 == 32 && TK_FEW % 4 == 0 && TK_MANY % 4 == 0,
+              "claim bits: one 32-bit word per 4 planes of TJ=8");
 
 // Left and right neighbour of a lane's value within the wavefront (lanes 0 and 63 receive
 // values that are never used: they are halo columns).
@@ -73,7 +79,7 @@ __device__ __forceinline__ float from_lane_above(float v) {
 // nothing, so no wavefront waits on a load in the claim path.  A claimed cell also records
 // its field value in cellval (and, with celld2, the value of lapfields[f]), indexed like
 // the claim array.
-template <bool TILE>
+template <bool TILE, int TK>
 __global__ __launch_bounds__(PF_THREADS) void pf_mark(const float* const* __restrict__ fields,
                                                const float* __restrict__ fcrit, int nfilt,
                                                int fbase, int n, int nbuff, int fside,
@@ -561,8 +567,8 @@ hnt_status compact_claims(hnt_ctx* ctx, const char* what, int n, int nbuff, int 
     return HNT_OK;
 }
 
-dim3 mark_grid(int m) {
-    return dim3((m + OI * WI - 1) / (OI * WI), (m + TJ * WJ - 1) / (TJ * WJ), (m + TK - 1) / TK);
+dim3 mark_grid(int m, int tk) {
+    return dim3((m + OI * WI - 1) / (OI * WI), (m + TJ * WJ - 1) / (TJ * WJ), (m + tk - 1) / tk);
 }
 
 }  // namespace
@@ -600,9 +606,13 @@ extern "C" hnt_status hnt_peak_find(hnt_ctx* ctx, const float* const* smoothed,
 
     stage_begin(ctx, HNT_STAGE_PF_MARK);
     HNT_HIP(hipMemsetAsync(ctx->claim.p, NONE, (size_t)ncell, st));
-    hipLaunchKernelGGL(pf_mark<false>, mark_grid(m), dim3(PF_THREADS), 0, st, dfields,
-                       (const float*)ctx->fcrit.p, nfilt, 0, n, nbuff, n, 0, (const int8_t*)mask, 0,
-                       (uint8_t*)ctx->claim.p, nullptr, nullptr, nullptr, nullptr);
+    const auto mark = [&](auto kernel, int tk) {
+        hipLaunchKernelGGL(kernel, mark_grid(m, tk), dim3(PF_THREADS), 0, st, dfields,
+                           (const float*)ctx->fcrit.p, nfilt, 0, n, nbuff, n, 0, (const int8_t*)mask, 0,
+                           (uint8_t*)ctx->claim.p, nullptr, nullptr, nullptr, nullptr);
+    };
+    if ((int64_t)n * n * n * 4 * nfilt > MANY_BYTES) mark(pf_mark<false, TK_MANY>, TK_MANY);
+    else mark(pf_mark<false, TK_FEW>, TK_FEW);
     stage_end(ctx, HNT_STAGE_PF_MARK);
     return compact_claims(ctx, "hnt_peak_find", n, nbuff, nfilt, tmp_bytes, dfields, nullptr,
                           nullptr, mask, out, nullptr);
@@ -657,8 +667,8 @@ extern "C" hnt_status hnt_peak_find_tile(hnt_ctx* ctx, const float* delta, int32
                 "fft = 0)", n);
     if (own) HNT_TRY(reserve(ctx, ctx->fb_wtab, sizeof(float) * (size_t)nwtab));
     // taken bits carried from filter to filter (one word per lane column, 8 rows, 4 planes)
-    const dim3 mg = mark_grid(m);
-    const int NJ = (int)mg.y * WJ, NKG = (int)mg.z * (TK / 4);
+    const dim3 mg = mark_grid(m, TK_FEW);
+    const int NJ = (int)mg.y * WJ, NKG = (int)mg.z * (TK_FEW / 4);
     const int64_t ntw = (int64_t)m * NJ * NKG;
     HNT_TRY(reserve(ctx, ctx->fb_taken, sizeof(uint32_t) * (size_t)ntw));
     hipfftHandle r2c = nullptr, c2r = nullptr;
@@ -747,7 +757,7 @@ extern "C" hnt_status hnt_peak_find_tile(hnt_ctx* ctx, const float* delta, int32
         }
         stage_end(ctx, HNT_STAGE_PF_SMOOTH);
         stage_begin(ctx, HNT_STAGE_PF_MARK);
-        hipLaunchKernelGGL(pf_mark<true>, mg, dim3(PF_THREADS), 0, st, dptrs,
+        hipLaunchKernelGGL((pf_mark<true, TK_FEW>), mg, dim3(PF_THREADS), 0, st, dptrs,
                            (const float*)ctx->fcrit.p + f, 1, f, n, nbuff, fside, fshift,
                            (const int8_t*)mask, 1, (uint8_t*)ctx->claim.p,
                            (float*)ctx->fb_val.p, lap ? dptrs + 1 : nullptr,
