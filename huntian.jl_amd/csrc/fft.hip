@@ -513,19 +513,23 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_r2c(
 // 8-byte aligned.
 __device__ __forceinline__ void store_rows(const float2* buf, int LS, int G, int row0, int nrows,
                                            int s, int n, float scale, int mode, float coef,
-                                           int pairs, float* __restrict__ out) {
+                                           int pairs, const float* __restrict__ base,
+                                           float* __restrict__ out) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     if (pairs) {
         const int np = (n / 2 + 63) >> 6;  // pieces of 64 pairs per row
         float2 old[ROW_U];
         if (mode != 0) {
+            const float* __restrict__ from = mode == 2 ? base : out;
 #pragma unroll
             for (int u = 0; u < ROW_U; ++u) {
                 const int piece = wave + u * (SMALL_T / 64), g = piece / np;
                 const int j = ((piece - g * np) << 6) + lane;
                 if (g < G && row0 + g < nrows && j < n / 2)
-                    old[u] = *reinterpret_cast<const float2*>(out + (int64_t)(row0 + g) * n + 2 * j);
+                    old[u] = *reinterpret_cast<const float2*>(from + (int64_t)(row0 + g) * n + 2 * j);
+                if (mode == 2)
+                    old[u] = make_float2((old[u].x * old[u].x) * 0.5f, (old[u].y * old[u].y) * 0.5f);
             }
         }
 #pragma unroll
@@ -551,19 +555,21 @@ __device__ __forceinline__ void store_rows(const float2* buf, int LS, int G, int
             const float v = ((xx & 1) ? zz.y : zz.x) * scale;
             const int64_t o = (int64_t)row * n + xo;
             if (mode == 0) out[o] = v;
-            else out[o] = out[o] - (v * v) * coef;
+            else if (mode == 1) out[o] = out[o] - (v * v) * coef;
+            else out[o] = (base[o] * base[o]) * 0.5f - (v * v) * coef;
         }
     }
 }
 
 // Inverse x pass: rows (s + jy, s + jz), jy, jz < n, of the half spectrum to real rows, of
 // which x in [s, s + n) is kept: out[(jy + n jz) n + x - s] = scale * x (mode 0), or
-// s2 -= (scale * x)^2 * coef (mode 1).  X[0] and X[M] enter through their real parts.
+// s2 -= (scale * x)^2 * coef (mode 1), or s2 = base^2 / 2 - (scale * x)^2 * coef (mode 2).  X[0] and X[M] enter through their real parts.
 // Z[k] = (X[k] + conj X[M-k]) + i (X[k] - conj X[M-k]) W_L^-k, z = IFFT_M(Z), x[2m] = Re z[m],
 // x[2m + 1] = Im z[m].
 __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r(
     const float2* __restrict__ spec, int lgM, int lgG, int s, int n, float scale, int mode,
-    float coef, int pairs, float* __restrict__ out, const float2* __restrict__ WM,
+    float coef, int pairs, const float* __restrict__ base, float* __restrict__ out,
+    const float2* __restrict__ WM,
     const float2* __restrict__ WL) {
     __shared__ float2 buf[SMALL_LDS];
     __shared__ float2 tw[ROW_TW];
@@ -627,7 +633,7 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r(
     }
     __syncthreads();
     stockham<true, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, tw);
-    store_rows(buf, LS, G, row0, nrows, s, n, scale, mode, coef, pairs, out);
+    store_rows(buf, LS, G, row0, nrows, s, n, scale, mode, coef, pairs, base, out);
 }
 
 // fft_rows_c2r for L = 512 (M = 256, 16 rows per workgroup; 0.50 -> 0.25 ms for 512^3 with the
@@ -639,7 +645,7 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r(
 template <int LGM>
 __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r_direct(
     const float2* __restrict__ spec, int s, int n, float scale, int mode, float coef, int pairs,
-    float* __restrict__ out, const float2* __restrict__ WM, const float2* __restrict__ WL) {
+    const float* __restrict__ base, float* __restrict__ out, const float2* __restrict__ WM, const float2* __restrict__ WL) {
     constexpr int lgM = LGM, M = 1 << LGM, G = SMALL_DATA / M, L = 2 * M, P = fft_pitch(L);
     constexpr int Q = M / 128, LGQ = LGM - 7;  // 1 KB chunks per row
     static_assert(LGM >= 8 && LGM <= 10 && G * padded_len(M) <= SMALL_LDS, "row shapes");
@@ -700,7 +706,7 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r_direct(
     }
     __syncthreads();
     stockham<true, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, tw);
-    store_rows(buf, LS, G, row0, nrows, s, n, scale, mode, coef, pairs, out);
+    store_rows(buf, LS, G, row0, nrows, s, n, scale, mode, coef, pairs, base, out);
 }
 
 // sqrt P per (ix, |iy|, |iz|) of the transfer: the (L/2 + 1)^3 table the inverse z pass reads
@@ -858,7 +864,8 @@ hnt_status fft_forward(hnt_ctx* ctx, const float* f, int w, int L, float2* spec)
 }
 
 hnt_status fft_inverse(hnt_ctx* ctx, const float2* spec, float2* work, int L, int s, int n,
-                       const FftOp& op, float scale, int mode, float coef, float* out) {
+                       const FftOp& op, float scale, int mode, float coef, float* out,
+                       const float* base) {
     hipStream_t st = ctx->stream;
     const int M = L / 2, nk = M + 1;
     const float2 *WL, *WM;
@@ -876,28 +883,28 @@ hnt_status fft_inverse(hnt_ctx* ctx, const float2* spec, float2* work, int L, in
                       s + n, none, WL, ctx->fft_direct != 0);
     const int lgG = rows_lgG(M);
     const int64_t rows = (int64_t)n * n;
-    const int pairs = s % 2 == 0 && n % 2 == 0 && ((uintptr_t)out & 7) == 0;
+    const int pairs = s % 2 == 0 && n % 2 == 0 && (((uintptr_t)out | (uintptr_t)base) & 7) == 0;
     if (ctx->fft_direct && L == 512 && lgG == 4) {
         hipLaunchKernelGGL(fft_rows_c2r_direct<8>, dim3((unsigned)((rows + 15) >> 4)),
                            dim3(SMALL_T), 0, st, (const float2*)work, s, n, scale, mode, coef,
-                           pairs, out, WM, WL);
+                           pairs, base, out, WM, WL);
         return HNT_OK;
     }
     if (ctx->fft_direct && L == 1024 && lgG == 3) {
         hipLaunchKernelGGL(fft_rows_c2r_direct<9>, dim3((unsigned)((rows + 7) >> 3)),
                            dim3(SMALL_T), 0, st, (const float2*)work, s, n, scale, mode, coef,
-                           pairs, out, WM, WL);
+                           pairs, base, out, WM, WL);
         return HNT_OK;
     }
     if (ctx->fft_direct && L == 2048 && lgG == 2) {
         hipLaunchKernelGGL(fft_rows_c2r_direct<10>, dim3((unsigned)((rows + 3) >> 2)),
                            dim3(SMALL_T), 0, st, (const float2*)work, s, n, scale, mode, coef,
-                           pairs, out, WM, WL);
+                           pairs, base, out, WM, WL);
         return HNT_OK;
     }
     hipLaunchKernelGGL(fft_rows_c2r, dim3((unsigned)((rows + (1 << lgG) - 1) >> lgG)),
                        dim3(SMALL_T), 0, st, (const float2*)work, ilog2(M), lgG, s, n, scale,
-                       mode, coef, pairs, out, WM, WL);
+                       mode, coef, pairs, base, out, WM, WL);
     return HNT_OK;
 }
 

@@ -204,9 +204,10 @@ hnt_status fft_twiddles(hnt_ctx* ctx, int L, const float2** out);
 // spec ((L/2+1) x L x L) = R2C of the w^3 field f zero-padded to L^3
 hnt_status fft_forward(hnt_ctx* ctx, const float* f, int w, int L, float2* spec);
 // out (n^3) = scale * C2R(op(spec)) cropped to [s, s + n)^3 (mode 0), or out -= (that)^2 * coef
-// (mode 1); work: a spectrum-sized scratch
+// (mode 1), or out = base^2 / 2 - (that)^2 * coef (mode 2, base n^3); work: a spectrum-sized scratch
 hnt_status fft_inverse(hnt_ctx* ctx, const float2* spec, float2* work, int L, int s, int n,
-                       const FftOp& op, float scale, int mode, float coef, float* out);
+                       const FftOp& op, float scale, int mode, float coef, float* out,
+                       const float* base = nullptr);
 hnt_status fft_amp_table(hnt_ctx* ctx, int L, double dk, const float* tab, int ntab,
                          float log_k_min, float d_log_k, float* amp);
 // reserve(), or a carve of `bytes` from `ar` when it is not NULL (HNT_ERR_CAPACITY if the
