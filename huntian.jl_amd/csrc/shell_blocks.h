@@ -12,8 +12,8 @@
 // them: no cell records are written.
 //
 // Measured against the lane-per-peak kernel with its records (same bits): shell analysis of the
-// 1024^3 tile 327 -> 225 ms, of the 512^3 tile 51.6 -> 27.3 ms, of a 128^3 tile 7.9 -> 1.38 ms, of a
-// 40^3 tile 1.33 -> 0.44 ms, of 24 tiles of 96^3 to 256^3 37.6 -> 21.6 ms.
+// 1024^3 tile 327 -> 211 ms, of the 512^3 tile 51.6 -> 25.8 ms, of a 128^3 tile 7.9 -> 1.10 ms, of a
+// 40^3 tile 1.33 -> 0.37 ms, of 24 tiles of 96^3 to 256^3 with their peak finding 37.6 -> 21.2 ms.
 //
 // A block's sums are five 128-byte lines side by side, one per field (delta, its transpose,
 // psi_1 xyz), four doubles per shell: {F, G0, G1, G2}, {H0, H1, H2, -}, {S, R0, R1, R2} x 3;
