@@ -220,6 +220,8 @@ hnt_status ensure_akk(hnt_ctx* ctx);
 hnt_status upload_tables_to(hnt_ctx* ctx, TablesDev& T, const hnt_shell_tables* t, Arena* ar);
 hnt_status upload_ctab_to(hnt_ctx* ctx, CTabDev& D, const hnt_ctab* c, Arena* ar);
 hnt_status ensure_akk_to(hnt_ctx* ctx, DevBuf& akk, Arena* ar);
+// Exclusive sums of n counts in 64 bits (shell_analyse.hip)
+hnt_status scan_counts(hnt_ctx* ctx, const int32_t* cnt, int64_t* off, int64_t n);
 // The fixed scratch of hnt_shell_analyse_noalloc: its device address on ctx's device,
 // looked up once per device (shell_analyse.hip)
 hnt_status noalloc_scratch_init(int device);

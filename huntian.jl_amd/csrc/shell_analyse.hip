@@ -1814,6 +1814,23 @@ __global__ __launch_bounds__(64) void shell_analyse_kernel(SAArgs a) {
 
 }  // namespace
 
+namespace hnt {
+
+// off[q] = cnt[0] + ... + cnt[q - 1], summed in 64 bits: the shell blocks of a call can pass
+// 2^31 (11.4 million peaks gathered to a hunt radius of 30), and a scan that takes its sums' type
+// from its input, as ExclusiveSum does, would wrap there.
+hnt_status scan_counts(hnt_ctx* ctx, const int32_t* cnt, int64_t* off, int64_t n) {
+    size_t tmp = 0;
+    HNT_HIP(hipcub::DeviceScan::ExclusiveScan(nullptr, tmp, cnt, off, hipcub::Sum(), (int64_t)0,
+                                              (int)n, ctx->stream));
+    HNT_TRY(reserve(ctx, ctx->cub_tmp, tmp > 0 ? tmp : 16));
+    HNT_HIP(hipcub::DeviceScan::ExclusiveScan(ctx->cub_tmp.p, tmp, cnt, off, hipcub::Sum(),
+                                              (int64_t)0, (int)n, ctx->stream));
+    return HNT_OK;
+}
+
+}  // namespace hnt
+
 using namespace hnt;
 
 namespace {
@@ -2033,9 +2050,6 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     int64_t* off = (int64_t*)W.boff.p;
     const int32_t* vals = (const int32_t*)W.vals_b.p;
     const uint64_t* keys = (const uint64_t*)W.keys_b.p;
-    size_t tmp = 0;
-    HNT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, cnt, off, (int)ntot, st));
-    HNT_TRY(reserve(ctx, W.cub_tmp, tmp > 0 ? tmp : 16));
     // bricks of 16^3 cells with their peaks, and the peaks they do not gather entirely (also where
     // a brick has one peak: against the gather from the fields, 1000 peaks of a 256^3 tile take
     // 1.09 instead of 1.22 ms, 16 000 of a 512^3 tile 5.0 instead of 8.5)
@@ -2054,8 +2068,7 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     int32_t* fcnt = bcount + 1;
     int32_t* far_slot = (int32_t*)W.slots3.p;
     hipLaunchKernelGGL(brick_head_kernel, dim3(nb), dim3(256), 0, st, keys, ntot, 11 + 3 * 4, cnt);
-    size_t tb = W.cub_tmp.bytes;
-    HNT_HIP(hipcub::DeviceScan::ExclusiveSum(W.cub_tmp.p, tb, cnt, off, (int)ntot, st));
+    HNT_TRY(scan_counts(ctx, cnt, off, ntot));
     hipLaunchKernelGGL(brick_list_kernel, dim3(nb), dim3(256), 0, st, keys, cnt,
                        (const int64_t*)off, ntot, bstart, btile, bcount);
     hipLaunchKernelGGL(fill_i32, dim3((unsigned)((ntiles + 256) / 256)), dim3(256), 0, st, fcnt,
@@ -2069,8 +2082,7 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
                   (const uint8_t*)TT.near_order.p, TT.near_cells, TT.near_shells};
     // profile offsets in the first order
     hipLaunchKernelGGL(block_count_kernel, dim3(nb), dim3(256), 0, st, vals, stops, ntot, cnt);
-    tmp = W.cub_tmp.bytes;
-    HNT_HIP(hipcub::DeviceScan::ExclusiveSum(W.cub_tmp.p, tmp, cnt, off, (int)ntot, st));
+    HNT_TRY(scan_counts(ctx, cnt, off, ntot));
     hipLaunchKernelGGL(block_base_kernel, dim3(nb), dim3(256), 0, st, vals, off, ntot,
                        (int64_t*)W.bbase.p);
     // profile space: every peak at its deepest if that is little (no word from the device
