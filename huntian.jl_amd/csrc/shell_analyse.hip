@@ -1717,8 +1717,7 @@ __device__ int crossing_stop(const SAArgs& a, double Rf, int scross) {
 // arithmetic as the gather, so each peak's exact gather extent.  Workgroup b takes group
 // (b % 8) * G8 + b / 8, G8 an eighth of the groups: each XCD walks its own contiguous eighth.
 __global__ __launch_bounds__(64) void crossing_kernel(SAArgs a, int64_t G8,
-                                                      int32_t* __restrict__ stop_out,
-                                                      int32_t* __restrict__ cross_out) {
+                                                      int32_t* __restrict__ stop_out) {
     const int64_t g = (int64_t)(blockIdx.x & 7) * G8 + (blockIdx.x >> 3);
     if (g >= a.ngroups) return;
     const TileDev& T = a.tiles[a.gtile[g]];
@@ -1758,7 +1757,6 @@ __global__ __launch_bounds__(64) void crossing_kernel(SAArgs a, int64_t G8,
     }
     if (!valid) return;
     stop_out[T.base + p] = crossing_stop(a, Rf, scross);
-    if (cross_out) cross_out[T.base + p] = scross;
 }
 
 #include "shell_blocks.h"
@@ -2004,12 +2002,15 @@ void launch_main(hipStream_t st, const LaunchDesc& d) {
 
 // The analysis by shell blocks, from the first order on: crossing pass, block offsets, the
 // radial logic's order, then per chunk of the schedule the gather, Fbar and the radial logic,
-// and the halos' mask.
+// and the halos' mask.  *lanes: the call is left, with its extents in W.stops, to the lane-per-peak
+// kernel, whose scratch does not grow with the peaks.  Nothing but schedule_extent is written before
+// that, nor before a buffer cannot be had (HNT_ERR_ALLOC).
 template <class OrderBy>
 hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT, int ntiles,
                           const hnt_batch* batches, hnt_results* results, int8_t* const* masks,
                           const std::vector<int64_t>& meta, int64_t ntot, int64_t ngroups,
-                          OrderBy&& order_by) {
+                          OrderBy&& order_by, bool* lanes) {
+    *lanes = false;
     hipStream_t st = ctx->stream;
     bool any_mask = false;
     for (int t = 0; t < ntiles; ++t) any_mask = any_mask || (masks && masks[t] && batches[t].npeaks);
@@ -2086,7 +2087,10 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     hipLaunchKernelGGL(block_base_kernel, dim3(nb), dim3(256), 0, st, vals, off, ntot,
                        (int64_t*)W.bbase.p);
     // profile space: every peak at its deepest if that is little (no word from the device
-    // needed), else what the scan found; at most kBlockBudget at a time
+    // needed), else what the scan found, in chunks of kBlockBudget and what is left of the brick in
+    // which a chunk ends.  A brick crowded so that this does not hold the profile to a quarter above
+    // the budget (it takes 80 k peaks of 650 blocks in a 64^3 brick, or many peaks per cell) is
+    // lane-per-peak work
     const int nbmax = (A.NS >> 2) + 1;
     constexpr int64_t kBlockBytes = BLK_DOUBLES * 8;
     constexpr int64_t kBlockBudget = ((int64_t)32 << 30) / kBlockBytes;
@@ -2122,6 +2126,11 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     }
     int64_t cap = 0;
     for (size_t c = 0; c + 1 < pos.size(); ++c) cap = std::max(cap, first[c + 1] - first[c]);
+    if (cap > kBlockBudget + kBlockBudget / 4) {
+        *lanes = true;
+        stage_end(ctx, HNT_STAGE_SA_CROSS);
+        return HNT_OK;
+    }
     HNT_TRY(reserve(ctx, W.prof, (size_t)cap * kBlockBytes));
     // the radial logic's order: like extents together (few peaks: the first order)
     int32_t* slot2 = (int32_t*)W.slots.p;
@@ -2314,22 +2323,13 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
                         params->precision == HNT_PREC_FP64 && ctx->gang == 1 && TT.blocks_ok &&
                         (int64_t)(tables->rmax + 1) * maxn * maxn < (1LL << 31);
 
-    // ---- repack every tile's fields into 32-byte cell records ----
-    if (!blocks) HNT_TRY(reserve_in(ctx, W.recs, (size_t)ncell * 32, W.arena));
     std::vector<TileDev>& TD = W.tile_host;
     TD.assign((size_t)ntiles, TileDev{});
-    std::vector<RepackJob> jobs;
     {
-        int64_t off = 0;
         for (int t = 0; t < ntiles; ++t) {
             const hnt_fields& f = fields[t];
             const int n = f.n1;
-            float4* recs = blocks ? nullptr : (float4*)W.recs.p + 2 * off;
-            if (batches[t].npeaks > 0 && !blocks)
-                jobs.push_back(RepackJob{f.delta, f.etax, f.etay, f.etaz, f.eta2x, f.eta2y,
-                                         f.eta2z, n, recs});
             TileDev& T = TD[t];
-            T.recs = recs;
             T.delta = f.delta;
             T.etax = f.etax;
             T.etay = f.etay;
@@ -2357,10 +2357,25 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
             T.res = results[t];
             T.npeaks = b.npeaks;
             T.base = meta[t];
-            off += (int64_t)n * n * n;
         }
     }
-    launch_repacks(st, jobs);
+    // ---- repack every tile's fields into 32-byte cell records (the lane-per-peak kernels') ----
+    std::vector<RepackJob> jobs;
+    const auto repack = [&]() -> hnt_status {
+        HNT_TRY(reserve_in(ctx, W.recs, (size_t)ncell * 32, W.arena));
+        float4* recs = (float4*)W.recs.p;
+        for (int t = 0; t < ntiles; ++t) {
+            const hnt_fields& f = fields[t];
+            TD[t].recs = recs;
+            if (batches[t].npeaks > 0)
+                jobs.push_back(RepackJob{f.delta, f.etax, f.etay, f.etaz, f.eta2x, f.eta2y,
+                                         f.eta2z, f.n1, recs});
+            recs += 2 * (int64_t)f.n1 * f.n1 * f.n1;
+        }
+        launch_repacks(st, jobs);
+        return HNT_OK;
+    };
+    if (!blocks) HNT_TRY(repack());
     HNT_TRY(reserve_in(ctx, W.tiles, TD.size() * sizeof(TileDev), W.arena));
     HNT_TRY(reserve_in(ctx, W.tilemeta, meta.size() * sizeof(int64_t), W.arena));
     W.meta_host = meta;
@@ -2453,10 +2468,27 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
     A.early = early ? 1 : 0;
     A.rmax2rs = params->rmax2rs;
 
+    bool have_stops = false;
     if (blocks) {
         stage_end(ctx, HNT_STAGE_SA_PREP);
-        return analyse_blocks(ctx, W, A, TT, ntiles, batches, results, masks, meta, ntot, ngroups,
-                              order_by);
+        const hnt_status done = analyse_blocks(ctx, W, A, TT, ntiles, batches, results, masks, meta,
+                                               ntot, ngroups, order_by, &have_stops);
+        if (done != HNT_ERR_ALLOC && !have_stops) return done;
+        stage_end(ctx, HNT_STAGE_SA_CROSS);
+        stage_end(ctx, HNT_STAGE_SA_KERNEL);
+        stage_begin(ctx, HNT_STAGE_SA_PREP);
+        if (done == HNT_ERR_ALLOC) {  // as much memory as the kernel without blocks would find
+            HNT_HIP(hipStreamSynchronize(st));
+            for (DevBuf* b : {&W.cross, &W.bcnt, &W.boff, &W.bbase, &W.slots2, &W.slots3, &W.brick,
+                              &W.far, &W.walk, &W.prof})
+                release(*b);
+            (void)hipGetLastError();
+            clear_error();
+            have_stops = false;
+        }
+        HNT_TRY(repack());
+        HNT_HIP(hipMemcpyAsync(W.tiles.p, TD.data(), TD.size() * sizeof(TileDev),
+                               hipMemcpyHostToDevice, st));
     }
 
     const bool kahan = params->precision == HNT_PREC_FP32_KAHAN;
@@ -2535,8 +2567,9 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
         int32_t* stops = (int32_t*)W.stops.p;
         if (params->order == HNT_ORDER_CROSSING) {
             const int64_t G8 = (ngroups + 7) / 8;
-            hipLaunchKernelGGL(crossing_kernel, dim3((unsigned)(8 * G8)), dim3(64), 0, st, A, G8,
-                               stops, nullptr);
+            if (!have_stops)
+                hipLaunchKernelGGL(crossing_kernel, dim3((unsigned)(8 * G8)), dim3(64), 0, st, A, G8,
+                                   stops);
         } else if (params->order == HNT_ORDER_GIVEN) {
             // the caller's extents order the peaks; no pass of the library's own
             HNT_HIP(hipMemcpyAsync(stops, params->extent, (size_t)ntot * 4,
