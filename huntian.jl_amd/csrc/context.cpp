@@ -366,6 +366,8 @@ hnt_status upload_tables_to(hnt_ctx* ctx, TablesDev& T, const hnt_shell_tables* 
     T.ncells = nc;
     T.near_cells = near_cells;
     T.near_shells = near_shells;
+    T.mid_shells = near_shells;
+    while (T.mid_shells < ns - 1 && t->shell_r2[T.mid_shells] <= 400) ++T.mid_shells;
     T.blocks_ok = !ar && blocks_ok && near_cells <= 2112 && near_shells <= 62 && even;
     T.host.swap(h);
     return HNT_OK;

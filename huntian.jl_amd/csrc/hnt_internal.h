@@ -45,6 +45,7 @@ struct TablesDev {
     DevBuf near_order;          // uint8: the shells within the halo by falling number of cells
     int32_t near_cells = 0;     // table cells of the shells within the halo
     int32_t near_shells = 0;    // those shells, 1 .. near_shells
+    int32_t mid_shells = 0;     // shells 1 .. mid_shells have r <= 20 cells
     bool blocks_ok = false;     // the shell-block path can use these tables
 };
 

@@ -2003,13 +2003,13 @@ void launch_main(hipStream_t st, const LaunchDesc& d) {
 // The analysis by shell blocks, from the first order on: crossing pass, block offsets, the
 // radial logic's order, then per chunk of the schedule the gather, Fbar and the radial logic,
 // and the halos' mask.  *lanes: the call is left, with its extents in W.stops, to the lane-per-peak
-// kernel, whose scratch does not grow with the peaks.  Nothing but schedule_extent is written before
+// kernel, because that is quicker or its scratch, which does not grow with the peaks, smaller.  Nothing but schedule_extent is written before
 // that, nor before a buffer cannot be had (HNT_ERR_ALLOC).
-template <class OrderBy>
+template <class OrderBy, class LaneRoom>
 hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT, int ntiles,
                           const hnt_batch* batches, hnt_results* results, int8_t* const* masks,
                           const std::vector<int64_t>& meta, int64_t ntot, int64_t ngroups,
-                          OrderBy&& order_by, bool* lanes) {
+                          int64_t ncell, OrderBy&& order_by, LaneRoom&& lane_room, bool* lanes) {
     *lanes = false;
     hipStream_t st = ctx->stream;
     bool any_mask = false;
@@ -2090,7 +2090,7 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     // needed), else what the scan found, in chunks of kBlockBudget and what is left of the brick in
     // which a chunk ends.  A brick crowded so that this does not hold the profile to a quarter above
     // the budget (it takes 80 k peaks of 650 blocks in a 64^3 brick, or many peaks per cell) is
-    // lane-per-peak work
+    // lane-per-peak work, if there is room for that
     const int nbmax = (A.NS >> 2) + 1;
     constexpr int64_t kBlockBytes = BLK_DOUBLES * 8;
     constexpr int64_t kBlockBudget = ((int64_t)32 << 30) / kBlockBytes;
@@ -2098,10 +2098,27 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     const int L2 = std::min(std::max(ctx->brick_log2, 4), 7);
     if (ntot * nbmax * kBlockBytes > ((int64_t)1 << 30)) {
         int64_t last_off = 0;
-        int32_t last_cnt = 0;
+        int32_t last_cnt = 0, nbricks = 0;
+        double part[WK_WG * WK_N], work[WK_N] = {0, 0, 0, 0, 0, 0};
+        const int64_t ns = std::min<int64_t>(ntot, 1 << 16);
+        HNT_TRY(reserve(ctx, W.flag, sizeof(part)));
+        hipLaunchKernelGGL(work_sample_kernel, dim3(WK_WG), dim3(256), 0, st, A, keys, vals,
+                           (const int32_t*)stops, ntot, ns, TT.near_shells, TT.mid_shells,
+                           (double*)W.flag.p);
+        HNT_HIP(hipMemcpyAsync(part, W.flag.p, sizeof(part), hipMemcpyDeviceToHost, st));
+        HNT_HIP(hipMemcpyAsync(&nbricks, bcount, 4, hipMemcpyDeviceToHost, st));
         HNT_HIP(hipMemcpyAsync(&last_off, off + (ntot - 1), 8, hipMemcpyDeviceToHost, st));
         HNT_HIP(hipMemcpyAsync(&last_cnt, cnt + (ntot - 1), 4, hipMemcpyDeviceToHost, st));
         HNT_HIP(hipStreamSynchronize(st));
+        for (int w = 0; w < WK_WG; ++w)
+            for (int c = 0; c < WK_N; ++c)
+                work[c] = c == 5 ? std::max(work[c], part[w * WK_N + c])
+                                 : work[c] + part[w * WK_N + c] * ((double)ntot / (double)ns);
+        if (lanes_quicker(work, (double)ntot, (double)nbricks, (double)ncell) && lane_room()) {
+            *lanes = true;
+            stage_end(ctx, HNT_STAGE_SA_CROSS);
+            return HNT_OK;
+        }
         const int64_t total = last_off + last_cnt;
         first[1] = total;
         if (total > kBlockBudget) {
@@ -2126,7 +2143,7 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     }
     int64_t cap = 0;
     for (size_t c = 0; c + 1 < pos.size(); ++c) cap = std::max(cap, first[c + 1] - first[c]);
-    if (cap > kBlockBudget + kBlockBudget / 4) {
+    if (cap > kBlockBudget + kBlockBudget / 4 && lane_room()) {
         *lanes = true;
         stage_end(ctx, HNT_STAGE_SA_CROSS);
         return HNT_OK;
@@ -2319,9 +2336,31 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
     const bool early0 = params->early_exit && !limited;
     int maxn = 1;
     for (int t = 0; t < ntiles; ++t) maxn = std::max(maxn, fields[t].n1);
-    const bool blocks = early0 && !desc && !W.arena && params->order == HNT_ORDER_CROSSING &&
-                        params->precision == HNT_PREC_FP64 && ctx->gang == 1 && TT.blocks_ok &&
-                        (int64_t)(tables->rmax + 1) * maxn * maxn < (1LL << 31);
+    const bool can_blocks = early0 && !desc && !W.arena && params->order == HNT_ORDER_CROSSING &&
+                            params->precision == HNT_PREC_FP64 && ctx->gang == 1 && TT.blocks_ok &&
+                            (int64_t)(tables->rmax + 1) * maxn * maxn < (1LL << 31);
+    // A lane per peak also where that is quicker.  Many peaks per cell share the lines it reads (ms,
+    // blocks / lanes: radius 8, 0.38 peaks per cell of a 64^3 tile 4.9 / 3.0, 0.11 1.8 / 2.2; radius
+    // 20, 0.48 of a 128^3 tile 49 / 41, 0.24 27 / 30).  And few shells around thinly spread peaks
+    // are less work than staging a brick's five boxes (0.125 us for each brick that has peaks,
+    // against the records' 15.5 ps per cell, the deepest lane's 1.1 us per cell and, per shell
+    // radius beyond 2, 1.5 ns a peak; ms: 100 k peaks of a 512^3 tile, radius 3 4.4 / 2.8, 6 6.0 /
+    // 4.8, 10 k 1.6 / 2.3 and 2.0 / 3.4; 1 M 7.0 / 6.4 and 10.7 / 16.9; 30 k peaks of a 256^3 tile, 2
+    // 0.88 / 0.70, 4 1.06 / 1.14).  There has to be room for the records; lanes_quicker decides on
+    // the larger calls.
+    int64_t pcell = 0;  // of the tiles with peaks
+    for (int t = 0; t < ntiles; ++t)
+        pcell += batches[t].npeaks > 0 ? (int64_t)fields[t].n1 * fields[t].n1 * fields[t].n1 : 0;
+    const double np = (double)ntot, bricks = (double)pcell / (BR_CORE * BR_CORE * BR_CORE);
+    const double staging = 0.07 + 0.125e-3 * bricks * (1.0 - std::exp(-np / bricks));
+    const double lanes = 15.5e-9 * (double)pcell + 1.1e-3 * (double)tables->ncells +
+                         1.5e-6 * (tables->rmax - 2) * np;
+    bool blocks = can_blocks && 3.0 * np <= (double)pcell && staging <= lanes;
+    if (can_blocks && !blocks && reserve(ctx, W.recs, (size_t)ncell * 32) != HNT_OK) {
+        (void)hipGetLastError();
+        clear_error();
+        blocks = true;
+    }
 
     std::vector<TileDev>& TD = W.tile_host;
     TD.assign((size_t)ntiles, TileDev{});
@@ -2468,11 +2507,59 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
     A.early = early ? 1 : 0;
     A.rmax2rs = params->rmax2rs;
 
+    const bool kahan = params->precision == HNT_PREC_FP32_KAHAN;
+    // the ganged kernels analyse every peak to the last shell: a shell limit takes the
+    // lane-per-peak kernel
+    const int gang = limited ? 1 : ctx->gang;
+    const void* kern = gang == 64 ? (kahan ? (const void*)shell_wave_kernel<SumKahan>
+                                           : (const void*)shell_wave_kernel<SumF64>)
+                     : gang == 16 ? (kahan ? (const void*)shell_gang_kernel<SumKahan>
+                                           : (const void*)shell_gang_kernel<SumF64>)
+                                  : (kahan ? (const void*)shell_analyse_kernel<SumKahan>
+                                           : (const void*)shell_analyse_kernel<SumF64>);
+    A.slot_doubles = (int64_t)(A.NS + 1) * PW;
+    // the lanes' profiles and the number of resident wavefronts they allow
+    const auto lane_profiles = [&](int64_t* nblocks_out) -> hnt_status {
+        int per_cu = 0;
+        HNT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64, 0));
+        if (per_cu < 1) per_cu = 1;
+        if (ctx->waves_per_cu > 0 && ctx->waves_per_cu < per_cu) per_cu = ctx->waves_per_cu;
+        const size_t slot_bytes = (size_t)A.slot_doubles * 8;
+        // profile scratch: 32 GiB at most, or what is left of a fixed region (fewer resident
+        // wavefronts then, same results)
+        size_t budget = (size_t)32 << 30;
+        if (W.arena) {
+            const size_t used = (W.arena->used + 255) & ~(size_t)255;
+            budget = used < W.arena->cap ? W.arena->cap - used : 0;
+        }
+        int64_t nblocks = (int64_t)per_cu * ctx->num_cus;
+        int64_t cap_blocks = (int64_t)(budget / (slot_bytes * 64));
+        if (nblocks > cap_blocks) nblocks = cap_blocks;
+        int64_t want = ((ngroups + 7) / 8) * 8;
+        if (nblocks > want) nblocks = want;
+        nblocks = (nblocks / 8) * 8;
+        if (nblocks < 8) nblocks = 8;
+        HNT_TRY(reserve_in(ctx, W.prof, (size_t)nblocks * 64 * slot_bytes, W.arena));
+        *nblocks_out = nblocks;
+        return HNT_OK;
+    };
+
     bool have_stops = false;
     if (blocks) {
         stage_end(ctx, HNT_STAGE_SA_PREP);
+        // room for the lane-per-peak kernel, without which a call stays with the blocks
+        const auto lane_room = [&]() {
+            int64_t nb = 0;
+            if (reserve(ctx, W.recs, (size_t)ncell * 32) == HNT_OK && lane_profiles(&nb) == HNT_OK)
+                return true;
+            (void)hipGetLastError();
+            clear_error();
+            release(W.recs);
+            return false;
+        };
         const hnt_status done = analyse_blocks(ctx, W, A, TT, ntiles, batches, results, masks, meta,
-                                               ntot, ngroups, order_by, &have_stops);
+                                               ntot, ngroups, ncell, order_by, lane_room,
+                                               &have_stops);
         if (done != HNT_ERR_ALLOC && !have_stops) return done;
         stage_end(ctx, HNT_STAGE_SA_CROSS);
         stage_end(ctx, HNT_STAGE_SA_KERNEL);
@@ -2491,10 +2578,6 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
                                hipMemcpyHostToDevice, st));
     }
 
-    const bool kahan = params->precision == HNT_PREC_FP32_KAHAN;
-    // the ganged kernels analyse every peak to the last shell: a shell limit takes the
-    // lane-per-peak kernel
-    const int gang = limited ? 1 : ctx->gang;
     std::vector<PremaskJob> premasks;
     if (limited && params->variant == HNT_VARIANT_B && masks) {
         for (int t = 0; t < ntiles; ++t)
@@ -2521,37 +2604,12 @@ hnt_status analyse_tiles(hnt_ctx* ctx, SAWork& W, int ntiles, const hnt_fields* 
         HNT_TRY(reserve_in(ctx, W.paint, (size_t)ntot * 4, W.arena));
         A.paint = (int32_t*)W.paint.p;
     }
-    const void* kern = gang == 64 ? (kahan ? (const void*)shell_wave_kernel<SumKahan>
-                                           : (const void*)shell_wave_kernel<SumF64>)
-                     : gang == 16 ? (kahan ? (const void*)shell_gang_kernel<SumKahan>
-                                           : (const void*)shell_gang_kernel<SumF64>)
-                                  : (kahan ? (const void*)shell_analyse_kernel<SumKahan>
-                                           : (const void*)shell_analyse_kernel<SumF64>);
-    int per_cu = 0;
-    HNT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64, 0));
-    if (per_cu < 1) per_cu = 1;
-    if (ctx->waves_per_cu > 0 && ctx->waves_per_cu < per_cu) per_cu = ctx->waves_per_cu;
-    A.slot_doubles = (int64_t)(A.NS + 1) * PW;
-    const size_t slot_bytes = (size_t)A.slot_doubles * 8;
     HNT_TRY(reserve_in(ctx, W.queue, 8 * sizeof(unsigned long long), W.arena));
     A.qctr = (unsigned long long*)W.queue.p;
     const bool sched = A.early && params->order != HNT_ORDER_PLAIN;
     if (sched && W.arena) HNT_TRY(reserve_in(ctx, W.stops, (size_t)ntot * 4, W.arena));
-    // profile scratch: 32 GiB at most, or what is left of a fixed region (fewer resident
-    // wavefronts then, same results)
-    size_t budget = (size_t)32 << 30;
-    if (W.arena) {
-        const size_t used = (W.arena->used + 255) & ~(size_t)255;
-        budget = used < W.arena->cap ? W.arena->cap - used : 0;
-    }
-    int64_t nblocks = (int64_t)per_cu * ctx->num_cus;
-    int64_t cap_blocks = (int64_t)(budget / (slot_bytes * 64));
-    if (nblocks > cap_blocks) nblocks = cap_blocks;
-    int64_t want = ((ngroups + 7) / 8) * 8;
-    if (nblocks > want) nblocks = want;
-    nblocks = (nblocks / 8) * 8;
-    if (nblocks < 8) nblocks = 8;
-    HNT_TRY(reserve_in(ctx, W.prof, (size_t)nblocks * 64 * slot_bytes, W.arena));
+    int64_t nblocks = 0;
+    HNT_TRY(lane_profiles(&nblocks));
     A.prof = (double*)W.prof.p;
     for (int x = 0; x < 8; ++x) {
         A.qbeg[x] = ngroups * x / 8;
