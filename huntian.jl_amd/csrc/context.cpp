@@ -301,10 +301,6 @@ hnt_status upload_tables_to(hnt_ctx* ctx, TablesDev& T, const hnt_shell_tables* 
         order[s - 1] = (uint8_t)s;
         even = even && (s == 1 || t->shell_count[s - 1] % 2 == 0);
     }
-    // a shell's cells by rising planes (the far gather takes them plane by plane)
-    for (int32_t s = 0; s < ns; ++s)
-        for (int32_t c = 1; c < t->shell_count[s]; ++c)
-            blocks_ok = blocks_ok && t->dk[t->shell_start[s] + c] >= t->dk[t->shell_start[s] + c - 1];
     std::stable_sort(order.begin(), order.end(), [&](uint8_t a, uint8_t b) {
         return t->shell_count[a - 1] > t->shell_count[b - 1];
     });
