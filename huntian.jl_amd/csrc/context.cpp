@@ -59,6 +59,14 @@ hnt_status reserve_in(hnt_ctx* ctx, DevBuf& b, size_t bytes, Arena* ar) {
     return HNT_OK;
 }
 
+void release_merge(hnt_ctx* ctx) {
+    MergeBufs& m = ctx->mg;
+    for (DevBuf* b : {&m.a, &m.b, &m.c, &m.d, &m.rank, &m.cidx, &m.cstart, &m.off, &m.e1,
+                      &m.e2, &m.e3, &m.e4, &m.state, &m.instart, &m.dv, &m.pk, &m.pv, &m.newr,
+                      &m.pos, &m.prank, &m.ext})
+        release(*b);
+}
+
 void release_work(SAWork& w) {
     if (w.arena) {  // carved from a fixed region: nothing to free
         w = SAWork();
@@ -459,11 +467,7 @@ static void release_scratch(hnt_ctx* ctx) {
                       &ctx->rec_tabs, &ctx->rec_keep, &ctx->rec_slot, &ctx->fs_real,
                       &ctx->fs_base, &ctx->fs_work, &ctx->fs_aux, &ctx->fs_tab})
         release(*b);
-    MergeBufs& m = ctx->mg;
-    for (DevBuf* b : {&m.a, &m.b, &m.c, &m.d, &m.rank, &m.cidx, &m.cstart, &m.off, &m.e1,
-                      &m.e2, &m.e3, &m.e4, &m.state, &m.instart, &m.dv, &m.pk, &m.pv, &m.newr,
-                      &m.pos, &m.prank, &m.ext})
-        release(*b);
+    release_merge(ctx);
     release_fft(ctx);
     release_field_plans(ctx);
     for (hnt_ctx::FftTw& t : ctx->fft_tw) release(t.buf);

@@ -168,6 +168,7 @@ namespace hnt {
 
 hnt_status reserve(hnt_ctx* ctx, DevBuf& b, size_t bytes);
 void release(DevBuf& b);
+void release_merge(hnt_ctx* ctx);  // scratch of hnt_merge_catalog
 void release_work(SAWork& w);
 void release_fft(hnt_ctx* ctx);  // FFT plans of hnt_peak_find_tile
 void release_field_plans(hnt_ctx* ctx);  // FFT plans of the field-synthesis entries

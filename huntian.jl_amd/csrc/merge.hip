@@ -417,10 +417,10 @@ unsigned nblk(int64_t n) { return (unsigned)((n + MB - 1) / MB); }
 
 }  // namespace
 
-extern "C" hnt_status hnt_merge_catalog(hnt_ctx* ctx, const float* records, int64_t nhalo,
-                                        int32_t nfields, int32_t volume_reduction,
-                                        int32_t fortran_ties, float* out, int64_t* nout) {
-    HNT_TRY(begin_call(ctx));
+// guess: entries that the scans have room for before their number is known (0: count first).
+static hnt_status merge_catalog(hnt_ctx* ctx, const float* records, int64_t nhalo, int32_t nfields,
+                                int32_t volume_reduction, int32_t fortran_ties, float* out,
+                                int64_t* nout, int64_t guess) {
     HNT_REQUIRE(nout && (nhalo == 0 || (records && out)), "hnt_merge_catalog: NULL argument");
     HNT_REQUIRE(nfields == 11 || nfields == 33, "hnt_merge_catalog: records of %d floats "
                 "(11 or 33)", nfields);
@@ -527,9 +527,8 @@ extern "C" hnt_status hnt_merge_catalog(hnt_ctx* ctx, const float* records, int6
     HNT_TRY(reserve(ctx, ctx->small, 64));
     unsigned long long* count = (unsigned long long*)ctx->small.p;
     const auto scan_grid = [&](int w) { return dim3((unsigned)((N + MB / w - 1) / (MB / w))); };
-    // entries of a scan: room for one per halo (up to 2^24) or what an earlier call had; more are
-    // counted, and scanned again with room for all
-    const int64_t guess = std::min<int64_t>(N, 1 << 24);
+    // entries of a scan: room for the guess or what an earlier call had; more are counted, and
+    // scanned again with room for all
     int bits = 1;
     while (((int64_t)1 << bits) < 2 * N) ++bits;  // of 2 N
     int64_t E = 0;
@@ -651,4 +650,21 @@ extern "C" hnt_status hnt_merge_catalog(hnt_ctx* ctx, const float* records, int6
     HNT_TRY(finish_call(ctx, "hnt_merge_catalog"));
     *nout = last_off + last_keep;
     return HNT_OK;
+}
+
+extern "C" hnt_status hnt_merge_catalog(hnt_ctx* ctx, const float* records, int64_t nhalo,
+                                        int32_t nfields, int32_t volume_reduction,
+                                        int32_t fortran_ties, float* out, int64_t* nout) {
+    HNT_TRY(begin_call(ctx));
+    // room for one entry per halo (80 bytes) saves a catalog's scans their second pass; a device
+    // without the memory for that counts first.  `out` is written last
+    const int64_t guess = std::min<int64_t>(std::max<int64_t>(nhalo, 0), 1 << 24);
+    const hnt_status done = merge_catalog(ctx, records, nhalo, nfields, volume_reduction,
+                                          fortran_ties, out, nout, guess);
+    if (done != HNT_ERR_ALLOC) return done;
+    HNT_HIP(hipStreamSynchronize(ctx->stream));
+    release_merge(ctx);
+    (void)hipGetLastError();
+    clear_error();
+    return merge_catalog(ctx, records, nhalo, nfields, volume_reduction, fortran_ties, out, nout, 0);
 }
