@@ -446,6 +446,17 @@ __global__ __launch_bounds__(C * L / 8, 8) void fft_cols_direct(
     }
 }
 
+// X[k] of a real row from Z, the M-point FFT of its pairs (padded, in LDS).
+__device__ __forceinline__ float2 half_coeff(const float2* row, int M, int k,
+                                             const float2* __restrict__ WL) {
+    const float2 zk = row[pad(k & (M - 1))];
+    const float2 zm = row[pad((M - k) & (M - 1))];
+    const float2 ev = make_float2((zk.x + zm.x) * 0.5f, (zk.y - zm.y) * 0.5f);
+    // (zk - conj zm) / 2i
+    const float2 od = make_float2((zk.y + zm.y) * 0.5f, -(zk.x - zm.x) * 0.5f);
+    return cadd(ev, ctw<false>(od, WL[k]));
+}
+
 // Forward x pass: rows (iy, iz) of a w^3 real field (iy, iz < w), zero-extended to L = 2M,
 // into rows of the (M + 1) x L x L half spectrum.  z[m] = x[2m] + i x[2m + 1], Z = FFT_M(z),
 // X[k] = E[k] + W_L^k O[k] with E = (Z[k] + conj Z[M-k]) / 2, O = (Z[k] - conj Z[M-k]) / 2i.
@@ -454,8 +465,12 @@ __global__ __launch_bounds__(C * L / 8, 8) void fft_cols_direct(
 // element they and the twiddles' L2 reads bounded the row passes, with 4-byte loads and stores
 // of neighbouring reals: 512^3 forward 0.42 -> 0.29 ms, 1024^3 3.1 -> 1.9, inverse 1.62 -> 1.22).
 // `pairs`: w is even and f 8-byte aligned.  The twiddles of the stages lie in LDS.
+// SHORT: rows of less than 64 elements, whose pieces would leave most lanes idle: a thread per
+// element of the workgroup's rows (2LPT of a 16^3 tile: pieces 187 us, elements 162).
 constexpr int ROW_TW = 256;  // entries the stages read: below M / 4 (1024 = 8 8 4 4)
 constexpr int ROW_U = SMALL_DATA / SMALL_T;  // pieces per wavefront
+constexpr int SHORT_LGM = 5;
+template <bool SHORT>
 __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_r2c(
     const float* __restrict__ f, int w, int lgM, int lgG, int pairs, float2* __restrict__ spec,
     const float2* __restrict__ WM, const float2* __restrict__ WL) {
@@ -466,6 +481,28 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_r2c(
     const int nrows = w * w;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if constexpr (SHORT) {
+        const int e = threadIdx.x, g = e >> lgM, x = 2 * (e & (M - 1));
+        if (g < G) {
+            float2 v = make_float2(0.0f, 0.0f);
+            if (row0 + g < nrows) {
+                const float* src = f + (int64_t)(row0 + g) * w;
+                if (x < w) v.x = src[x];
+                if (x + 1 < w) v.y = src[x + 1];
+            }
+            buf[g * LS + pad(e & (M - 1))] = v;
+        }
+        __syncthreads();
+        stockham<false, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, WM);
+        for (int e2 = threadIdx.x; e2 < G * nk; e2 += SMALL_T) {
+            const int g2 = e2 / nk, k = e2 - g2 * nk, row = row0 + g2;
+            if (row >= nrows) break;
+            const int iz = row / w, iy = row - iz * w;
+            spec[k + (int64_t)fft_pitch(L) * iy + fft_plane(L) * iz] =
+                half_coeff(buf + g2 * LS, M, k, WL);
+        }
+        return;
+    }
     const int lgP = lgM > 6 ? lgM - 6 : 0;  // pieces per row
     if ((int)threadIdx.x < min(M, ROW_TW)) tw[threadIdx.x] = WM[threadIdx.x];
     float2 v[ROW_U];
@@ -497,16 +534,19 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_r2c(
         if (row >= nrows) break;
         const int iz = row / w, iy = row - iz * w;
         float2* __restrict__ dst = spec + (int64_t)fft_pitch(L) * iy + fft_plane(L) * iz;
-        for (int k = lane; k < nk; k += 64) {
-            const float2 zk = buf[g * LS + pad(k & (M - 1))];
-            const float2 zm = buf[g * LS + pad((M - k) & (M - 1))];
-            const float2 ev = make_float2((zk.x + zm.x) * 0.5f, (zk.y - zm.y) * 0.5f);
-            // (zk - conj zm) / 2i
-            const float2 od = make_float2((zk.y + zm.y) * 0.5f, -(zk.x - zm.x) * 0.5f);
-            const float2 t = ctw<false>(od, WL[k]);
-            dst[k] = cadd(ev, t);
-        }
+        for (int k = lane; k < nk; k += 64) dst[k] = half_coeff(buf + g * LS, M, k, WL);
     }
+}
+
+// Element xx of a row of the inverse x pass into out[o].
+__device__ __forceinline__ void store_real(const float2* row, int xx, float scale, int mode,
+                                           float coef, int64_t o, const float* __restrict__ base,
+                                           float* __restrict__ out) {
+    const float2 zz = row[pad(xx >> 1)];
+    const float v = ((xx & 1) ? zz.y : zz.x) * scale;
+    if (mode == 0) out[o] = v;
+    else if (mode == 1) out[o] = out[o] - (v * v) * coef;
+    else out[o] = (base[o] * base[o]) * 0.5f - (v * v) * coef;
 }
 
 // The kept part of the inverse x pass's rows, from their FFTs in LDS; `pairs`: s and n even, out
@@ -549,15 +589,8 @@ __device__ __forceinline__ void store_rows(const float2* buf, int LS, int G, int
     for (int g = wave; g < G; g += SMALL_T / 64) {
         const int row = row0 + g;
         if (row >= nrows) break;
-        for (int xo = lane; xo < n; xo += 64) {
-            const int xx = s + xo;
-            const float2 zz = buf[g * LS + pad(xx >> 1)];
-            const float v = ((xx & 1) ? zz.y : zz.x) * scale;
-            const int64_t o = (int64_t)row * n + xo;
-            if (mode == 0) out[o] = v;
-            else if (mode == 1) out[o] = out[o] - (v * v) * coef;
-            else out[o] = (base[o] * base[o]) * 0.5f - (v * v) * coef;
-        }
+        for (int xo = lane; xo < n; xo += 64)
+            store_real(buf + g * LS, s + xo, scale, mode, coef, (int64_t)row * n + xo, base, out);
     }
 }
 
@@ -566,6 +599,8 @@ __device__ __forceinline__ void store_rows(const float2* buf, int LS, int G, int
 // s2 -= (scale * x)^2 * coef (mode 1), or s2 = base^2 / 2 - (scale * x)^2 * coef (mode 2).  X[0] and X[M] enter through their real parts.
 // Z[k] = (X[k] + conj X[M-k]) + i (X[k] - conj X[M-k]) W_L^-k, z = IFFT_M(Z), x[2m] = Re z[m],
 // x[2m + 1] = Im z[m].
+// SHORT: as fft_rows_r2c's.
+template <bool SHORT>
 __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r(
     const float2* __restrict__ spec, int lgM, int lgG, int s, int n, float scale, int mode,
     float coef, int pairs, const float* __restrict__ base, float* __restrict__ out,
@@ -578,9 +613,19 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r(
     const int nrows = n * n;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int lgP = lgM > 6 ? lgM - 6 : 0;  // pieces per row
-    if ((int)threadIdx.x < min(M, ROW_TW)) tw[threadIdx.x] = WM[threadIdx.x];
-    {
+    if constexpr (SHORT) {
+        for (int e = threadIdx.x; e < G * (M + 1); e += SMALL_T) {
+            const int g = e / (M + 1), k = e - g * (M + 1), row = row0 + g;
+            float2 v = make_float2(0.0f, 0.0f);
+            if (row < nrows) {
+                const int jz = row / n, jy = row - jz * n;
+                v = spec[k + (int64_t)fft_pitch(L) * (s + jy) + fft_plane(L) * (s + jz)];
+            }
+            buf[g * LS + pad(k)] = v;
+        }
+    } else {
+        const int lgP = lgM > 6 ? lgM - 6 : 0;  // pieces per row
+        if ((int)threadIdx.x < min(M, ROW_TW)) tw[threadIdx.x] = WM[threadIdx.x];
         float2 v[ROW_U], nyq = make_float2(0.0f, 0.0f);
 #pragma unroll
         for (int u = 0; u < ROW_U; ++u) {
@@ -606,7 +651,7 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r(
     }
     __syncthreads();
     // untwist into Z (registers first: Z[k] needs X[M - k] of the same row)
-    constexpr int MAXB = SMALL_DATA / SMALL_T;
+    constexpr int MAXB = SHORT ? 1 : SMALL_DATA / SMALL_T;
     float2 z[MAXB];
 #pragma unroll
     for (int q = 0; q < MAXB; ++q) {
@@ -632,8 +677,16 @@ __global__ __launch_bounds__(SMALL_T, 8) void fft_rows_c2r(
         if (e < G * M) buf[(e >> lgM) * LS + pad(e & (M - 1))] = z[q];
     }
     __syncthreads();
-    stockham<true, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, tw);
-    store_rows(buf, LS, G, row0, nrows, s, n, scale, mode, coef, pairs, base, out);
+    stockham<true, SMALL_T, SMALL_DATA>(buf, LS, G, lgM, SHORT ? WM : tw);
+    if constexpr (SHORT) {
+        for (int e = threadIdx.x; e < G * n; e += SMALL_T) {
+            const int g = e / n, xo = e - g * n;
+            if (row0 + g >= nrows) break;
+            store_real(buf + g * LS, s + xo, scale, mode, coef, (int64_t)(row0 + g) * n + xo, base, out);
+        }
+    } else {
+        store_rows(buf, LS, G, row0, nrows, s, n, scale, mode, coef, pairs, base, out);
+    }
 }
 
 // fft_rows_c2r for L = 512 (M = 256, 16 rows per workgroup; 0.50 -> 0.25 ms for 512^3 with the
@@ -847,9 +900,9 @@ hnt_status fft_forward(hnt_ctx* ctx, const float* f, int w, int L, float2* spec)
     HNT_TRY(fft_twiddles(ctx, M, &WM));
     const int lgG = rows_lgG(M);
     const int64_t rows = (int64_t)w * w;
-    hipLaunchKernelGGL(fft_rows_r2c, dim3((unsigned)((rows + (1 << lgG) - 1) >> lgG)),
-                       dim3(SMALL_T), 0, st, f, w, ilog2(M), lgG, w % 2 == 0 && ((uintptr_t)f & 7) == 0, spec,
-                       WM, WL);
+    hipLaunchKernelGGL(ilog2(M) <= SHORT_LGM ? fft_rows_r2c<true> : fft_rows_r2c<false>,
+                       dim3((unsigned)((rows + (1 << lgG) - 1) >> lgG)), dim3(SMALL_T), 0, st, f, w,
+                       ilog2(M), lgG, w % 2 == 0 && ((uintptr_t)f & 7) == 0, spec, WM, WL);
     FftOp none;
     const int lgC = cols_lgC(L);
     const unsigned gx = (unsigned)((nk + (1 << lgC) - 1) >> lgC);
@@ -902,9 +955,10 @@ hnt_status fft_inverse(hnt_ctx* ctx, const float2* spec, float2* work, int L, in
                            pairs, base, out, WM, WL);
         return HNT_OK;
     }
-    hipLaunchKernelGGL(fft_rows_c2r, dim3((unsigned)((rows + (1 << lgG) - 1) >> lgG)),
-                       dim3(SMALL_T), 0, st, (const float2*)work, ilog2(M), lgG, s, n, scale,
-                       mode, coef, pairs, base, out, WM, WL);
+    hipLaunchKernelGGL(ilog2(M) <= SHORT_LGM ? fft_rows_c2r<true> : fft_rows_c2r<false>,
+                       dim3((unsigned)((rows + (1 << lgG) - 1) >> lgG)), dim3(SMALL_T), 0, st,
+                       (const float2*)work, ilog2(M), lgG, s, n, scale, mode, coef, pairs, base, out,
+                       WM, WL);
     return HNT_OK;
 }
 
