@@ -13,7 +13,8 @@
 //
 // Measured against the lane-per-peak kernel with its records (same bits): shell analysis of the
 // 1024^3 tile 327 -> 211 ms, of the 512^3 tile 51.6 -> 25.8 ms, of a 128^3 tile 7.9 -> 1.10 ms, of a
-// 40^3 tile 1.33 -> 0.37 ms, of 24 tiles of 96^3 to 256^3 with their peak finding 37.6 -> 21.2 ms.
+// 40^3 tile 1.33 -> 0.37 ms, of 24 tiles of 96^3 to 256^3 in one call 37.6 -> 20.9 ms.  Calls that a
+// lane per peak answers quicker stay with that kernel (analyse_tiles, lanes_quicker).
 //
 // A block's sums are five 128-byte lines side by side, one per field (delta, its transpose,
 // psi_1 xyz), four doubles per shell: {F, G0, G1, G2}, {H0, H1, H2, -}, {S, R0, R1, R2} x 3;
@@ -513,7 +514,7 @@ __global__ __launch_bounds__(FAR_T) void gather_far_kernel(SAArgs a, BlockArgs B
 }
 
 // ------------------------------------------------------------------ gather from the fields
-// The peaks whose balls leave the grid, read from the fields as they are.
+// The peaks whose balls leave the grid (far_list_kernel's slots), read from the fields as they are.
 struct BlockSums {
     double F, G0, G1, G2, H0, H1, H2;
     double S0, S1, S2, R00, R01, R02, R10, R11, R12, R20, R21, R22;
@@ -552,44 +553,16 @@ struct BlockFields {
 };
 
 // The shell's sums of one lane: cells [st, st + nc) of the table around the peak whose cell is
-// c0 (cT in the transposed field).  CHECK: some lane's ball leaves the grid; its cells outside
-// are skipped.
-template <bool CHECK>
+// c0 (cT in the transposed field); cells outside the grid are skipped.
 __device__ __forceinline__ void block_shell(const BlockFields& f, const uint32_t* __restrict__ cell8,
                                             int st, int nc, int n, int ci, int cj, int ck,
                                             int64_t c0, int64_t cT, BlockSums& A) {
     const int s1 = n, s2 = n * n;
-    constexpr int U = CHECK ? 1 : 4;
-    int c = 0;
-    if (!CHECK) {
-        for (; c + U <= nc; c += U) {
-            uint32_t w[U];
-            float d[U], t[U], x[U], y[U], z[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) w[u] = cell8[st + c + u];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int ox = byte_of(w[u], 0), oy = byte_of(w[u], 1), oz = byte_of(w[u], 2);
-                const int64_t o = c0 + (ox + oy * s1 + oz * s2);
-                d[u] = f.d[o];
-                t[u] = f.d[cT + (oz + ox * s1 + oy * s2)];
-                x[u] = f.x[o];
-                y[u] = f.y[o];
-                z[u] = f.z[o];
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                A.add(d[u], t[u], x[u], y[u], z[u], (float)byte_of(w[u], 0),
-                      (float)byte_of(w[u], 1), (float)byte_of(w[u], 2));
-        }
-    }
-    for (; c < nc; ++c) {
+    for (int c = 0; c < nc; ++c) {
         const uint32_t w = cell8[st + c];
         const int ox = byte_of(w, 0), oy = byte_of(w, 1), oz = byte_of(w, 2);
-        if (CHECK) {
-            const int i1 = ci + ox, i2 = cj + oy, i3 = ck + oz;
-            if (i1 < 1 || i1 > n || i2 < 1 || i2 > n || i3 < 1 || i3 > n) continue;
-        }
+        const int i1 = ci + ox, i2 = cj + oy, i3 = ck + oz;
+        if (i1 < 1 || i1 > n || i2 < 1 || i2 > n || i3 < 1 || i3 > n) continue;
         const int64_t o = c0 + (ox + oy * s1 + oz * s2);
         A.add(f.d[o], f.d[cT + (oz + ox * s1 + oy * s2)], f.x[o], f.y[o], f.z[o], (float)ox,
               (float)oy, (float)oz);
@@ -606,7 +579,7 @@ __global__ __launch_bounds__(256) void gather_blocks_kernel(SAArgs a, BlockArgs 
     uint64_t* mask = lds;                    // [nbmax] peaks with more than b blocks
     int* pre = (int*)(mask + nbmax);         // [nbmax + 1] items before block b
     __shared__ int64_t s_base[64];
-    __shared__ int s_pos[3][64], s_stop[64], s_out[64], s_nb;
+    __shared__ int s_pos[3][64], s_stop[64], s_nb;
     // contiguous runs of groups per XCD (workgroups are dealt to the XCDs in turn)
     const int64_t nwg = (int64_t)gridDim.x, per = nwg >> 3;
     const int64_t w = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -621,15 +594,13 @@ __global__ __launch_bounds__(256) void gather_blocks_kernel(SAArgs a, BlockArgs 
         if (p >= 0) {
             const int64_t b0 = B.base[T.base + p] - B.e0;
             if (b0 >= 0 && b0 < B.ne) {
-                const int stop = B.stop[T.base + p], R = (int)a.rad[stop];
-                const int ci = T.pi[p], cj = T.pj[p], ck = T.pk[p];
+                const int stop = B.stop[T.base + p];
                 nb = blocks_of(stop);
                 s_base[tid] = b0;
                 s_stop[tid] = stop;
-                s_pos[0][tid] = ci;
-                s_pos[1][tid] = cj;
-                s_pos[2][tid] = ck;
-                s_out[tid] = ball_outside(T, ci, cj, ck, R);
+                s_pos[0][tid] = T.pi[p];
+                s_pos[1][tid] = T.pj[p];
+                s_pos[2][tid] = T.pk[p];
             }
         }
         int sum = 0, b = 0;
@@ -666,7 +637,6 @@ __global__ __launch_bounds__(256) void gather_blocks_kernel(SAArgs a, BlockArgs 
         const int n = T.n;
         const int64_t c0 = (int64_t)(ci - 1) + (cj - 1) * T.s1 + (ck - 1) * T.s2;
         const int64_t cT = (int64_t)(ck - 1) + (ci - 1) * T.s1 + (cj - 1) * T.s2;
-        const bool check = __ballot(on && s_out[q]) != 0ull;
         const int64_t e = on ? s_base[q] + b : 0;
         for (int u = 0; u < BLK; ++u) {
             const int s = BLK * b + u;
@@ -681,8 +651,7 @@ __global__ __launch_bounds__(256) void gather_blocks_kernel(SAArgs a, BlockArgs 
                 A.S2 = 0.0 + (double)f.z[c0];
             } else {
                 const int st = a.shell_start[s - 1], nc = a.shell_count[s - 1];
-                if (check) block_shell<true>(f, B.cell8, st, nc, n, ci, cj, ck, c0, cT, A);
-                else block_shell<false>(f, B.cell8, st, nc, n, ci, cj, ck, c0, cT, A);
+                block_shell(f, B.cell8, st, nc, n, ci, cj, ck, c0, cT, A);
                 const double r = a.rad[s], y = B.rinv[s];
                 for (double* v : {&A.G0, &A.G1, &A.G2, &A.H0, &A.H1, &A.H2, &A.R00, &A.R01, &A.R02,
                                   &A.R10, &A.R11, &A.R12, &A.R20, &A.R21, &A.R22})
