@@ -53,3 +53,24 @@ def test_too_little_memory_for_the_profiles(websky):
         torch.cuda.empty_cache()
         ctx.release_scratch()
     _same(got, plain, "little memory")
+
+
+def test_several_chunks_over_uneven_tiles(websky):
+    """Profiles of more than the 32 GiB that a call holds at a time: chunks of the schedule that begin
+    and end in the middle of tiles, every peak of every tile compared."""
+    tiles = []
+    for n, count in ((97, 100_000), (320, 7_000_000), (64, 40_000)):
+        tiles.append(dict(fields=_fields(n, n, False), **_peaks(n, count, n, 9, n - 9)))
+    tab = api.build_shell_tables(8)
+    kw = dict(alatt=2.0, ZZon=1.0, fcrit=api.fsc_of_z(websky, 0.0))
+    plain = api.shell_analyse_tiles(tiles, tab, websky, order="plain", **kw)
+    ctx = api.context(0)
+    ctx.release_scratch()
+    got = api.shell_analyse_tiles(tiles, tab, websky, order="crossing", **kw)
+    blocks = sum(float((r["nshells_used"].double() / 4).floor().sum()) + len(r["nshells_used"])
+                 for r in got)
+    ctx.release_scratch()
+    print(f"{blocks * 672 / 2 ** 30:.1f} GiB of profiles", flush=True)
+    assert blocks * 672 > 2 ** 35
+    for q, (a, b) in enumerate(zip(got, plain)):
+        _same(a, b, f"tile {q}")
