@@ -1979,7 +1979,8 @@ void launch_repacks(hipStream_t st, const std::vector<RepackJob>& jobs) {
 void launch_paint(hipStream_t st, const LaunchDesc& d) {
     if (!d.A.paint) return;
     const int64_t G8 = (d.A.ngroups + 7) / 8;
-    // groups that would not fill the CUs are shared out (128^3 tile 64 -> 16 us)
+    // groups that would not fill the CUs are shared out (us, 1 / 16 shares: 5 groups 13 / 5, 47 39 /
+    // 14, 313 90 / 26, 1563 189 / 54)
     const unsigned shares = d.A.ngroups < 2048 ? 16 : 1;
     hipLaunchKernelGGL(paint_mask_kernel, dim3((unsigned)(8 * G8), shares), dim3(64), 0, st, d.A, G8);
 }
@@ -2097,29 +2098,26 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
     std::vector<int64_t> pos{0, ntot}, first{0, ntot * nbmax};  // chunk boundaries
     const int L2 = std::min(std::max(ctx->brick_log2, 4), 7);
     if (ntot * nbmax * kBlockBytes > ((int64_t)1 << 30)) {
-        int64_t last_off = 0;
-        int32_t last_cnt = 0, nbricks = 0;
-        double part[WK_WG * WK_N], work[WK_N] = {0, 0, 0, 0, 0, 0};
+        WorkSample found;
+        double work[WK_N] = {0, 0, 0, 0, 0, 0};
         const int64_t ns = std::min<int64_t>(ntot, 1 << 16);
-        HNT_TRY(reserve(ctx, W.flag, sizeof(part)));
+        HNT_TRY(reserve(ctx, W.flag, sizeof(found)));
         hipLaunchKernelGGL(work_sample_kernel, dim3(WK_WG), dim3(256), 0, st, A, keys, vals,
-                           (const int32_t*)stops, ntot, ns, TT.near_shells, TT.mid_shells,
-                           (double*)W.flag.p);
-        HNT_HIP(hipMemcpyAsync(part, W.flag.p, sizeof(part), hipMemcpyDeviceToHost, st));
-        HNT_HIP(hipMemcpyAsync(&nbricks, bcount, 4, hipMemcpyDeviceToHost, st));
-        HNT_HIP(hipMemcpyAsync(&last_off, off + (ntot - 1), 8, hipMemcpyDeviceToHost, st));
-        HNT_HIP(hipMemcpyAsync(&last_cnt, cnt + (ntot - 1), 4, hipMemcpyDeviceToHost, st));
+                           (const int32_t*)stops, (const int64_t*)off, (const int32_t*)cnt,
+                           (const int32_t*)bcount, ntot, ns, TT.near_shells, TT.mid_shells,
+                           (WorkSample*)W.flag.p);
+        HNT_HIP(hipMemcpyAsync(&found, W.flag.p, sizeof(found), hipMemcpyDeviceToHost, st));
         HNT_HIP(hipStreamSynchronize(st));
         for (int w = 0; w < WK_WG; ++w)
             for (int c = 0; c < WK_N; ++c)
-                work[c] = c == 5 ? std::max(work[c], part[w * WK_N + c])
-                                 : work[c] + part[w * WK_N + c] * ((double)ntot / (double)ns);
-        if (lanes_quicker(work, (double)ntot, (double)nbricks, (double)ncell) && lane_room()) {
+                work[c] = c == 5 ? std::max(work[c], found.v[w][c])
+                                 : work[c] + found.v[w][c] * ((double)ntot / (double)ns);
+        if (lanes_quicker(work, (double)ntot, (double)found.bricks, (double)ncell) && lane_room()) {
             *lanes = true;
             stage_end(ctx, HNT_STAGE_SA_CROSS);
             return HNT_OK;
         }
-        const int64_t total = last_off + last_cnt;
+        const int64_t total = found.blocks;
         first[1] = total;
         if (total > kBlockBudget) {
             const int nc = (int)((total + kBlockBudget - 1) / kBlockBudget);
@@ -2219,7 +2217,9 @@ hnt_status analyse_blocks(hnt_ctx* ctx, SAWork& W, SAArgs A, const TablesDev& TT
         else if (beyond)
             for (int f : {0, 2, 3, 4}) far(f);
         // the peaks whose balls leave the grid are in no chunk's order: every launch looks
-        // through all of them
+        // through all of them.  A group's items are shared out where there are few groups (us, 1 /
+        // 8 / 32 shares: 5 groups 294 / 174 / 171, 24 1540 / 633 / 886, 47 2373 / 1026 / 1527; 313,
+        // 1 / 6 / 26: 3444 / 2585 / 2627)
         SAArgs A1 = A;
         A1.slot = far_slot;
         const int shares = (int)std::min<int64_t>(8, std::max<int64_t>(1, 2048 / ngroups));

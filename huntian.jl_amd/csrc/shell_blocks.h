@@ -1432,14 +1432,26 @@ __global__ __launch_bounds__(64) void crossing_rows_kernel(SAArgs a,
 
 // What the gather of a call amounts to, from `ns` of its peaks: per workgroup the cells within
 // BR_H, from there to 20 cells, beyond, those of the peaks whose balls leave the grid, the shells
-// (sums over the samples), and the largest ball's cells.
+// (sums over the samples), and the largest ball's cells.  With them what else the host looks at: the
+// number of blocks and of bricks.
 constexpr int WK_WG = 64, WK_N = 6;
+struct WorkSample {
+    double v[WK_WG][WK_N];
+    int64_t blocks, bricks;
+};
 
 __global__ __launch_bounds__(256) void work_sample_kernel(SAArgs a, const uint64_t* __restrict__ keys,
                                                           const int32_t* __restrict__ vals,
                                                           const int32_t* __restrict__ stop,
+                                                          const int64_t* __restrict__ off,
+                                                          const int32_t* __restrict__ cnt,
+                                                          const int32_t* __restrict__ bricks,
                                                           int64_t ntot, int64_t ns, int near, int mid,
-                                                          double* __restrict__ out) {
+                                                          WorkSample* __restrict__ out) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        out->blocks = off[ntot - 1] + cnt[ntot - 1];
+        out->bricks = *bricks;
+    }
     double v[WK_N] = {0, 0, 0, 0, 0, 0};
     auto cells_to = [&](int s) { return (double)(a.shell_start[s - 1] + a.shell_count[s - 1]); };
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < ns; i += (int64_t)WK_WG * 256) {
@@ -1469,7 +1481,7 @@ __global__ __launch_bounds__(256) void work_sample_kernel(SAArgs a, const uint64
     const int c = threadIdx.x;
     if (c < WK_N) {
         const double x = part[0][c], y = part[1][c], z = part[2][c], w = part[3][c];
-        out[blockIdx.x * WK_N + c] = c == 5 ? fmax(fmax(x, y), fmax(z, w)) : x + y + z + w;
+        out->v[blockIdx.x][c] = c == 5 ? fmax(fmax(x, y), fmax(z, w)) : x + y + z + w;
     }
 }
 
