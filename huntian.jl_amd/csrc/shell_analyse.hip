@@ -29,8 +29,8 @@
 //    of the sorted peak list, so neighbouring peaks share an XCD's L2.  A wave that
 //    drains its queue moves on to the next queue; every wave exits once all eight are
 //    empty.
-// The crossing schedule of a direct call, the default, no longer runs this way but by blocks
-// of shells (shell_blocks.h), with the same results bit for bit.
+// The crossing schedule of a direct call, the default, runs by blocks of shells instead
+// (shell_blocks.h) unless a lane per peak is quicker, with the same results bit for bit.
 #include <hipcub/hipcub.hpp>
 
 #include <mutex>

@@ -352,11 +352,11 @@ hnt_status hnt_shell_analyse_noalloc(hnt_ctx* ctx, const hnt_fields* fields,
                                      hnt_results* results, int8_t* mask);
 
 /*
- * hnt_shell_analyse_tiles -- hnt_shell_analyse over many tiles in one persistent launch (no
+ * hnt_shell_analyse_tiles -- hnt_shell_analyse over many tiles in one call (no
  * counterpart in the reference, whose drivers call analyse_peaks_gpu_cuda_multirf once per
  * tile, src/MultiResolution.jl:532-644).  fields, batches, results: arrays of ntiles
  * structs; masks: host array of ntiles device pointers (entries may be NULL) or NULL.  Tiles
- * may differ in size; peaks of all tiles share the work queues, so tiles of uneven
+ * may differ in size; peaks of all tiles share every launch, so tiles of uneven
  * candidate count and shell depth keep every CU busy.  Results equal those of one
  * hnt_shell_analyse call per tile.
  */
@@ -373,7 +373,10 @@ hnt_status hnt_shell_analyse_tiles(hnt_ctx* ctx, int32_t ntiles, const hnt_field
  * re-reads the fields, peak arrays, ZZon and fcrit at the same addresses (contents may
  * change between launches, sizes and pointers may not) and rewrites results and masks.  The
  * peak schedule of the creating call is kept, so a replay over changed fields is exact but
- * may be slower.  A plan owns its device buffers; it must not outlive its context.
+ * may be slower.  It runs the lane-per-peak kernel (no extent is known before a replay), so
+ * that a direct call of the crossing schedule, which gathers by shell blocks, is the quicker
+ * one for most inputs (64 uneven tiles, 5.4 M peaks: 63 ms against 82).  A plan owns its device
+ * buffers; it must not outlive its context.
  */
 typedef struct hnt_plan hnt_plan;
 hnt_status hnt_plan_create(hnt_ctx* ctx, int32_t ntiles, const hnt_fields* fields,
